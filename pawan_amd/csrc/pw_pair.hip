@@ -36,6 +36,7 @@
 #include <map>
 #include <mutex>
 
+#include "pw_core64.h"
 #include "pw_internal.h"
 
 namespace pw {
@@ -164,7 +165,7 @@ struct AccF64 {
   double bx = 0, by = 0, bz = 0;  // B
 };
 
-__device__ __forceinline__ void pair64(const T64& t, const Rec64& s, AccF64& a) {
+__device__ __forceinline__ void pair64(const T64& t, const Rec64& s, const double* __restrict__ tab, AccF64& a) {
   const double dx = t.x - s.x, dy = t.y - s.y, dz = t.z - s.z;
   const double r2 = dx * dx + dy * dy + dz * dz;
   const double sig2 = 0.5 * s.s2 + t.hs2;
@@ -175,14 +176,15 @@ __device__ __forceinline__ void pair64(const T64& t, const Rec64& s, AccF64& a) 
   const bool core = r2 <= kFar64 * sig2;
   if (core) {
     const double isg = rsqrt_pos(sig2);
-    const double isg3 = isg * isg * isg;
-    const double rb = (r2 * ir) * isg;    // rho / sigma
-    const double irb = (sig2 * isg) * ir;  // sigma / rho
-    const double Z = exp(-0.5 * rb * rb) * isg3 * kK;
-    const double phi = kQ * erf(kSqrtHalf * rb) * isg3;
-    q = (phi * irb - Z) * (irb * irb);
-    F = (Z - 3.0 * q) * ir2;
-    const double c = t.nu2 * Z * (isg * isg);  // 2 nu Z / sigma^2
+    const double isg2 = isg * isg;
+    const double kisg3 = kCore64K * (isg2 * isg);
+    double e, g;
+    // coincident particles (ir not finite) stay non-finite, as in the reference
+    const double sb = fma(ir, 0.0, r2 * isg2);
+    core64(sb, tab, e, g);
+    q = kisg3 * fma(sb, g, e * (1.0 / 3.0));
+    F = -3.0 * (kisg3 * isg2) * g;
+    const double c = t.nu2 * (kisg3 * isg2) * e;  // 2 nu Z / sigma^2
     a.bx += c * (t.vol * s.ax - s.vol * t.ax);
     a.by += c * (t.vol * s.ay - s.vol * t.ay);
     a.bz += c * (t.vol * s.az - s.vol * t.az);
@@ -289,6 +291,8 @@ __device__ __forceinline__ void pair64s(double tx, double ty, double tz, double 
 __device__ __forceinline__ void item_fp64(const PairArgs& pa, const WorkItem& it, TileF64* tile) {
   __shared__ double s_tb[kTB / 64][6];  // each wave's targets' box
   __shared__ double s_b[kTB / 64][7];   // each staged chunk's box (relative to c_T) and largest sigma^2/2
+  __shared__ __align__(16) double tab[kCore64Pieces * kCore64Row];
+  stage_core64(tab);  // (synchronised with the first tile)
   const Rec64* __restrict__ state = pa.state;
   const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
   const int t = it.t0 + static_cast<int>(threadIdx.x);
@@ -381,7 +385,7 @@ __device__ __forceinline__ void item_fp64(const PairArgs& pa, const WorkItem& it
       }
       const bool own = diag && cw == wave;  // the chunk holding this wave's own targets
       for (int l = c0; l < c1; ++l)
-        if (!(own && l == self)) pair64(me, tile[l].rec, a);  // the self pair is never evaluated
+        if (!(own && l == self)) pair64(me, tile[l].rec, tab, a);  // the self pair is never evaluated
     }
   }
   if (active) {
@@ -1495,7 +1499,7 @@ __device__ __forceinline__ Rec64 load(ConstPtr<Rec64> p, int i) {
 // Targets [tb, tb + 64) of item it (a 64-lane wave of its own).
 __device__ __forceinline__ void wave_fp64s(const WorkItem& it, int tb, double nu, const Rec64* state_g,
                                            const Chunk32* chunks_g, int nchunks, const Src64* src_g,
-                                           Rate64* __restrict__ out) {
+                                           const double* __restrict__ tab, Rate64* __restrict__ out) {
   const ConstPtr<Rec64> state = as_const(state_g);
   const ConstPtr<Chunk32> chunks = as_const(chunks_g);
   const ConstPtr<Src64> src = as_const(src_g);
@@ -1549,7 +1553,7 @@ __device__ __forceinline__ void wave_fp64s(const WorkItem& it, int tb, double nu
     } else {
 #pragma unroll 1
       for (int l = l0; l < l1; ++l)
-        if (l != t) pair64(me, load(state, l), a);  // the self pair is never evaluated
+        if (l != t) pair64(me, load(state, l), tab, a);  // the self pair is never evaluated
     }
   }
   if (active) {
@@ -1564,6 +1568,9 @@ __device__ __forceinline__ void wave_fp64s(const WorkItem& it, int tb, double nu
 
 template <bool Persistent>
 __device__ __forceinline__ void fp64s_entry(const PairArgs& a) {
+  __shared__ __align__(16) double tab[kCore64Pieces * kCore64Row];
+  stage_core64(tab);
+  __syncthreads();
   const int waves = 4 * a.nitems;
   for (int w = Persistent ? -1 : static_cast<int>(blockIdx.x);;) {
     if (Persistent) {
@@ -1576,7 +1583,7 @@ __device__ __forceinline__ void fp64s_entry(const PairArgs& a) {
     const int tb = it.t0 + 64 * (w & 3);
     if (tb < it.t1) {
       Rate64* out = it.part < 0 ? a.rates : a.partial + static_cast<size_t>(it.part) * a.n;
-      wave_fp64s(it, tb, a.nu, a.state, a.chunks, a.nchunks, a.src64, out);
+      wave_fp64s(it, tb, a.nu, a.state, a.chunks, a.nchunks, a.src64, tab, out);
     }
     if (!Persistent) break;
   }
@@ -1957,7 +1964,9 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
   pair_entry<kPairFP64HO, P>(a);
 }
 template <bool P>
-__global__ __launch_bounds__(64) void k_pair_fp64s(PairArgs a) { fp64s_entry<P>(a); }
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pair_fp64s(PairArgs a) {
+  fp64s_entry<P>(a);
+}
 // FP32C at the register budget of 7 waves/SIMD (no spills) and of 8
 // waves/SIMD (one spill slot, touched once per tile)
 template <bool P>
