@@ -316,7 +316,9 @@ int pw_get_pair_timing(pw_ctx *ctx, double *total_ms, int64_t *launches);
  *                           it reads feeds two pairs (WAVES8 is ignored);
  * bits that do not apply to the precision are ignored.
  * No counterpart in the reference (its OpenMP loops have no launch shape);
- * defaults are parts 1, grid launch, variant 0.  A variant outside those
+ * defaults are parts 1, grid launch, variant 0, which leaves the launch to
+ * the library: source ranges split over the chip for small systems, the
+ * scalar-fed kernels over many parts for large ones.  A variant outside those
  * bits is PW_ERR_ARG. */
 enum {
   PW_VARIANT_WAVES8 = 1,

@@ -87,7 +87,10 @@ void free_buffers(pw_ctx* c) {
   (void)hipFree(c->d_lin);
   (void)hipFree(c->d_quad);
   (void)hipFree(c->d_flag);
-  for (auto& k : c->ks) (void)hipFree(k.d_items);
+  for (auto& k : c->ks) {
+    (void)hipFree(k.d_items);
+    (void)hipFree(k.d_groups);
+  }
   (void)hipFree(c->partial);
   (void)hipFree(c->d_queue);
   (void)hipFree(c->d_chunks);
@@ -105,11 +108,13 @@ void free_buffers(pw_ctx* c) {
   c->d_flag = c->d_queue = nullptr;
   for (auto& k : c->ks) {
     k.d_items = nullptr;
-    k.nitems = 0;
-    k.built_parts = 0;
+    k.d_groups = nullptr;
+    k.nitems = k.ngroups = 0;
+    k.built_parts = k.built_split = 0;
+    k.lean = false;
   }
   c->partial = nullptr;
-  c->partial_parts = 0;
+  c->partial_rows = 0;
   pwi::ff_release(c);
 }
 
@@ -296,34 +301,146 @@ void drop_graphs(pw_ctx* c) {
   c->graphs.clear();
 }
 
-int ensure_kind(pw_ctx* c, int kind) {
-  if (kind == kKindLearned) return PW_OK;  // the tree path sets itself up
-  auto& k = c->ks[kind];
-  // the scalar-fed FP64 kernel's source records, allocated before any
-  // step is captured (no allocation may happen inside a capture)
-  if (k.cfg.scalar_feed && kind == pw::kPairFP64 && !c->d_src64 && dalloc(&c->d_src64, c->n) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(PW_ERR_NOMEM, "scalar-fed FP64 source records");
+// the pair-kernel kind a precision launches under the context's kernel and
+// summation settings
+int launch_kind_of(const pw_ctx* c, int kind) {
+  if (c->smoothing == PW_KERNEL_HIGHORDER) return kind == pw::kPairFP32C ? pw::kPairFP32CHO : pw::kPairFP64HO;
+  if (kind == pw::kPairFP32C && !c->compensated) return pw::kPairFP32CPlain;
+  return kind;
+}
+
+bool is_default(const pw::PairConfig& p) {
+  return p.parts == 1 && !p.persistent && !p.waves8 && !p.scalar_feed && !p.two_per_lane && p.split == 0;
+}
+
+// Items and groups of a split launch: every system's targets in groups of 64,
+// each against source ranges of `split` particles, items group by group.
+void make_split(const pw_ctx* c, int split, std::vector<WorkItem>& items, std::vector<pw::SplitGroup>& groups) {
+  for (const auto& s : c->systems)
+    for (int64_t t0 = s.a; t0 < s.b; t0 += 64) {
+      const int32_t t1 = static_cast<int32_t>(std::min<int64_t>(t0 + 64, s.b));
+      pw::SplitGroup g{static_cast<int32_t>(t0), t1, static_cast<int32_t>(items.size()), 0};
+      for (int64_t a = s.a; a < s.b; a += split, ++g.count)
+        items.push_back({static_cast<int32_t>(t0), t1, static_cast<int32_t>(a),
+                         static_cast<int32_t>(std::min<int64_t>(a + split, s.b)),
+                         static_cast<int32_t>(items.size()), 0, 0, 0});
+      groups.push_back(g);
+    }
+}
+
+int64_t split_items(const pw_ctx* c, int split) {
+  int64_t items = 0;
+  for (const auto& s : c->systems) items += ((s.b - s.a + 63) / 64) * ((s.b - s.a + split - 1) / split);
+  return items;
+}
+
+// The launch of a kind whose configuration is the default (one part, grid, LDS
+// tiles, as set by nobody or set again).  Two launches cover the sizes; times
+// are one right-hand side in microseconds, leapfrogging rings or helix:
+//
+// * The split kernel while the largest system has at most kSplitUpTo*
+//   particles.  Its source ranges are the longest of 64, 128 and 256 that
+//   leave kSplitItems items, ten blocks per CU: shorter ones add partial sums
+//   (N = 10,000 FP64: 247 at 64, 238 at 128, 248 at 256, 301 at 1,024), longer
+//   ones leave the chip idle (N = 1,000: 15 at 64, 21 at 128, 96 at 1,024, 347
+//   in one part).  Beyond kSplitItemsMax items (403 MB of partial rates) the
+//   ranges double.
+// * Beyond, the scalar-fed kernels, whose separated loops are shorter, over 64
+//   source parts and a persistent queue (32 from 196,608 particles: there 32
+//   are 3% faster in FP64 and level in FP32C at half the partial rates).
+//   FP64, split against scalar-fed: 24,000 particles 1,197 against 1,431,
+//   32,768 2,149 against 2,023, 65,536 8,088 against 6,955; FP32C: 32,000
+//   938 against 1,045, 49,152 2,062 against 2,031, 131,072 14,200 against
+//   11,216.  The high-order FP64 kernel has no scalar-fed form: split at every
+//   size (131,072: 33.8 ms against 34.7 LDS-tiled in 16 parts, 39.7 in one).
+//
+// Systems of a batch are far below these sizes: split wins there by the same
+// rule (48 rings of 512-16,384, FP64 4.1 ms against 5.4 over 64 parts).
+constexpr int64_t kSplitUpTo64 = 32768, kSplitUpTo32 = 45056;
+constexpr int64_t kSplitItems = 2560, kSplitItemsMax = 131072;
+
+pw::PairConfig auto_config(const pw_ctx* c, int launch_kind) {
+  pw::PairConfig p;
+  const bool f32 = launch_kind == pw::kPairFP32C || launch_kind == pw::kPairFP32CHO;
+  if (!f32 && launch_kind != pw::kPairFP64 && launch_kind != pw::kPairFP64HO) return p;
+  const int64_t largest = c->systems.empty() ? 0 : c->systems.front().b - c->systems.front().a;
+  if (launch_kind == pw::kPairFP64HO || largest <= (f32 ? kSplitUpTo32 : kSplitUpTo64)) {
+    p.split = 64;
+    while (p.split < 256 && split_items(c, 2 * p.split) >= kSplitItems) p.split *= 2;
+    while (split_items(c, p.split) > kSplitItemsMax && p.split < largest) p.split *= 2;
+    return p;
   }
-  if (k.built_parts == k.cfg.parts && k.d_items) return PW_OK;
-  std::vector<WorkItem> items = make_items(c, k.cfg.parts);
+  p.parts = c->n < 196608 ? 64 : 32;
+  p.persistent = true;
+  p.waves8 = f32;
+  p.scalar_feed = true;
+  return p;
+}
+
+int ensure_partial(pw_ctx* c, size_t rows) {
+  if (rows <= c->partial_rows) return PW_OK;
+  (void)hipFree(c->partial);
+  c->partial = nullptr;
+  c->partial_rows = 0;
+  if (dalloc(&c->partial, rows) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(PW_ERR_NOMEM, "partial-sum buffer");
+  }
+  c->partial_rows = rows;
+  return PW_OK;
+}
+
+// Work items of cfg on the device, and the partial buffer they need.
+int build_kind(pw_ctx* c, int kind, const pw::PairConfig& cfg) {
+  auto& k = c->ks[kind];
+  std::vector<WorkItem> items;
+  std::vector<pw::SplitGroup> groups;
+  if (cfg.split > 0) make_split(c, cfg.split, items, groups);
+  else items = make_items(c, cfg.parts);
   PW_HIP(hipStreamSynchronize(c->stream));
   drop_graphs(c);  // captured steps point at the buffers replaced here
   (void)hipFree(k.d_items);
+  (void)hipFree(k.d_groups);
   k.d_items = nullptr;
-  if (dalloc(&k.d_items, items.size()) != hipSuccess) return fail(PW_ERR_NOMEM, "work items");
-  PW_HIP(hipMemcpy(k.d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
-  k.nitems = static_cast<int>(items.size());
-  k.built_parts = k.cfg.parts;
-  if (k.cfg.parts > 1 && c->partial_parts < k.cfg.parts) {
-    (void)hipFree(c->partial);
-    c->partial = nullptr;
-    c->partial_parts = 0;
-    if (dalloc(&c->partial, static_cast<size_t>(k.cfg.parts) * c->n) != hipSuccess)
-      return fail(PW_ERR_NOMEM, "partial-sum buffer");
-    c->partial_parts = k.cfg.parts;
+  k.d_groups = nullptr;
+  k.built_parts = k.built_split = 0;
+  if (dalloc(&k.d_items, items.size()) != hipSuccess ||
+      (!groups.empty() && dalloc(&k.d_groups, groups.size()) != hipSuccess)) {
+    (void)hipGetLastError();
+    return fail(PW_ERR_NOMEM, "work items");
   }
+  PW_HIP(hipMemcpy(k.d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
+  if (!groups.empty())
+    PW_HIP(hipMemcpy(k.d_groups, groups.data(), groups.size() * sizeof(pw::SplitGroup), hipMemcpyHostToDevice));
+  if (cfg.split > 0) PW_TRY(ensure_partial(c, 64 * items.size()));
+  else if (cfg.parts > 1) PW_TRY(ensure_partial(c, static_cast<size_t>(cfg.parts) * c->n));
+  k.nitems = static_cast<int>(items.size());
+  k.ngroups = static_cast<int>(groups.size());
+  k.built_parts = cfg.parts;
+  k.built_split = cfg.split;
   return PW_OK;
+}
+
+int ensure_kind(pw_ctx* c, int kind) {
+  if (kind == kKindLearned) return PW_OK;  // the tree path sets itself up
+  auto& k = c->ks[kind];
+  const bool chosen = is_default(k.cfg) && !k.lean;
+  k.run = chosen ? auto_config(c, launch_kind_of(c, kind)) : k.cfg;
+  for (;;) {
+    // the scalar-fed FP64 kernel's source records, allocated before any
+    // step is captured (no allocation may happen inside a capture)
+    int rc = PW_OK;
+    if (k.run.scalar_feed && kind == pw::kPairFP64 && !c->d_src64 && dalloc(&c->d_src64, c->n) != hipSuccess) {
+      (void)hipGetLastError();
+      rc = fail(PW_ERR_NOMEM, "scalar-fed FP64 source records");
+    }
+    if (rc == PW_OK && k.d_items && k.built_parts == k.run.parts && k.built_split == k.run.split) return PW_OK;
+    if (rc == PW_OK) rc = build_kind(c, kind, k.run);
+    // a launch chosen here that does not fit in memory: the one that needs none
+    if (rc != PW_ERR_NOMEM || !chosen || is_default(k.run)) return rc;
+    k.run = pw::PairConfig{};
+    k.lean = true;
+  }
 }
 
 // Blocks of wake pairs for the per-wake hooks: pairs (a, b) with a <= b,
@@ -347,16 +464,10 @@ void append_items(const pw_ctx* c, int a, int b, int nself, std::vector<WorkItem
                    chunk_of(c, c->woff[b]), 0});
 }
 
-// the pair-kernel kind a precision launches under the context's kernel and
-// summation settings
-int launch_kind_of(const pw_ctx* c, int kind) {
-  if (c->smoothing == PW_KERNEL_HIGHORDER) return kind == pw::kPairFP32C ? pw::kPairFP32CHO : pw::kPairFP64HO;
-  if (kind == pw::kPairFP32C && !c->compensated) return pw::kPairFP32CPlain;
-  return kind;
-}
-
-// One right-hand side f(state) -> out, with optional event timing.
-int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out) {
+// One right-hand side f(state) -> out, with optional event timing, and the
+// stage arithmetic that follows it.
+int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp& op = pw::StageOp{}) {
+  const int n = static_cast<int>(c->n);
   if (kind == kKindLearned) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (c->profiling) {
@@ -368,15 +479,15 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out) {
       PW_HIP(hipEventRecord(e1, c->stream));
       c->ev_used.emplace_back(e0, e1);
     }
-    PW_HIP(pw::launch_check_finite(out, static_cast<int>(c->n), c->d_flag, c->stream));
+    PW_HIP(pw::launch_finish(pw::SumForm{}, out, n, c->d_flag, op, c->stream));
     return PW_OK;
   }
   if (kind == pw::kPairFP32C && !c->compensated && c->smoothing == PW_KERNEL_GAUSSIAN) {
     // plain FP32 sums: one item per 256-target block over all its sources
-    pw::PairArgs args{state, c->pair_items, c->npair, static_cast<int>(c->n), out, nullptr, c->d_queue, c->nu,
+    pw::PairArgs args{state, c->pair_items, c->npair, n, out, nullptr, c->d_queue, c->nu,
                       c->d_chunks, c->d_src32, nullptr, c->nchunks};
     PW_HIP(pw::launch_pair(pw::kPairFP32CPlain, pw::PairConfig{}, args, c->npair, c->stream));
-    PW_HIP(pw::launch_check_finite(out, static_cast<int>(c->n), c->d_flag, c->stream));
+    PW_HIP(pw::launch_finish(pw::SumForm{}, out, n, c->d_flag, op, c->stream));
     return PW_OK;
   }
   PW_TRY(ensure_kind(c, kind));
@@ -385,7 +496,7 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out) {
   args.state = state;
   args.items = k.d_items;
   args.nitems = k.nitems;
-  args.n = static_cast<int>(c->n);
+  args.n = n;
   args.rates = out;
   args.partial = c->partial;
   args.queue = c->d_queue;
@@ -394,21 +505,28 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out) {
   args.src = c->d_src32;
   args.src64 = nullptr;
   args.nchunks = c->nchunks;
-  if (k.cfg.scalar_feed && launch_kind_of(c, kind) == pw::kPairFP64) args.src64 = c->d_src64;  // ensure_kind made it
   // the high-order kernel replaces the Gaussian kinds (pw_set_kernel)
   const int launch_kind = launch_kind_of(c, kind);
-  const int grid = c->num_cus * pw::pair_kernel_waves(launch_kind, k.cfg);
+  if (k.run.scalar_feed && launch_kind == pw::kPairFP64) args.src64 = c->d_src64;  // ensure_kind made it
+  const int grid = c->num_cus * pw::pair_kernel_waves(launch_kind, k.run);
+  pw::SumForm sum;
+  sum.partial = c->partial;
+  sum.parts = k.run.parts;
+  if (k.run.split > 0) {
+    sum.groups = k.d_groups;
+    sum.ngroups = k.ngroups;
+  }
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (c->profiling) {
     PW_TRY(pwi::prof_begin(c, &e0, &e1));
     PW_HIP(hipEventRecord(e0, c->stream));
   }
-  PW_HIP(pw::launch_pair(launch_kind, k.cfg, args, grid, c->stream));
+  PW_HIP(pw::launch_pair(launch_kind, k.run, args, grid, c->stream));
   if (c->profiling) {
     PW_HIP(hipEventRecord(e1, c->stream));
     c->ev_used.emplace_back(e0, e1);
   }
-  PW_HIP(pw::launch_check_finite(out, static_cast<int>(c->n), c->d_flag, c->stream));
+  PW_HIP(pw::launch_finish(sum, out, n, c->d_flag, op, c->stream));
   return PW_OK;
 }
 
@@ -918,33 +1036,48 @@ int pw_solve(pw_ctx* c, int precision) {
 
 namespace {
 
-// The kernels of one step of `scheme` on the context stream.
+// The kernels of one step of `scheme` on the context stream; each right-hand
+// side carries the stage arithmetic that uses it.
 int enqueue_step(pw_ctx* c, int scheme, int kind, double dt) {
-  const int n = static_cast<int>(c->n);
-  hipStream_t st = c->stream;
   Rate64** k = c->k;
+  pw::StageOp op;
+  op.y = c->y;
+  op.out = c->ys;
   if (scheme == PW_RK4) {
     // rk4.cpp:20-66
-    PW_TRY(rhs(c, kind, c->y, k[0]));
-    PW_HIP(pw::launch_stage(c->y, k[0], 0.5 * dt, c->ys, n, st));
-    PW_TRY(rhs(c, kind, c->ys, k[1]));
-    PW_HIP(pw::launch_stage(c->y, k[1], 0.5 * dt, c->ys, n, st));
-    PW_TRY(rhs(c, kind, c->ys, k[2]));
-    PW_HIP(pw::launch_stage(c->y, k[2], dt, c->ys, n, st));
-    PW_TRY(rhs(c, kind, c->ys, k[3]));
-    PW_HIP(pw::launch_rk4_final(c->y, k[0], k[1], k[2], k[3], dt / 6., dt / 3., n, st));
+    op.kind = pw::kStageLin;
+    op.a = 0.5 * dt;
+    PW_TRY(rhs(c, kind, c->y, k[0], op));
+    PW_TRY(rhs(c, kind, c->ys, k[1], op));
+    op.a = dt;
+    PW_TRY(rhs(c, kind, c->ys, k[2], op));
+    op.kind = pw::kStageRk4;
+    op.k1 = k[0];
+    op.k2 = k[1];
+    op.k3 = k[2];
+    op.a = dt / 6.;
+    op.b = dt / 3.;
+    PW_TRY(rhs(c, kind, c->ys, k[3], op));
   } else if (scheme == PW_RK3) {
     // rk3.cpp:20-55
-    PW_TRY(rhs(c, kind, c->y, k[0]));
-    PW_HIP(pw::launch_stage(c->y, k[0], 0.5 * dt, c->ys, n, st));
-    PW_TRY(rhs(c, kind, c->ys, k[1]));
-    PW_HIP(pw::launch_rk3_mid(c->y, k[0], k[1], dt, 2. * dt, c->ys, n, st));
-    PW_TRY(rhs(c, kind, c->ys, k[2]));
-    PW_HIP(pw::launch_rk3_final(c->y, k[0], k[1], k[2], dt / 6.0, dt * 2.0 / 3.0, n, st));
+    op.kind = pw::kStageLin;
+    op.a = 0.5 * dt;
+    PW_TRY(rhs(c, kind, c->y, k[0], op));
+    op.kind = pw::kStageRk3Mid;
+    op.k1 = k[0];
+    op.a = dt;
+    op.b = 2. * dt;
+    PW_TRY(rhs(c, kind, c->ys, k[1], op));
+    op.kind = pw::kStageRk3;
+    op.k2 = k[1];
+    op.a = dt / 6.0;
+    op.b = dt * 2.0 / 3.0;
+    PW_TRY(rhs(c, kind, c->ys, k[2], op));
   } else {
     // integration.cpp:126-136
-    PW_TRY(rhs(c, kind, c->y, k[0]));
-    PW_HIP(pw::launch_euler(c->y, k[0], dt, n, st));
+    op.kind = pw::kStageEuler;
+    op.a = dt;
+    PW_TRY(rhs(c, kind, c->y, k[0], op));
   }
   return PW_OK;
 }

@@ -110,14 +110,19 @@ struct pw_ctx {
 
   // per pair-kernel kind: launch configuration and its work items
   struct KindState {
-    pw::PairConfig cfg;
+    pw::PairConfig cfg;   // as set or tuned (the default: launch chosen by auto_config)
+    pw::PairConfig run;   // as launched
     pw::WorkItem* d_items = nullptr;
     int nitems = 0;
-    int built_parts = 0;  // parts the items were built for (0: none yet)
+    pw::SplitGroup* d_groups = nullptr;  // split launches
+    int ngroups = 0;
+    int built_parts = 0;  // parts and split the items were built for (0: none yet)
+    int built_split = 0;
+    bool lean = false;    // the chosen launch's buffers did not fit in memory
     bool tuned = false;
   } ks[3];
-  pw::Rate64* partial = nullptr;  // source-split partial rates, parts x n
-  int partial_parts = 0;
+  pw::Rate64* partial = nullptr;  // source-split partial rates (parts x n, or 64 rows per split item)
+  size_t partial_rows = 0;
   int* d_queue = nullptr;     // work counter of the persistent kernels
   // source chunks of the scalar-fed FP32C kernel: runs of up to 64
   // particles of one system (chunk_first: their first particles, ascending)

@@ -38,6 +38,13 @@ struct WorkItem {
   int32_t pad2;
 };
 
+// One group of at most 64 targets [t0, t1) of the split kernel: its items'
+// partial rates are the 64-row slabs [first, first + count) of the partial
+// buffer, summed in that order.
+struct SplitGroup {
+  int32_t t0, t1, first, count;
+};
+
 // Sources as the scalar-fed FP32C kernel reads them, rebuilt from the state
 // before each of its launches.  The sources of each system are cut into
 // chunks of up to 64 consecutive particles; a chunk carries its bounding
@@ -68,7 +75,7 @@ struct PairArgs {
   int nitems;
   int n;              // particles (stride of the partial buffer)
   Rate64* rates;
-  Rate64* partial;    // parts x n, used by items with part >= 0
+  Rate64* partial;    // parts x n, used by items with part >= 0 (split: 64 rows per item)
   int* queue;         // work counter of the persistent kernels
   double nu;
   Chunk32* chunks;    // scalar-fed FP32C: source chunks (geometry rebuilt per launch)
@@ -86,6 +93,8 @@ struct PairConfig {
                            // scalar loads (Chunk32/Src32) instead of LDS
                            // tiles shared by the block's four waves
   bool two_per_lane = false;// FP32C scalar-fed: two targets per lane
+  int split = 0;           // sources per item of the split kernel (one block
+                           // per 64 targets and source range); 0: not used
 };
 
 // Pair-kernel variants.
@@ -103,9 +112,9 @@ enum PairKind : int {
                        // 256-target block, grid launch)
 };
 
-// Pair kernel of `kind` over args.items; for parts > 1 also the reduction
-// of the partial sums into args.rates.  grid = resident blocks for the
-// persistent form.
+// Pair kernel of `kind` over args.items.  Source-split launches (parts > 1 or
+// split) leave their partial sums in args.partial for launch_finish.  grid =
+// resident blocks for the persistent form.
 hipError_t launch_pair(int kind, const PairConfig& cfg, const PairArgs& args, int grid,
                        hipStream_t st);
 // resident blocks per CU of the persistent pair kernel of `kind` (256-thread
@@ -115,26 +124,38 @@ int pair_kernel_waves(int kind, const PairConfig& cfg);
 // resident one-wave blocks per CU of the tree path's near-field kernel
 int near_kernel_blocks_per_cu(bool highorder, bool uniform_sigma);
 
-// Stage arithmetic of the steppers (FP64, no contraction, the reference's
-// operation order).  n = number of particles.
-//   out = k * c + y                     (rk4.cpp:31-34 etc.)
-hipError_t launch_stage(const Rec64* y, const Rate64* k, double c, Rec64* out,
-                        int n, hipStream_t st);
-//   y = y + ((k1 + k4) * c6 + (k2 + k3) * c3)      (rk4.cpp:58-66)
-hipError_t launch_rk4_final(Rec64* y, const Rate64* k1, const Rate64* k2,
-                            const Rate64* k3, const Rate64* k4, double c6,
-                            double c3, int n, hipStream_t st);
-//   k1 = k1 * dt ; out = (k2 * 2dt + y) - k1      (rk3.cpp:37-41)
-hipError_t launch_rk3_mid(const Rec64* y, Rate64* k1, const Rate64* k2,
-                          double dt, double two_dt, Rec64* out, int n,
-                          hipStream_t st);
-//   y = y + ((k1 * (1/6) + k3 * (dt/6)) + k2 * (dt*2/3))   (rk3.cpp:47-55)
-hipError_t launch_rk3_final(Rec64* y, const Rate64* k1, const Rate64* k2,
-                            const Rate64* k3, double c6, double c23, int n,
-                            hipStream_t st);
-//   y = y + k * dt                      (integration.cpp:130-133)
-hipError_t launch_euler(Rec64* y, const Rate64* k, double dt, int n,
-                        hipStream_t st);
+// What becomes of a right-hand side's rates k beside being stored: the stage
+// arithmetic of the steppers (FP64, no contraction, the reference's operation
+// order).
+enum StageKind : int {
+  kStageNone = 0,
+  kStageLin,       // out = k * a + y                           (rk4.cpp:31-34 etc.)
+  kStageRk4,       // y = y + ((k1 + k) * a + (k2 + k3) * b)     (rk4.cpp:58-66)
+  kStageRk3Mid,    // k1 = k1 * a; out = (k * b + y) - k1        (rk3.cpp:37-41)
+  kStageRk3,       // y = y + ((k1 * (1/6) + k * a) + k2 * b)    (rk3.cpp:47-55)
+  kStageEuler,     // y = y + k * a                             (integration.cpp:130-133)
+};
+struct StageOp {
+  int kind = kStageNone;
+  Rec64* y = nullptr;
+  Rec64* out = nullptr;
+  Rate64* k1 = nullptr;
+  const Rate64* k2 = nullptr;
+  const Rate64* k3 = nullptr;
+  double a = 0.0, b = 0.0;
+};
+// How a right-hand side's rates were left: in `rates` already (parts = 1,
+// groups = nullptr), as `parts` slices of n rows in `partial`, or as the split
+// kernel's slabs.
+struct SumForm {
+  const Rate64* partial = nullptr;
+  int parts = 1;
+  const SplitGroup* groups = nullptr;
+  int ngroups = 0;
+};
+// Sum of the partial rates into `rates` (in order), flag |= any non-finite
+// rate, and the stage arithmetic, in one pass.
+hipError_t launch_finish(const SumForm& sum, Rate64* rates, int n, int* flag, const StageOp& op, hipStream_t st);
 // count of non-finite entries of the rates -> *flag (device int)
 hipError_t launch_check_finite(const Rate64* k, int n, int* flag,
                                hipStream_t st);

@@ -103,7 +103,7 @@ __device__ __forceinline__ void pair64_exact(const Rec64& t, const Rec64& s,
 }
 
 // Where an item's rates go: straight to the rates, or to its part's slice
-// of the partial-sum buffer (source-split items, summed by k_reduce_parts).
+// of the partial-sum buffer (source-split items, summed by k_finish).
 __device__ __forceinline__ Rate64* out_rates(const PairArgs& a, const WorkItem& it) {
   return it.part < 0 ? a.rates : a.partial + static_cast<size_t>(it.part) * a.n;
 }
@@ -2007,18 +2007,172 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 // aid, not a production path
 __global__ __launch_bounds__(kTB) void k_pair_fp32c_plain(PairArgs a) { pair_entry<kPairFP32CPlain, false>(a); }
 
-// rates[t] = sum over parts of partial[p][t], parts in order (FP64).
-__global__ __launch_bounds__(256) void k_reduce_parts(const Rate64* __restrict__ partial,
-                                                      int parts, int n, Rate64* __restrict__ rates) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= n) return;
-  Rate64 s = partial[t];
-  for (int p = 1; p < parts; ++p) {
-    const Rate64 q = partial[static_cast<size_t>(p) * n + t];
-    s.ux += q.ux; s.uy += q.uy; s.uz += q.uz;
-    s.wx += q.wx; s.wy += q.wy; s.wz += q.wz;
+// ---------------------------------------------------------------------
+// Split direct sum: one block per (64 targets, source range).  The block's
+// four waves hold the same 64 targets, one per lane; a tile of up to 256
+// sources is staged in LDS and each wave takes a quarter of it, so a wave's
+// serial chain is a quarter of the range; the four waves' sums are added in
+// LDS in wave order and leave as one 64-row slab of the partial buffer.
+//
+// For wakes whose targets alone do not fill the chip.  One lane per target
+// against all sources (the LDS-tiled and scalar-fed kernels with one part)
+// leaves 4 blocks for 1,000 particles and runs at the latency of one pair
+// after another.  Here the source range of an item shrinks until about a
+// thousand blocks exist (auto_config in pw_capi.hip), down to 64 sources, 16
+// per wave.  Measured per right-hand side, one part LDS-tiled against this:
+// ring of 1,000 FP64 347 -> 15 us, two rings of 4,816 1,155 -> 74 us (FP64),
+// 1,017 -> 63 us (high-order), 728 -> 42 us (FP32C); at 24,000 FP64 it runs
+// 481 G pairs/s, bound by its instructions per pair (52 beyond the core, 98 in
+// it), no longer by waves in flight.
+// ---------------------------------------------------------------------
+template <int Kind>
+struct SplitSum;
+
+template <>
+struct SplitSum<kPairFP64> {
+  using Src = Rec64;
+  static constexpr bool kTable = true;
+  T64 me;
+  AccF64 a;
+  __device__ __forceinline__ void init(const Rec64& m, double nu) {
+    me.x = m.x; me.y = m.y; me.z = m.z; me.hs2 = 0.5 * m.s2;
+    me.ax = m.ax; me.ay = m.ay; me.az = m.az; me.vol = m.vol;
+    me.nu2 = 2.0 * nu;
   }
-  rates[t] = s;
+  static __device__ __forceinline__ Src source(const Rec64& r) { return r; }
+  __device__ __forceinline__ void pair(const Src& s, const double* __restrict__ tab) { pair64(me, s, tab, a); }
+  __device__ __forceinline__ void chunk_end() {}
+  __device__ __forceinline__ void result(double (&r)[6]) const {
+    r[0] = a.ux; r[1] = a.uy; r[2] = a.uz;
+    r[3] = (me.ay * a.az - me.az * a.ay) + a.bx;
+    r[4] = (me.az * a.ax - me.ax * a.az) + a.by;
+    r[5] = (me.ax * a.ay - me.ay * a.ax) + a.bz;
+  }
+};
+
+template <>
+struct SplitSum<kPairFP64HO> {
+  using Src = Rec64;
+  static constexpr bool kTable = false;
+  T64 me;
+  AccHO a;
+  __device__ __forceinline__ void init(const Rec64& m, double nu) {
+    me.x = m.x; me.y = m.y; me.z = m.z; me.hs2 = 0.5 * m.s2;
+    me.ax = m.ax; me.ay = m.ay; me.az = m.az; me.vol = m.vol;
+    me.nu2 = 2.0 * nu;
+  }
+  static __device__ __forceinline__ Src source(const Rec64& r) { return r; }
+  __device__ __forceinline__ void pair(const Src& s, const double* __restrict__) { pair64_ho(me, s, a); }
+  __device__ __forceinline__ void chunk_end() {}
+  __device__ __forceinline__ void result(double (&r)[6]) const {
+    r[0] = a.ux; r[1] = a.uy; r[2] = a.uz;
+    r[3] = ((me.ay * a.az - me.az * a.ay) + a.bx) + (me.vol * a.cx - a.d * me.ax);
+    r[4] = ((me.az * a.ax - me.ax * a.az) + a.by) + (me.vol * a.cy - a.d * me.ay);
+    r[5] = ((me.ax * a.ay - me.ay * a.ax) + a.bz) + (me.vol * a.cz - a.d * me.az);
+  }
+};
+
+// FP32C: plain FP32 sums over at most 64 pairs (a wave's quarter of a tile),
+// then the compensated totals, as in the other FP32C kernels
+template <bool HighOrder>
+struct SplitSum32 {
+  using Src = SrcT;
+  static constexpr bool kTable = false;
+  T32 me;
+  P32 p;
+  PSE32 pse;
+  float hi[kAcc], lo[kAcc];
+  __device__ __forceinline__ void init(const Rec64& m, double nu) {
+    me.x = m.x; me.y = m.y; me.z = m.z;
+    me.hs2 = static_cast<float>(0.5 * m.s2);
+    me.ax = static_cast<float>(m.ax);
+    me.ay = static_cast<float>(m.ay);
+    me.az = static_cast<float>(m.az);
+    me.vol = static_cast<float>(m.vol);
+    me.nu2 = 2.0f * static_cast<float>(nu);
+#pragma unroll
+    for (int k = 0; k < kAcc; ++k) hi[k] = lo[k] = 0.0f;
+  }
+  static __device__ __forceinline__ Src source(const Rec64& r) {
+    Src s;
+    s.x = r.x; s.y = r.y; s.z = r.z;
+    s.hs2 = static_cast<float>(0.5 * r.s2);
+    s.ax = static_cast<float>(r.ax);
+    s.ay = static_cast<float>(r.ay);
+    s.az = static_cast<float>(r.az);
+    s.vol = static_cast<float>(r.vol);
+    s.pad = 0.0f;
+    return s;
+  }
+  __device__ __forceinline__ void pair(const Src& s, const double* __restrict__) {
+    if (HighOrder) pair32_ho(me, s, p, pse);
+    else pair32(me, s, p, pse);
+  }
+  __device__ __forceinline__ void chunk_end() {
+    fold(p, me.ax, me.ay, me.az, hi, lo);
+    p = P32{};
+  }
+  __device__ __forceinline__ void result(double (&r)[6]) const {
+#pragma unroll
+    for (int k = 0; k < kAcc; ++k) r[k] = kQ * (static_cast<double>(hi[k]) + static_cast<double>(lo[k]));
+    r[3] += static_cast<double>(pse.x);
+    r[4] += static_cast<double>(pse.y);
+    r[5] += static_cast<double>(pse.z);
+  }
+};
+template <>
+struct SplitSum<kPairFP32C> : SplitSum32<false> {};
+template <>
+struct SplitSum<kPairFP32CHO> : SplitSum32<true> {};
+
+template <int Kind>
+__global__ __launch_bounds__(kTB) void k_pair_split(PairArgs pa) {
+  using Sum = SplitSum<Kind>;
+  constexpr int kWaves = kTB / 64;
+  constexpr size_t kTileBytes = kTB * sizeof(typename Sum::Src);
+  constexpr size_t kRedBytes = (kWaves - 1) * 64 * 6 * sizeof(double);
+  __shared__ __align__(16) unsigned char mem[kTileBytes > kRedBytes ? kTileBytes : kRedBytes];
+  __shared__ __align__(16) double tab[Sum::kTable ? kCore64Pieces * kCore64Row : 2];
+  typename Sum::Src* tile = reinterpret_cast<typename Sum::Src*>(mem);
+  const Rec64* __restrict__ state = pa.state;
+  const WorkItem it = pa.items[blockIdx.x];
+  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+  if (Sum::kTable) stage_core64(tab);  // (synchronised with the first tile)
+  const int t = it.t0 + lane;
+  const bool active = t < it.t1;
+  Sum sum;
+  sum.init(state[active ? t : it.t0], pa.nu);
+  for (int base = it.s0; base < it.s1; base += kTB) {
+    const int cnt = min(kTB, it.s1 - base);
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = Sum::source(state[base + threadIdx.x]);
+    __syncthreads();
+    const int l0 = cnt * wave / kWaves, l1 = cnt * (wave + 1) / kWaves;
+    if (base + l0 < it.t1 && base + l1 > it.t0) {  // the wave's own targets may be among these sources
+      for (int l = l0; l < l1; ++l)
+        if (base + l != t) sum.pair(tile[l], tab);  // the self pair is never evaluated
+    } else {
+      for (int l = l0; l < l1; ++l) sum.pair(tile[l], tab);
+    }
+    sum.chunk_end();
+  }
+  double r[6];
+  sum.result(r);
+  __syncthreads();  // the last tile is read
+  double* red = reinterpret_cast<double*>(mem);
+  if (wave > 0)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) red[((wave - 1) * 6 + k) * 64 + lane] = r[k];
+  __syncthreads();
+  if (wave > 0 || !active) return;
+#pragma unroll
+  for (int w = 0; w < kWaves - 1; ++w)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) r[k] += red[(w * 6 + k) * 64 + lane];
+  Rate64 o;
+  o.ux = r[0]; o.uy = r[1]; o.uz = r[2];
+  o.wx = r[3]; o.wy = r[4]; o.wz = r[5];
+  pa.partial[static_cast<size_t>(it.part) * 64 + lane] = o;
 }
 
 }  // namespace
@@ -2066,6 +2220,17 @@ hipError_t launch_fp32s(int kind, const PairConfig& cfg, const PairArgs& args, i
 hipError_t launch_pair(int kind, const PairConfig& cfg, const PairArgs& args, int grid,
                        hipStream_t st) {
   if (args.nitems <= 0) return hipSuccess;
+  if (cfg.split > 0) {
+    const dim3 g(static_cast<unsigned>(args.nitems)), block(kTB);
+    switch (kind) {
+      case kPairFP64: hipLaunchKernelGGL(k_pair_split<kPairFP64>, g, block, 0, st, args); break;
+      case kPairFP64HO: hipLaunchKernelGGL(k_pair_split<kPairFP64HO>, g, block, 0, st, args); break;
+      case kPairFP32C: hipLaunchKernelGGL(k_pair_split<kPairFP32C>, g, block, 0, st, args); break;
+      case kPairFP32CHO: hipLaunchKernelGGL(k_pair_split<kPairFP32CHO>, g, block, 0, st, args); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   if (cfg.scalar_feed && kind == kPairFP64) {
     if (!args.chunks || !args.src64 || args.nchunks <= 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_src_chunks64, dim3(args.nchunks), dim3(64), 0, st, args.state, args.chunks, args.src64);
@@ -2080,18 +2245,10 @@ hipError_t launch_pair(int kind, const PairConfig& cfg, const PairArgs& args, in
     } else {
       hipLaunchKernelGGL(k_pair_fp64s<false>, dim3(static_cast<unsigned>(waves)), dim3(64), 0, st, args);
     }
-    e = hipGetLastError();
-    if (e != hipSuccess || cfg.parts <= 1) return e;
-    hipLaunchKernelGGL(k_reduce_parts, dim3((args.n + 255) / 256), dim3(256), 0, st, args.partial,
-                       cfg.parts, args.n, args.rates);
     return hipGetLastError();
   }
   if (cfg.scalar_feed && (kind == kPairFP32C || kind == kPairFP32CHO)) {
-    hipError_t e = launch_fp32s(kind, cfg, args, grid, st);
-    if (e != hipSuccess || cfg.parts <= 1) return e;
-    hipLaunchKernelGGL(k_reduce_parts, dim3((args.n + 255) / 256), dim3(256), 0, st, args.partial,
-                       cfg.parts, args.n, args.rates);
-    return hipGetLastError();
+    return launch_fp32s(kind, cfg, args, grid, st);
   }
   const dim3 block(kTB);
   const dim3 g(cfg.persistent ? static_cast<unsigned>(std::min(grid, args.nitems))
@@ -2139,10 +2296,6 @@ const bool P = cfg.persistent;
     default:
       return hipErrorInvalidValue;
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || cfg.parts <= 1) return e;
-  hipLaunchKernelGGL(k_reduce_parts, dim3((args.n + 255) / 256), dim3(256), 0, st, args.partial,
-                     cfg.parts, args.n, args.rates);
   return hipGetLastError();
 }
 

@@ -14,115 +14,87 @@ namespace {
 
 constexpr int kEW = 256;
 
-__global__ __launch_bounds__(kEW) void k_stage(const Rec64* __restrict__ y,
-                                               const Rate64* __restrict__ k,
-                                               double c, Rec64* __restrict__ out,
-                                               int n) {
+// One right-hand side's tail: the sum of its partial rates, the finite check
+// and the stage arithmetic, one thread per rate component (component c of
+// particle t is double 6 t + c of the rates, so every partial slice or slab is
+// read coalesced).  A small wake's step is bound by its launches: 3 kernels
+// per right-hand side became 1, and by the latency of the partial loads, which
+// the unrolled loop keeps several in flight of.
+//
+// The partial rates are summed in order (deterministic).  Sum: 0 none, 1
+// slices of n rows, 2 slabs of 64 rows (k_pair_split).
+constexpr int kGroupThreads = 6 * 64;  // a group's 64 rows
+
+struct FinishArgs {
+  const double* partial;
+  int parts;
+  const SplitGroup* groups;
+  double* rates;
+  int n;
+  int* flag;
+  StageOp op;
+};
+
+template <int Op>
+__device__ __forceinline__ void stage_component(const StageOp& op, int64_t e, double k) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * kEW + threadIdx.x;
-  if (i >= n) return;
-  const Rec64 a = y[i];
-  const Rate64 r = k[i];
-  Rec64 o;
-  o.x = r.ux * c + a.x;
-  o.y = r.uy * c + a.y;
-  o.z = r.uz * c + a.z;
-  o.s2 = a.s2;
-  o.ax = r.wx * c + a.ax;
-  o.ay = r.wy * c + a.ay;
-  o.az = r.wz * c + a.az;
-  o.vol = a.vol;
-  out[i] = o;
+  if (Op == kStageNone) return;
+  const int64_t t = e / 6;
+  const int c = static_cast<int>(e - 6 * t);
+  const int64_t at = 8 * t + c + (c >= 3 ? 1 : 0);  // the component in Rec64: x y z s2 ax ay az vol
+  double* y = reinterpret_cast<double*>(op.y);
+  const double yc = y[at];
+  if (Op == kStageLin || Op == kStageRk3Mid) {
+    double* out = reinterpret_cast<double*>(op.out);
+    if (Op == kStageLin) {
+      out[at] = k * op.a + yc;
+    } else {
+      double* k1 = reinterpret_cast<double*>(op.k1);
+      const double b1 = k1[e] * op.a;
+      out[at] = (k * op.b + yc) - b1;
+      k1[e] = b1;
+    }
+    if (c == 2 || c == 5) out[at + 1] = y[at + 1];  // s2, vol
+  } else if (Op == kStageRk4) {
+    const double a1 = reinterpret_cast<const double*>(op.k1)[e], a2 = reinterpret_cast<const double*>(op.k2)[e],
+                 a3 = reinterpret_cast<const double*>(op.k3)[e];
+    y[at] = yc + ((a1 + k) * op.a + (a2 + a3) * op.b);
+  } else if (Op == kStageRk3) {
+    const double b1 = reinterpret_cast<const double*>(op.k1)[e], a2 = reinterpret_cast<const double*>(op.k2)[e];
+    y[at] = yc + ((b1 * (1.0 / 6.0) + k * op.a) + a2 * op.b);
+  } else {
+    y[at] = yc + k * op.a;
+  }
 }
 
-__device__ __forceinline__ double rk4c(double y, double a1, double a4,
-                                       double a2, double a3, double c6,
-                                       double c3) {
-#pragma clang fp contract(off)
-  return y + ((a1 + a4) * c6 + (a2 + a3) * c3);
-}
-
-__global__ __launch_bounds__(kEW) void k_rk4_final(
-    Rec64* __restrict__ y, const Rate64* __restrict__ k1,
-    const Rate64* __restrict__ k2, const Rate64* __restrict__ k3,
-    const Rate64* __restrict__ k4, double c6, double c3, int n) {
-  const int i = blockIdx.x * kEW + threadIdx.x;
-  if (i >= n) return;
-  Rec64 a = y[i];
-  const Rate64 r1 = k1[i], r2 = k2[i], r3 = k3[i], r4 = k4[i];
-  a.x = rk4c(a.x, r1.ux, r4.ux, r2.ux, r3.ux, c6, c3);
-  a.y = rk4c(a.y, r1.uy, r4.uy, r2.uy, r3.uy, c6, c3);
-  a.z = rk4c(a.z, r1.uz, r4.uz, r2.uz, r3.uz, c6, c3);
-  a.ax = rk4c(a.ax, r1.wx, r4.wx, r2.wx, r3.wx, c6, c3);
-  a.ay = rk4c(a.ay, r1.wy, r4.wy, r2.wy, r3.wy, c6, c3);
-  a.az = rk4c(a.az, r1.wz, r4.wz, r2.wz, r3.wz, c6, c3);
-  y[i] = a;
-}
-
-__global__ __launch_bounds__(kEW) void k_rk3_mid(const Rec64* __restrict__ y,
-                                                 Rate64* __restrict__ k1,
-                                                 const Rate64* __restrict__ k2,
-                                                 double dt, double two_dt,
-                                                 Rec64* __restrict__ out, int n) {
-#pragma clang fp contract(off)
-  const int i = blockIdx.x * kEW + threadIdx.x;
-  if (i >= n) return;
-  const Rec64 a = y[i];
-  Rate64 r1 = k1[i];
-  const Rate64 r2 = k2[i];
-  r1.ux = r1.ux * dt; r1.uy = r1.uy * dt; r1.uz = r1.uz * dt;
-  r1.wx = r1.wx * dt; r1.wy = r1.wy * dt; r1.wz = r1.wz * dt;
-  Rec64 o;
-  o.x = (r2.ux * two_dt + a.x) - r1.ux;
-  o.y = (r2.uy * two_dt + a.y) - r1.uy;
-  o.z = (r2.uz * two_dt + a.z) - r1.uz;
-  o.s2 = a.s2;
-  o.ax = (r2.wx * two_dt + a.ax) - r1.wx;
-  o.ay = (r2.wy * two_dt + a.ay) - r1.wy;
-  o.az = (r2.wz * two_dt + a.az) - r1.wz;
-  o.vol = a.vol;
-  k1[i] = r1;
-  out[i] = o;
-}
-
-__device__ __forceinline__ double rk3c(double y, double b1, double a2,
-                                       double a3, double c6, double c23) {
-#pragma clang fp contract(off)
-  return y + ((b1 * (1.0 / 6.0) + a3 * c6) + a2 * c23);
-}
-
-__global__ __launch_bounds__(kEW) void k_rk3_final(
-    Rec64* __restrict__ y, const Rate64* __restrict__ k1,
-    const Rate64* __restrict__ k2, const Rate64* __restrict__ k3, double c6,
-    double c23, int n) {
-  const int i = blockIdx.x * kEW + threadIdx.x;
-  if (i >= n) return;
-  Rec64 a = y[i];
-  const Rate64 r1 = k1[i], r2 = k2[i], r3 = k3[i];
-  a.x = rk3c(a.x, r1.ux, r2.ux, r3.ux, c6, c23);
-  a.y = rk3c(a.y, r1.uy, r2.uy, r3.uy, c6, c23);
-  a.z = rk3c(a.z, r1.uz, r2.uz, r3.uz, c6, c23);
-  a.ax = rk3c(a.ax, r1.wx, r2.wx, r3.wx, c6, c23);
-  a.ay = rk3c(a.ay, r1.wy, r2.wy, r3.wy, c6, c23);
-  a.az = rk3c(a.az, r1.wz, r2.wz, r3.wz, c6, c23);
-  y[i] = a;
-}
-
-__global__ __launch_bounds__(kEW) void k_euler(Rec64* __restrict__ y,
-                                               const Rate64* __restrict__ k,
-                                               double dt, int n) {
-#pragma clang fp contract(off)
-  const int i = blockIdx.x * kEW + threadIdx.x;
-  if (i >= n) return;
-  Rec64 a = y[i];
-  const Rate64 r = k[i];
-  a.x = a.x + r.ux * dt;
-  a.y = a.y + r.uy * dt;
-  a.z = a.z + r.uz * dt;
-  a.ax = a.ax + r.wx * dt;
-  a.ay = a.ay + r.wy * dt;
-  a.az = a.az + r.wz * dt;
-  y[i] = a;
+template <int Sum, int Op>
+__global__ __launch_bounds__(Sum == 2 ? kGroupThreads : kEW) void k_finish(FinishArgs f) {
+  int64_t e;
+  double k;
+  if (Sum == 2) {
+    const SplitGroup g = f.groups[blockIdx.x];
+    if (static_cast<int>(threadIdx.x) >= 6 * (g.t1 - g.t0)) return;
+    e = 6 * static_cast<int64_t>(g.t0) + threadIdx.x;
+    const double* p = f.partial + static_cast<size_t>(g.first) * kGroupThreads + threadIdx.x;
+    k = p[0];
+#pragma unroll 8
+    for (int i = 1; i < g.count; ++i) k += p[static_cast<size_t>(i) * kGroupThreads];
+    f.rates[e] = k;
+  } else {
+    e = static_cast<int64_t>(blockIdx.x) * kEW + threadIdx.x;
+    const int64_t total = 6 * static_cast<int64_t>(f.n);
+    if (e >= total) return;
+    if (Sum == 1) {
+      k = f.partial[e];
+#pragma unroll 8
+      for (int i = 1; i < f.parts; ++i) k += f.partial[static_cast<size_t>(i) * total + e];
+      f.rates[e] = k;
+    } else {
+      k = f.rates[e];
+    }
+  }
+  if (!isfinite(k)) atomicOr(f.flag, 1);
+  stage_component<Op>(f.op, e, k);
 }
 
 __global__ __launch_bounds__(kEW) void k_check_finite(
@@ -171,44 +143,30 @@ hipError_t launch_add_rates(Rate64* acc, const Rate64* add, int first, int last,
   return hipGetLastError();
 }
 
-hipError_t launch_stage(const Rec64* y, const Rate64* k, double c, Rec64* out,
-                        int n, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_stage, dim3(ew_blocks(n)), dim3(kEW), 0, st, y, k, c, out, n);
-  return hipGetLastError();
+namespace {
+template <int Op>
+void finish_kernel(const SumForm& sum, const FinishArgs& f, hipStream_t st) {
+  const dim3 flat(static_cast<unsigned>((6 * static_cast<int64_t>(f.n) + kEW - 1) / kEW));
+  if (sum.groups) hipLaunchKernelGGL((k_finish<2, Op>), dim3(sum.ngroups), dim3(kGroupThreads), 0, st, f);
+  else if (sum.parts > 1) hipLaunchKernelGGL((k_finish<1, Op>), flat, dim3(kEW), 0, st, f);
+  else hipLaunchKernelGGL((k_finish<0, Op>), flat, dim3(kEW), 0, st, f);
 }
+}  // namespace
 
-hipError_t launch_rk4_final(Rec64* y, const Rate64* k1, const Rate64* k2,
-                            const Rate64* k3, const Rate64* k4, double c6,
-                            double c3, int n, hipStream_t st) {
+hipError_t launch_finish(const SumForm& sum, Rate64* rates, int n, int* flag, const StageOp& op, hipStream_t st) {
+  static_assert(sizeof(Rate64) == 6 * sizeof(double) && sizeof(Rec64) == 8 * sizeof(double), "flat components");
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rk4_final, dim3(ew_blocks(n)), dim3(kEW), 0, st, y, k1, k2, k3, k4,
-                     c6, c3, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_rk3_mid(const Rec64* y, Rate64* k1, const Rate64* k2,
-                          double dt, double two_dt, Rec64* out, int n,
-                          hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rk3_mid, dim3(ew_blocks(n)), dim3(kEW), 0, st, y, k1, k2, dt, two_dt,
-                     out, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_rk3_final(Rec64* y, const Rate64* k1, const Rate64* k2,
-                            const Rate64* k3, double c6, double c23, int n,
-                            hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rk3_final, dim3(ew_blocks(n)), dim3(kEW), 0, st, y, k1, k2, k3, c6,
-                     c23, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_euler(Rec64* y, const Rate64* k, double dt, int n,
-                        hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_euler, dim3(ew_blocks(n)), dim3(kEW), 0, st, y, k, dt, n);
+  const FinishArgs f{reinterpret_cast<const double*>(sum.partial), sum.parts, sum.groups,
+                     reinterpret_cast<double*>(rates), n, flag, op};
+  switch (op.kind) {
+    case kStageNone: finish_kernel<kStageNone>(sum, f, st); break;
+    case kStageLin: finish_kernel<kStageLin>(sum, f, st); break;
+    case kStageRk4: finish_kernel<kStageRk4>(sum, f, st); break;
+    case kStageRk3Mid: finish_kernel<kStageRk3Mid>(sum, f, st); break;
+    case kStageRk3: finish_kernel<kStageRk3>(sum, f, st); break;
+    case kStageEuler: finish_kernel<kStageEuler>(sum, f, st); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
