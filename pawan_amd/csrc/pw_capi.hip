@@ -93,6 +93,9 @@ void free_buffers(pw_ctx* c) {
   }
   (void)hipFree(c->partial);
   (void)hipFree(c->d_queue);
+  (void)hipFree(c->d_points);
+  c->d_points = nullptr;
+  c->points_len = 0;
   (void)hipFree(c->d_chunks);
   (void)hipFree(c->d_src32);
   (void)hipFree(c->d_src64);
@@ -594,6 +597,13 @@ int download_rates(pw_ctx* c, std::vector<Rate64>& h) {
   return PW_OK;
 }
 
+// velocities at m points on the device; the partial sums go to the second
+// rate array, which holds no result between calls
+hipError_t point_velocity(pw_ctx* c, const double* d_pts, int m, double* d_u) {
+  return pw::launch_point_velocity(c->y, static_cast<int>(c->n), d_pts, m, d_u, reinterpret_cast<double*>(c->k[1]),
+                                   6 * static_cast<size_t>(c->n), c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
+}
+
 }  // namespace
 
 namespace pwi {
@@ -875,22 +885,34 @@ int pw_velocity_at(pw_ctx* c, const double* points, int64_t m, double* u) {
   if (m == 0) return PW_OK;
   if (!points || !u) return fail(PW_ERR_ARG, "null points or output");
   PW_TRY(ensure_built(c));
-  double *d_pts = nullptr, *d_u = nullptr;
   const size_t len = 3 * static_cast<size_t>(m);
-  if (dalloc(&d_pts, len) != hipSuccess || dalloc(&d_u, len) != hipSuccess) {
-    (void)hipGetLastError();
-    (void)hipFree(d_pts);
-    return fail(PW_ERR_NOMEM, "point buffers");
+  // the points and their velocities pass through a buffer the context keeps
+  // (bounded: larger sets get one of their own)
+  constexpr size_t kKeepPoints = size_t(1) << 20;
+  double* own = nullptr;
+  double* d_pts = c->d_points;
+  if (2 * len > c->points_len) {
+    double* fresh = nullptr;
+    if (dalloc(&fresh, 2 * len) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(PW_ERR_NOMEM, "point buffers");
+    }
+    d_pts = fresh;
+    if (static_cast<size_t>(m) <= kKeepPoints) {
+      (void)hipFree(c->d_points);
+      c->d_points = fresh;
+      c->points_len = 2 * len;
+    } else {
+      own = fresh;
+    }
   }
+  double* d_u = d_pts + len;
   hipError_t e = hipMemcpyAsync(d_pts, points, len * sizeof(double), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess)
-    e = pw::launch_point_velocity(c->y, static_cast<int>(c->n), d_pts, static_cast<int>(m), d_u,
-                                  c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
+  if (e == hipSuccess) e = point_velocity(c, d_pts, static_cast<int>(m), d_u);
   if (e == hipSuccess) e = hipMemcpyAsync(u, d_u, len * sizeof(double), hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   else (void)hipStreamSynchronize(c->stream);  // nothing queued may still use the buffers
-  (void)hipFree(d_pts);
-  (void)hipFree(d_u);
+  (void)hipFree(own);
   if (e != hipSuccess) return fail(PW_ERR_HIP, std::string("pw_velocity_at: ") + hipGetErrorString(e));
   return PW_OK;
 }
@@ -913,9 +935,7 @@ int pw_velocity_at_noalloc(pw_ctx* c, const double* points, int64_t m, double* u
   double *d_pts = st, *d_u = st + 3 * kNoAllocPoints;
   const size_t bytes = 3 * static_cast<size_t>(m) * sizeof(double);
   hipError_t e = hipMemcpyAsync(d_pts, points, bytes, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess)
-    e = pw::launch_point_velocity(c->y, static_cast<int>(c->n), d_pts, static_cast<int>(m), d_u,
-                                  c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
+  if (e == hipSuccess) e = point_velocity(c, d_pts, static_cast<int>(m), d_u);
   if (e == hipSuccess) e = hipMemcpyAsync(u, d_u, bytes, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   else (void)hipStreamSynchronize(c->stream);

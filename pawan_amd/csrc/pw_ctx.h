@@ -124,6 +124,8 @@ struct pw_ctx {
   pw::Rate64* partial = nullptr;  // source-split partial rates (parts x n, or 64 rows per split item)
   size_t partial_rows = 0;
   int* d_queue = nullptr;     // work counter of the persistent kernels
+  double* d_points = nullptr; // points and velocities of pw_velocity_at
+  size_t points_len = 0;
   // source chunks of the scalar-fed FP32C kernel: runs of up to 64
   // particles of one system (chunk_first: their first particles, ascending)
   std::vector<int32_t> chunk_first;

@@ -373,9 +373,11 @@ constexpr int kVringMaxCells = 1024;
 hipError_t launch_vring_resolve(Rec64* y, int off, int m, int nazi, bool high_order, double* M,
                                 double* lu, const double* ideal, double* s, int* flag, hipStream_t st);
 
-// velocity at m points (AoS doubles, device) from the n particles of state
-hipError_t launch_point_velocity(const Rec64* state, int n, const double* pts, int m, double* u,
-                                 bool high_order, hipStream_t st);
+// velocity at m points (AoS doubles, device) from the n particles of state;
+// scratch: partial sums of split sources (as many splits as it holds, none if
+// null)
+hipError_t launch_point_velocity(const Rec64* state, int n, const double* pts, int m, double* u, double* scratch,
+                                 size_t scratch_doubles, bool high_order, hipStream_t st);
 // near field of the tree path (highorder: the algebraic kernel's pairs)
 hipError_t launch_near_fp32c(const Rec64* sorted, const NodeRec* nodes, const TreeBuffers& tb, int nleaf,
                              double nu, float sigma_max2, bool uniform_sigma, bool highorder, int grid,

@@ -46,10 +46,8 @@ constexpr int kTB = 256;  // targets per block = sources per LDS tile
 
 // 1/(4 pi) as the reference forms it (0.25 * M_1_PI, gaussian.h:35).
 constexpr double kQ = 0x1.45f306dc9c883p-4;
-// (2 pi)^1.5 (the divisor pow(2.0*M_PI,1.5) of gaussian.h:22) and its
-// reciprocal.
+// (2 pi)^1.5 (the divisor pow(2.0*M_PI,1.5) of gaussian.h:22).
 constexpr double kP15 = 0x1.f7fccdff344acp+3;
-constexpr double kK = 0x1.0411e71d77959p-4;
 constexpr double kSqrtHalf = 0.70710678118654752440;
 
 // FP64 far field: beyond rho^2 > 90 sigma^2, exp(-rho_bar^2/2) and
@@ -509,28 +507,52 @@ __device__ __forceinline__ void item_fp64_ho(const PairArgs& pa, const WorkItem&
 // Point-evaluation velocity (the reference's getVi,
 // src/interaction/interaction.cpp:453-476): the velocity at m arbitrary
 // points from every particle, with each particle's own radius as sigma,
-// in FP64 with the closed far form beyond 90 sigma^2.  One lane per point,
-// sources through LDS in tiles of 256 as in the pair kernels.  A point that
-// coincides with a particle gets no contribution from it (a_s x d = 0).
+// in FP64 with the closed far form beyond 90 sigma^2.  One block per (64
+// points, source range): its four waves hold the same points, one per lane,
+// and take a quarter of every 256-source LDS tile each; their sums are added
+// in wave order and, when the sources are split over several blocks, leave as
+// a 64-row slab that k_point_sum adds in order.  A point that coincides with a
+// particle gets no contribution from it (a_s x d = 0).
 // HighOrder: the algebraic kernel's q (highorder.h:31-39) instead.
+//
+// Few points against a large wake were the case to fix: with one lane per
+// point against every source, 1,200 points ran on 5 blocks, 105 ms a call
+// against 262,144 particles.  Split (launch_point_velocity), the same runs on
+// 2,052 blocks, 0.75 ms a call with its copies, FP64 issue-bound.
 // ---------------------------------------------------------------------
+struct PointArgs {
+  const Rec64* state;
+  int n;
+  const double* pts;
+  int m;
+  double* u;        // splits == 1
+  double* partial;  // (group, split) slabs of 64 x 3
+  int splits, range;  // source ranges, particles per range
+};
+
 template <bool HighOrder>
-__global__ __launch_bounds__(kTB) void k_point_velocity(const Rec64* __restrict__ state, int n,
-                                                        const double* __restrict__ pts, int m,
-                                                        double* __restrict__ u) {
+__global__ __launch_bounds__(kTB) void k_point_velocity(PointArgs a) {
+  constexpr int kWaves = kTB / 64;
   __shared__ Rec64 tile[kTB];
-  const int k = blockIdx.x * kTB + static_cast<int>(threadIdx.x);
-  const bool active = k < m;
-  const double px = active ? pts[3 * k] : 0.0, py = active ? pts[3 * k + 1] : 0.0,
-               pz = active ? pts[3 * k + 2] : 0.0;
-  double ux = 0.0, uy = 0.0, uz = 0.0;
-  for (int base = 0; base < n; base += kTB) {
-    const int cnt = min(kTB, n - base);
+  __shared__ double red[kWaves - 1][3][64];
+  __shared__ __align__(16) double tab[HighOrder ? 2 : kCore64Pieces * kCore64Row];
+  if (!HighOrder) stage_core64(tab);  // (synchronised with the first tile)
+  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+  const int g = static_cast<int>(blockIdx.x) / a.splits, part = static_cast<int>(blockIdx.x) % a.splits;
+  const int k = 64 * g + lane;
+  const bool active = k < a.m;
+  const size_t kp = 3 * static_cast<size_t>(active ? k : 64 * g);
+  const double px = a.pts[kp], py = a.pts[kp + 1], pz = a.pts[kp + 2];
+  const int s0 = part * a.range, s1 = min(a.n, s0 + a.range);
+  double u[3] = {0.0, 0.0, 0.0};
+  for (int base = s0; base < s1; base += kTB) {
+    const int cnt = min(kTB, s1 - base);
     __syncthreads();
-    if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = state[base + threadIdx.x];
+    if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = a.state[base + threadIdx.x];
     __syncthreads();
-    if (!active) continue;
-    for (int l = 0; l < cnt; ++l) {
+    const int l1 = cnt * (wave + 1) / kWaves;
+#pragma unroll 2
+    for (int l = cnt * wave / kWaves; l < l1; ++l) {
       const Rec64& s = tile[l];
       const double dx = px - s.x, dy = py - s.y, dz = pz - s.z;
       const double r2 = dx * dx + dy * dy + dz * dz;
@@ -541,29 +563,43 @@ __global__ __launch_bounds__(kTB) void k_point_velocity(const Rec64* __restrict_
         const double ib2 = ib * ib;
         q = kQ * fma(2.5, s.s2, r2) * (ib2 * ib2 * ib);
       } else {
-      const double ir = rsqrt_pos(r2);
-      const double ir2 = ir * ir;
-      q = kQ * (ir * ir2);
-      if (r2 <= kFar64 * s.s2) {
-        const double isg = rsqrt_pos(s.s2);
-        const double isg3 = isg * isg * isg;
-        const double rb = (r2 * ir) * isg;    // rho / sigma
-        const double irb = (s.s2 * isg) * ir;  // sigma / rho
-        const double Z = exp(-0.5 * rb * rb) * isg3 * kK;
-        const double phi = kQ * erf(kSqrtHalf * rb) * isg3;
-        q = (phi * irb - Z) * (irb * irb);
+        const double ir = rsqrt_pos(r2);
+        q = kQ * (ir * (ir * ir));
+        if (r2 <= kFar64 * s.s2) {
+          const double isg = rsqrt_pos(s.s2);
+          const double isg2 = isg * isg;
+          const double sb = r2 * isg2;
+          double e, gg;
+          core64(sb, tab, e, gg);
+          q = kCore64K * (isg2 * isg) * fma(sb, gg, e * (1.0 / 3.0));
+        }
       }
-      }
-      ux += q * (s.ay * dz - s.az * dy);
-      uy += q * (s.az * dx - s.ax * dz);
-      uz += q * (s.ax * dy - s.ay * dx);
+      u[0] += q * (s.ay * dz - s.az * dy);
+      u[1] += q * (s.az * dx - s.ax * dz);
+      u[2] += q * (s.ax * dy - s.ay * dx);
     }
   }
-  if (active) {
-    u[3 * k] = ux;
-    u[3 * k + 1] = uy;
-    u[3 * k + 2] = uz;
-  }
+  if (wave > 0)
+    for (int c = 0; c < 3; ++c) red[wave - 1][c][lane] = u[c];
+  __syncthreads();
+  if (wave > 0 || !active) return;
+  for (int w = 0; w < kWaves - 1; ++w)
+    for (int c = 0; c < 3; ++c) u[c] += red[w][c][lane];
+  double* out = a.splits > 1 ? a.partial + 192 * static_cast<size_t>(blockIdx.x) + 3 * lane
+                             : a.u + 3 * static_cast<size_t>(k);
+  for (int c = 0; c < 3; ++c) out[c] = u[c];
+}
+
+// u of a point group: its slabs added in order, one thread per component
+__global__ __launch_bounds__(192) void k_point_sum(const double* __restrict__ partial, int splits, int m,
+                                                   double* __restrict__ u) {
+  const int g = static_cast<int>(blockIdx.x), e = static_cast<int>(threadIdx.x);
+  if (64 * g + e / 3 >= m) return;
+  const double* p = partial + 192 * static_cast<size_t>(g) * splits + e;
+  double v = p[0];
+#pragma unroll 8
+  for (int i = 1; i < splits; ++i) v += p[192 * static_cast<size_t>(i)];
+  u[192 * static_cast<size_t>(g) + e] = v;
 }
 
 // ---------------------------------------------------------------------
@@ -2299,13 +2335,26 @@ const bool P = cfg.persistent;
   return hipGetLastError();
 }
 
-hipError_t launch_point_velocity(const Rec64* state, int n, const double* pts, int m, double* u,
-                                 bool high_order, hipStream_t st) {
+hipError_t launch_point_velocity(const Rec64* state, int n, const double* pts, int m, double* u, double* scratch,
+                                 size_t scratch_doubles, bool high_order, hipStream_t st) {
   if (m <= 0) return hipSuccess;
-  if (high_order)
-    hipLaunchKernelGGL(k_point_velocity<true>, dim3((m + kTB - 1) / kTB), dim3(kTB), 0, st, state, n, pts, m, u);
-  else
-    hipLaunchKernelGGL(k_point_velocity<false>, dim3((m + kTB - 1) / kTB), dim3(kTB), 0, st, state, n, pts, m, u);
+  PointArgs a{state, n, pts, m, u, scratch, 1, n};
+  const int groups = (m + 63) / 64;
+  // source ranges until about 2,048 blocks exist (two full rounds of 4 blocks
+  // per CU), whole 256-source tiles each, as far as the scratch holds the slabs
+  const int64_t want = std::min<int64_t>((2048 + groups - 1) / groups, (n + kTB - 1) / kTB);
+  const int64_t fits = scratch ? static_cast<int64_t>(scratch_doubles / (192 * static_cast<size_t>(groups))) : 0;
+  const int64_t splits = std::min(want, fits);
+  if (splits > 1) {
+    a.range = static_cast<int>((n + splits * kTB - 1) / (splits * kTB)) * kTB;
+    a.splits = (n + a.range - 1) / a.range;
+  }
+  const dim3 grid(static_cast<unsigned>(groups) * a.splits);
+  if (high_order) hipLaunchKernelGGL(k_point_velocity<true>, grid, dim3(kTB), 0, st, a);
+  else hipLaunchKernelGGL(k_point_velocity<false>, grid, dim3(kTB), 0, st, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.splits == 1) return e;
+  hipLaunchKernelGGL(k_point_sum, dim3(groups), dim3(192), 0, st, scratch, a.splits, m, u);
   return hipGetLastError();
 }
 
