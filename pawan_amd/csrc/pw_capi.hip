@@ -86,6 +86,11 @@ void free_buffers(pw_ctx* c) {
   (void)hipFree(c->lin_items);
   (void)hipFree(c->d_lin);
   (void)hipFree(c->d_quad);
+  (void)hipFree(c->diag_items);
+  (void)hipFree(c->d_diag_first);
+  c->diag_items = nullptr;
+  c->d_diag_first = nullptr;
+  c->ndiag = 0;
   (void)hipFree(c->d_flag);
   for (auto& k : c->ks) {
     (void)hipFree(k.d_items);
@@ -147,7 +152,6 @@ int32_t chunk_of(const pw_ctx* c, int64_t s) {
 // grid is made of short blocks.
 void build_items(pw_ctx* c) {
   c->h_pair_items.clear();
-  c->pair_sys.clear();
   c->h_lin_items.clear();
   c->lin_wake.clear();
   const int nw = static_cast<int>(c->wn.size());
@@ -169,7 +173,6 @@ void build_items(pw_ctx* c) {
       c->h_pair_items.push_back({static_cast<int32_t>(t0),
                                  static_cast<int32_t>(std::min<int64_t>(t0 + kTargetsPerItem, s.b)),
                                  static_cast<int32_t>(s.a), static_cast<int32_t>(s.b), -1, 0, 0, 0});
-      c->pair_sys.push_back(s.id);
     }
   for (int w = 0; w < nw; ++w)
     for (int64_t t0 = c->woff[w]; t0 < c->woff[w + 1]; t0 += kTargetsPerItem) {
@@ -208,7 +211,6 @@ int ensure_built(pw_ctx* c) {
       dalloc(&c->pair_items, c->h_pair_items.size()) != hipSuccess ||
       dalloc(&c->lin_items, c->h_lin_items.size()) != hipSuccess ||
       dalloc(&c->d_lin, 11 * c->h_lin_items.size()) != hipSuccess ||
-      dalloc(&c->d_quad, pw::kDiagQuad * c->h_pair_items.size()) != hipSuccess ||
       dalloc(&c->d_flag, 1) != hipSuccess || dalloc(&c->d_queue, 1) != hipSuccess ||
       dalloc(&c->d_chunks, static_cast<size_t>(c->nchunks)) != hipSuccess ||
       dalloc(&c->d_src32, n) != hipSuccess) {
@@ -465,6 +467,64 @@ void append_items(const pw_ctx* c, int a, int b, int nself, std::vector<WorkItem
     out.push_back({static_cast<int32_t>(t0), static_cast<int32_t>(std::min<int64_t>(t0 + kTargetsPerItem, c->woff[a + 1])),
                    static_cast<int32_t>(c->woff[b]), static_cast<int32_t>(c->woff[b + 1]), -1, nself,
                    chunk_of(c, c->woff[b]), 0});
+}
+
+// Source range of the diagnostics' pair items over `systems` ([a, b) each):
+// the longest of 64 ... 1,024 particles that leaves ten blocks per CU (short
+// ranges cost the staging of a block's tiles and table per few pairs), longer
+// where the items would exceed 131,072.
+int diag_range(const std::vector<std::pair<int64_t, int64_t>>& systems) {
+  const auto count = [&](int64_t range) {
+    int64_t items = 0;
+    for (const auto& s : systems) {
+      const int64_t len = s.second - s.first;
+      items += (len + 63) / 64 * ((len + range - 1) / range + 1) / 2;
+    }
+    return items;
+  };
+  int range = 64;
+  while (range < 1024 && count(2 * range) >= 2560) range *= 2;
+  while (range < (1 << 28) && count(range) > 131072) range *= 2;
+  return range;
+}
+
+// pair items of one system's unordered pairs
+void append_diag_items(int64_t a, int64_t b, int range, std::vector<WorkItem>& out) {
+  for (int64_t t0 = a; t0 < b; t0 += 64) {
+    const int64_t t1 = std::min<int64_t>(t0 + 64, b);
+    for (int64_t s0 = a; s0 < t1; s0 += range)
+      out.push_back({static_cast<int32_t>(t0), static_cast<int32_t>(t1), static_cast<int32_t>(s0),
+                     static_cast<int32_t>(std::min<int64_t>(s0 + range, t1)), -1, 0, 0, 0});
+  }
+}
+
+int ensure_diag(pw_ctx* c) {
+  if (c->diag_items) return PW_OK;
+  // systems in their own order (c->systems is sorted by size)
+  std::vector<std::pair<int64_t, int64_t>> sys(c->nsys());
+  for (const auto& s : c->systems) sys[s.id] = {s.a, s.b};
+  std::vector<WorkItem> items;
+  std::vector<int> first{0};
+  const int range = diag_range(sys);
+  for (const auto& s : sys) {
+    append_diag_items(s.first, s.second, range, items);
+    first.push_back(static_cast<int>(items.size()));
+  }
+  // each item's sums, then each system's
+  const size_t rows = items.size() + sys.size();
+  if (dalloc(&c->diag_items, items.size()) != hipSuccess || dalloc(&c->d_diag_first, first.size()) != hipSuccess ||
+      dalloc(&c->d_quad, pw::kDiagQuad * rows) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFree(c->diag_items);
+    (void)hipFree(c->d_diag_first);
+    c->diag_items = nullptr;
+    c->d_diag_first = nullptr;
+    return fail(PW_ERR_NOMEM, "diagnostic buffers");
+  }
+  PW_HIP(hipMemcpy(c->diag_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
+  PW_HIP(hipMemcpy(c->d_diag_first, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice));
+  c->ndiag = static_cast<int>(items.size());
+  return PW_OK;
 }
 
 // One right-hand side f(state) -> out, with optional event timing, and the
@@ -1268,7 +1328,16 @@ int pw_diagnose_wakes(pw_ctx* c, int wa, int wb, double* out, int64_t out_len) {
   PW_TRY(check_blocks(c, pair, 1));
   PW_TRY(ensure_built(c));
   std::vector<WorkItem> items;
-  append_items(c, wa, wb, wa == wb ? 0 : 1, items);
+  if (wa == wb) {
+    append_diag_items(c->woff[wa], c->woff[wa + 1], diag_range({{c->woff[wa], c->woff[wa + 1]}}), items);
+  } else {
+    // every source of wake b, 1,024 at a time, for each 64 targets of wake a
+    for (int64_t t0 = c->woff[wa]; t0 < c->woff[wa + 1]; t0 += 64)
+      for (int64_t s0 = c->woff[wb]; s0 < c->woff[wb + 1]; s0 += 1024)
+        items.push_back({static_cast<int32_t>(t0), static_cast<int32_t>(std::min<int64_t>(t0 + 64, c->woff[wa + 1])),
+                         static_cast<int32_t>(s0), static_cast<int32_t>(std::min<int64_t>(s0 + 1024, c->woff[wb + 1])),
+                         -1, 1, 0, 0});
+  }
   constexpr int Q = pw::kDiagQuad;
   const int ni = static_cast<int>(items.size());
   // the wake's linear-sum items are contiguous in the context's list
@@ -1321,9 +1390,8 @@ int pw_diagnose_wakes(pw_ctx* c, int wa, int wb, double* out, int64_t out_len) {
   double q[Q] = {0};
   for (int b = 0; b < ni; ++b)
     for (int m = 0; m < Q; ++m) q[m] += quad[Q * b + m];
-  // ordered sum over the block's (target, source) pairs: within a wake it is
-  // 2 sum_{i<j} plus the self terms; across wakes one direction, doubled as
-  // in calculate*(W1, W2) (interaction.cpp:551-718)
+  // within a wake 2 sum_{i<j} plus the self terms; across wakes one
+  // direction, doubled as in calculate*(W1, W2) (interaction.cpp:551-718)
   const double f = wa == wb ? 1.0 : 2.0;
   out[9] = f * q[0];   // helicity
   out[10] = f * q[3];  // enstrophy
@@ -1340,26 +1408,23 @@ int pw_diagnose(pw_ctx* c, double* out, int64_t out_len) {
   const int ns = c->nsys();
   if (out_len < 15 * static_cast<int64_t>(ns))
     return fail(PW_ERR_ARG, "output needs 15 doubles per system");
+  PW_TRY(ensure_diag(c));
   PW_HIP(pw::launch_diag_linear(c->y, c->lin_items, c->nlin, c->d_lin, c->stream));
   const bool ho = c->smoothing == PW_KERNEL_HIGHORDER;
   constexpr int Q = pw::kDiagQuad;
-  PW_HIP(pw::launch_diag_pairs(c->y, c->d_radius, c->pair_items, c->npair, c->d_quad, ho, c->stream));
-  std::vector<double> lin(11 * static_cast<size_t>(c->nlin)), quad(Q * static_cast<size_t>(c->npair));
+  double* d_sys = c->d_quad + Q * static_cast<size_t>(c->ndiag);
+  PW_HIP(pw::launch_diag_pairs(c->y, c->d_radius, c->diag_items, c->ndiag, c->d_quad, ho, c->stream));
+  PW_HIP(pw::launch_diag_sum(c->d_quad, c->d_diag_first, ns, d_sys, c->stream));
+  std::vector<double> lin(11 * static_cast<size_t>(c->nlin)), sq(Q * static_cast<size_t>(ns));
   PW_HIP(hipMemcpyAsync(lin.data(), c->d_lin, lin.size() * sizeof(double), hipMemcpyDeviceToHost,
                         c->stream));
-  PW_HIP(hipMemcpyAsync(quad.data(), c->d_quad, quad.size() * sizeof(double),
-                        hipMemcpyDeviceToHost, c->stream));
+  PW_HIP(hipMemcpyAsync(sq.data(), d_sys, sq.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   PW_HIP(hipStreamSynchronize(c->stream));
   const int nw = static_cast<int>(c->wn.size());
   // per-wake linear sums in block order
   std::vector<double> wl(11 * static_cast<size_t>(nw), 0.0);
   for (int b = 0; b < c->nlin; ++b)
     for (int m = 0; m < 11; ++m) wl[11 * c->lin_wake[b] + m] += lin[11 * b + m];
-  // per-system quadratic sums in item order (items of one system are
-  // contiguous and in target order)
-  std::vector<double> sq(Q * static_cast<size_t>(ns), 0.0);
-  for (int b = 0; b < c->npair; ++b)
-    for (int m = 0; m < Q; ++m) sq[Q * c->pair_sys[b] + m] += quad[Q * b + m];
   for (int s = 0; s < ns; ++s) {
     double* o = out + 15 * s;
     for (int m = 0; m < 9; ++m) o[m] = 0.0;

@@ -103,8 +103,13 @@ struct pw_ctx {
   pw::WorkItem* lin_items = nullptr;
   int nlin = 0;
   std::vector<pw::WorkItem> h_pair_items, h_lin_items;
-  std::vector<int> pair_sys, lin_wake;  // system / wake of each item
+  std::vector<int> lin_wake;  // wake of each linear-sum item
   double* d_lin = nullptr;
+  // diagnostics: pair items of every system (first use), their sums, and the
+  // items of system s, [diag_first[s], diag_first[s + 1])
+  pw::WorkItem* diag_items = nullptr;
+  int ndiag = 0;
+  int* d_diag_first = nullptr;
   double* d_quad = nullptr;
   int* d_flag = nullptr;
 

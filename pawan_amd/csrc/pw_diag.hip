@@ -10,12 +10,13 @@
 //     div-free variant (interaction_utils.h:107-331; the enstrophies are
 //     identically zero for the Gaussian kernel, gaussian.h:69-92, and
 //     nonzero for the high-order algebraic one, highorder.h:77-106).
-// Both are computed here as per-block partial sums in a fixed tree order;
-// the host adds the partials in block order, so results are deterministic.
-// Pair terms are symmetric in the two particles, so the ordered sum over
-// j != i equals the reference's 2 * sum over i < j.
+// Both are computed here as per-block partial sums in a fixed tree order, and
+// the partials are added in a fixed order, so results are deterministic.
+// Pair terms are symmetric in the two particles: each unordered pair of a
+// system is evaluated once, with the weight 2 of the reference's sums.
 #include <hip/hip_runtime.h>
 
+#include "pw_core64.h"
 #include "pw_internal.h"
 
 namespace pw {
@@ -25,8 +26,7 @@ constexpr int kTB = 256;
 constexpr double kPi = 3.14159265358979323846;
 constexpr double k1Pi = 0.31830988618379067154;  // M_1_PI
 constexpr double kQ = 0x1.45f306dc9c883p-4;      // 0.25 * M_1_PI
-constexpr double kP15 = 0x1.f7fccdff344acp+3;    // pow(2 pi, 1.5)
-constexpr double kSqrtHalf = 0.70710678118654752440;
+constexpr double kFar64 = 90.0;                  // beyond 90 sigma^2 the Gaussian terms are below FP64 rounding
 
 // Sum of v over the block, exact same tree every call: butterfly within
 // each 64-lane wavefront, then the four wave totals in wave order.
@@ -80,119 +80,139 @@ __global__ __launch_bounds__(kTB) void k_diag_linear(
     for (int m = 0; m < 11; ++m) out[blockIdx.x * 11 + m] = v[m];
 }
 
-// QSIG (gaussian.h:30-37) with the reference's operation order.
-__device__ __forceinline__ double qsig(double rho, double sigma) {
-#pragma clang fp contract(off)
-  const double rho_bar = rho / sigma;
-  const double sig3 = sigma * sigma * sigma;
-  const double Z = exp(-0.5 * rho_bar * rho_bar) / sig3 / kP15;
-  const double phi = kQ * erf(kSqrtHalf * rho_bar) / sig3;
-  return (phi / rho_bar - Z) / (rho_bar * rho_bar);
+// 1/sqrt(x) for positive finite x: the hardware estimate and one third-order
+// correction (relative error below 2^-52)
+__device__ __forceinline__ double rsqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// QSIG of the high-order algebraic kernel (highorder.h:31-39), same
-// operation order, pow(x, 2.5) as x^2 sqrt(x).
-__device__ __forceinline__ double qsig_ho(double rho, double sigma) {
-#pragma clang fp contract(off)
-  const double rho_bar = rho / sigma;
-  const double rho_bar2 = rho_bar * rho_bar;
-  const double rho3 = rho * rho * rho;
-  const double b = rho_bar2 + 1.0;
-  return 0.25 * k1Pi * rho_bar2 * rho_bar * (rho_bar2 + 2.5) / (b * b * sqrt(b)) / rho3;
+// Sums of one target's pairs, the constants of the energies factored out.
+struct DiagSum {
+  double h = 0.0, ke = 0.0, kef = 0.0, en = 0.0, enf = 0.0;
+};
+
+// helicity, KE, KEF (and, for the high-order kernel, the two enstrophies) of
+// one pair (interaction_utils.h:141-331), I = target, J = source
+template <bool HighOrder>
+__device__ __forceinline__ void diag_pair(const Rec64& me, const Rec64& s, const double* __restrict__ tab,
+                                          DiagSum& d) {
+  const double x0 = s.x - me.x, x1 = s.y - me.y, x2 = s.z - me.z;  // x12 = x_J - x_I
+  const double rho2 = x0 * x0 + x1 * x1 + x2 * x2;
+  const double sigma2 = 0.5 * (me.s2 + s.s2);
+  const double ib = rsqrt_pos(rho2 + sigma2);
+  const double ib2 = ib * ib, ib3 = ib2 * ib;
+  double q;
+  if (HighOrder) {
+    // QSIG (highorder.h:31-39) in closed form; 0/0 for coincident particles
+    q = kQ * fma(2.5, sigma2, rho2) * (ib3 * ib2);
+    if (rho2 == 0.0) q = __builtin_nan("");
+  } else {
+    const double ir = rsqrt_pos(rho2);
+    q = kQ * (ir * (ir * ir));
+    if (rho2 <= kFar64 * sigma2) {
+      const double isg = rsqrt_pos(sigma2);
+      const double isg2 = isg * isg;
+      double e, g;
+      const double sb = fma(ir, 0.0, rho2 * isg2);  // not finite for coincident particles, as in the reference
+      core64(sb, tab, e, g);
+      q = kCore64K * (isg2 * isg) * fma(sb, g, e * (1.0 / 3.0));
+    }
+  }
+  const double c0 = me.ay * s.az - me.az * s.ay;
+  const double c1 = me.az * s.ax - me.ax * s.az;
+  const double c2 = me.ax * s.ay - me.ay * s.ax;
+  d.h = fma(q, x0 * c0 + x1 * c1 + x2 * c2, d.h);
+  const double a1a2 = me.ax * s.ax + me.ay * s.ay + me.az * s.az;
+  const double xx = (x0 * me.ax + x1 * me.ay + x2 * me.az) * (x0 * s.ax + x1 * s.ay + x2 * s.az);
+  // ((rho^2 + 2 sigma^2) a1.a2 + (x12.a1)(x12.a2)) / b^1.5 / 16 pi and
+  // (rho^2 + 1.5 sigma^2) a1.a2 / b^1.5 / 8 pi (:278-331)
+  const double a3 = a1a2 * ib3;
+  d.ke = fma(ib3, xx, fma(fma(2.0, sigma2, rho2), a3, d.ke));
+  d.kef = fma(fma(1.5, sigma2, rho2), a3, d.kef);
+  if (HighOrder) {
+    // ENST / ENSTF (highorder.h:77-96): F1 a1.a2 + F2 (x12.a1)(x12.a2), b^3.5 below
+    const double ib7 = ib3 * (ib2 * ib2);
+    const double r4 = rho2 * rho2, rs = rho2 * sigma2, s4 = sigma2 * sigma2;
+    const double f1 = 2.0 * r4 + 7.0 * rs + 20.0 * s4;
+    const double f2 = 6.0 * r4 + 27.0 * rs + 21.0 * s4;
+    d.en = fma(ib7, fma(f1, a1a2, -(f2 * ib2) * xx), d.en);
+    d.enf = fma(s4 * ib7, a1a2, d.enf);
+  }
 }
 
-// Per-target rows of helicity, KE, KEF (and, for the high-order kernel,
-// enstrophy and its div-free variant) over one work item's sources; the
-// block total goes to out[kDiagQuad * b].  radius is needed for the self
-// terms.
+// One item: its targets [t0, t1) (at most 64, one per lane of each of the
+// block's four waves) against its sources [s0, s1), a quarter of each
+// 256-source tile per wave.  nself = 0: a range of the targets' own system,
+// of which only the sources before the target count, twice, and the item
+// whose range ends with the targets adds their self terms; nself = 1: a
+// cross-wake block, every source once, no self terms.  The block total goes
+// to out[kDiagQuad * b].
+//
+// The ordered pairs of 94 blocks, each with an exp, an erf, two square roots
+// and seven divisions, took 18.7 ms for 24,000 particles; unordered, split
+// over 9,000 blocks and with the divisions taken out (about 60 instructions a
+// pair, the core from pw_core64.h) FP64 issue bounds it.
 template <bool HighOrder>
 __global__ __launch_bounds__(kTB) void k_diag_pairs(
     const Rec64* __restrict__ y, const double* __restrict__ radius,
     const WorkItem* __restrict__ items, double* __restrict__ out) {
-#pragma clang fp contract(off)
+  constexpr int kWaves = kTB / 64;
   __shared__ Rec64 tile[kTB];
-  __shared__ double red[(kTB / 64) * kDiagQuad];
+  __shared__ double red[kWaves * kDiagQuad];
+  __shared__ __align__(16) double tab[HighOrder ? 2 : kCore64Pieces * kCore64Row];
+  if (!HighOrder) stage_core64(tab);  // (synchronised with the first tile)
   const WorkItem it = items[blockIdx.x];
-  const int t = it.t0 + static_cast<int>(threadIdx.x);
+  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+  const int t = it.t0 + lane;
   const bool active = t < it.t1;
+  const bool cross = it.nself != 0;
   const Rec64 me = y[active ? t : it.t0];
-  double h = 0.0, ke = 0.0, kef = 0.0, en = 0.0, enf = 0.0;
+  DiagSum d;
   for (int base = it.s0; base < it.s1; base += kTB) {
     const int cnt = min(kTB, it.s1 - base);
     __syncthreads();
     if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = y[base + threadIdx.x];
     __syncthreads();
-    if (active) {
-      for (int l = 0; l < cnt; ++l) {
-        if (base + l == t) continue;
-        const Rec64 s = tile[l];
-        // x12 = x_J - x_I with I = target, J = source
-        const double x0 = s.x - me.x, x1 = s.y - me.y, x2 = s.z - me.z;
-        double rho2 = 0.0;
-        rho2 += x0 * x0;
-        rho2 += x1 * x1;
-        rho2 += x2 * x2;
-        // HELICITY (interaction_utils.h:214-242)
-        const double rho = sqrt(rho2);
-        const double sigma = sqrt(0.5 * (me.s2 + s.s2));
-        const double q = HighOrder ? qsig_ho(rho, sigma) : qsig(rho, sigma);
-        const double c0 = me.ay * s.az - me.az * s.ay;
-        const double c1 = me.az * s.ax - me.ax * s.az;
-        const double c2 = me.ax * s.ay - me.ay * s.ax;
-        double roaxa = 0.0;
-        roaxa += x0 * c0;
-        roaxa += x1 * c1;
-        roaxa += x2 * c2;
-        h += q * roaxa;
-        // KINETICENERGY / KINETICENERGYF (:278-331)
-        const double sigma2 = 0.5 * (me.s2 + s.s2);
-        double a1a2 = 0.0, x12a1 = 0.0, x12a2 = 0.0;
-        a1a2 += me.ax * s.ax;
-        a1a2 += me.ay * s.ay;
-        a1a2 += me.az * s.az;
-        x12a1 += x0 * me.ax;
-        x12a1 += x1 * me.ay;
-        x12a1 += x2 * me.az;
-        x12a2 += x0 * s.ax;
-        x12a2 += x1 * s.ay;
-        x12a2 += x2 * s.az;
-        const double b = rho2 + sigma2;
-        const double p15 = b * sqrt(b);  // pow(b, 1.5)
-        ke += ((rho2 + 2.0 * sigma2) * a1a2 + (x12a1 * x12a2)) / p15 / 16.0 / kPi;
-        kef += (rho2 + 1.5 * sigma2) * a1a2 / p15 / 8.0 / kPi;
-        if (HighOrder) {
-          // ENSTROPHY / ENSTROPHYF pairs (interaction_utils.h:141-202) with
-          // ENST / ENSTF (highorder.h:77-96); sqrt(b^7) as b^3 sqrt(b)
-          const double sig2 = sigma * sigma;
-          const double bb = rho2 + sig2;
-          const double s7 = bb * bb * bb * sqrt(bb);
-          const double factor = (k1Pi / 8.0) / s7;
-          const double F1 = factor * (2.0 * rho2 * rho2 + 7.0 * sig2 * rho2 + 20.0 * sig2 * sig2);
-          const double F2 = factor * (-6.0 * rho2 * rho2 - 27.0 * sig2 * rho2 - 21.0 * sig2 * sig2) / bb;
-          en += F1 * a1a2 + F2 * x12a1 * x12a2;
-          enf += (15.0 * k1Pi * sig2 * sig2 / 8.0) / s7 * a1a2;
-        }
-      }
+    const int l0 = cnt * wave / kWaves, l1 = cnt * (wave + 1) / kWaves;
+    if (cross || base + l1 <= it.t0) {
+#pragma unroll 2
+      for (int l = l0; l < l1; ++l) diag_pair<HighOrder>(me, tile[l], tab, d);
+    } else {
+      for (int l = l0; l < l1; ++l)
+        if (base + l < t) diag_pair<HighOrder>(me, tile[l], tab, d);
     }
   }
-  if (active && it.nself == 0) {
-    // self terms (interaction_utils.h:249-267); items of a cross-wake block
-    // (nself = 1) have none
+  const double f = cross ? 1.0 : 2.0;
+  double v[kDiagQuad] = {active ? f * d.h : 0.0, active ? f * d.ke / 16.0 / kPi : 0.0,
+                         active ? f * d.kef / 8.0 / kPi : 0.0, active ? f * d.en * (k1Pi / 8.0) : 0.0,
+                         active ? f * d.enf * (15.0 * k1Pi / 8.0) : 0.0};
+  if (active && !cross && wave == 0 && it.s1 == it.t1) {
+    // self terms (interaction_utils.h:249-267)
     const double sg = radius[t];
-    double a2 = 0.0;
-    a2 += me.ax * me.ax;
-    a2 += me.ay * me.ay;
-    a2 += me.az * me.az;
-    ke += k1Pi * a2 / sg / 8.0;
-    kef += 3 * k1Pi * a2 / (sg * 16.0);
+    const double a2 = me.ax * me.ax + me.ay * me.ay + me.az * me.az;
+    v[1] += k1Pi * a2 / sg / 8.0;
+    v[2] += 3 * k1Pi * a2 / (sg * 16.0);
     if (HighOrder) {
       // ENST(sigma), ENSTF(sigma) (highorder.h:98-106)
-      en += 5.0 * k1Pi / 2.0 / (sg * sg * sg) * a2;
-      enf += 15.0 * k1Pi / 8.0 / (sg * sg * sg) * a2;
+      v[3] += 5.0 * k1Pi / 2.0 / (sg * sg * sg) * a2;
+      v[4] += 15.0 * k1Pi / 8.0 / (sg * sg * sg) * a2;
     }
   }
-  double v[kDiagQuad] = {active ? h : 0.0, active ? ke : 0.0, active ? kef : 0.0,
-                         active ? en : 0.0, active ? enf : 0.0};
+  block_sum<kDiagQuad>(v, red);
+  if (threadIdx.x == 0)
+    for (int m = 0; m < kDiagQuad; ++m) out[kDiagQuad * blockIdx.x + m] = v[m];
+}
+
+// out[kDiagQuad * s + m] = sum of the items [first[s], first[s + 1]): one
+// block per system, lanes over the items, then the fixed tree
+__global__ __launch_bounds__(kTB) void k_diag_sum(const double* __restrict__ items, const int* __restrict__ first,
+                                                  double* __restrict__ out) {
+  __shared__ double red[(kTB / 64) * kDiagQuad];
+  double v[kDiagQuad] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  for (int i = first[blockIdx.x] + static_cast<int>(threadIdx.x); i < first[blockIdx.x + 1]; i += kTB)
+    for (int m = 0; m < kDiagQuad; ++m) v[m] += items[static_cast<size_t>(kDiagQuad) * i + m];
   block_sum<kDiagQuad>(v, red);
   if (threadIdx.x == 0)
     for (int m = 0; m < kDiagQuad; ++m) out[kDiagQuad * blockIdx.x + m] = v[m];
@@ -215,6 +235,12 @@ hipError_t launch_diag_pairs(const Rec64* y, const double* radius,
     hipLaunchKernelGGL(k_diag_pairs<true>, dim3(nitems), dim3(kTB), 0, st, y, radius, items, out);
   else
     hipLaunchKernelGGL(k_diag_pairs<false>, dim3(nitems), dim3(kTB), 0, st, y, radius, items, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_diag_sum(const double* items, const int* first, int nsys, double* out, hipStream_t st) {
+  if (nsys <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_diag_sum, dim3(nsys), dim3(kTB), 0, st, items, first, out);
   return hipGetLastError();
 }
 

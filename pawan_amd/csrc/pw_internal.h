@@ -181,13 +181,18 @@ hipError_t launch_vorticity_field(const Rec64* y, const WorkItem* items, int nit
 // [a (3), x x a (3), x x (x x a) (3), |a| z (x^2+y^2), |a| (x^2+y^2)].
 hipError_t launch_diag_linear(const Rec64* y, const WorkItem* items,
                               int nitems, double* out, hipStream_t st);
-// Quadratic sums over the pair work items: out[kDiagQuad * b + m] gets the
-// block's total of [helicity, KE, KEF, enstrophy, div-free enstrophy] rows
+// Quadratic sums over pair items of at most 64 targets: out[kDiagQuad * b + m]
+// gets the item's total of [helicity, KE, KEF, enstrophy, div-free enstrophy]
 // (self terms included; the enstrophies are zero for the Gaussian kernel).
+// Items of one system (nself 0) count the sources before each target, twice:
+// together the ranges of a target group cover its system up to the group's
+// end, and the last one ends with it.  nself 1: a cross-wake block.
 constexpr int kDiagQuad = 5;
 hipError_t launch_diag_pairs(const Rec64* y, const double* radius,
                              const WorkItem* items, int nitems, double* out,
                              bool high_order, hipStream_t st);
+// out[kDiagQuad * s + m] = total of the items [first[s], first[s + 1])
+hipError_t launch_diag_sum(const double* items, const int* first, int nsys, double* out, hipStream_t st);
 
 // ---------------------------------------------------------------------
 // Cluster tree of the learned far field.
