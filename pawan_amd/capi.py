@@ -299,15 +299,22 @@ class Solver:
         _check(self._lib.pw_get_wake_rates(self._h, w, vel, ret))
         return vel, ret
 
+    def _all_wakes(self, get):
+        """Two N x 3 arrays, wake after wake, filled by get(ctx, wake, a, b)."""
+        first, second = np.empty((self.n, 3)), np.empty((self.n, 3))
+        at = 0
+        for w, n in enumerate(self.wake_sizes):
+            _check(get(self._h, w, first[at:at + n], second[at:at + n]))
+            at += n
+        return first, second
+
     def state(self):
         """(pos, alpha) of all particles, wakes concatenated."""
-        parts = [self.wake_state(w) for w in range(len(self.wake_sizes))]
-        return np.concatenate([p for p, _ in parts]), np.concatenate([a for _, a in parts])
+        return self._all_wakes(self._lib.pw_get_wake_state)
 
     def rates(self):
         """(vel, retvor) of all particles from the last right-hand side."""
-        parts = [self.wake_rates(w) for w in range(len(self.wake_sizes))]
-        return np.concatenate([p for p, _ in parts]), np.concatenate([a for _, a in parts])
+        return self._all_wakes(self._lib.pw_get_wake_rates)
 
     def set_states(self, state: np.ndarray) -> None:
         state = np.ascontiguousarray(state, dtype=np.float64)

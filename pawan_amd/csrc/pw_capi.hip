@@ -12,6 +12,7 @@
 #include <new>
 #include <tuple>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -91,7 +92,11 @@ void free_buffers(pw_ctx* c) {
   c->diag_items = nullptr;
   c->d_diag_first = nullptr;
   c->ndiag = 0;
-  (void)hipFree(c->d_flag);
+  (void)hipHostFree(c->h_flag);
+  (void)hipHostFree(c->h_stage);
+  c->h_flag = nullptr;
+  c->h_stage = nullptr;
+  c->stage_particles = 0;
   for (auto& k : c->ks) {
     (void)hipFree(k.d_items);
     (void)hipFree(k.d_groups);
@@ -113,7 +118,7 @@ void free_buffers(pw_ctx* c) {
   c->d_radius = nullptr;
   c->pair_items = c->lin_items = nullptr;
   c->d_lin = c->d_quad = nullptr;
-  c->d_flag = c->d_queue = nullptr;
+  c->d_queue = nullptr;
   for (auto& k : c->ks) {
     k.d_items = nullptr;
     k.d_groups = nullptr;
@@ -211,7 +216,8 @@ int ensure_built(pw_ctx* c) {
       dalloc(&c->pair_items, c->h_pair_items.size()) != hipSuccess ||
       dalloc(&c->lin_items, c->h_lin_items.size()) != hipSuccess ||
       dalloc(&c->d_lin, 11 * c->h_lin_items.size()) != hipSuccess ||
-      dalloc(&c->d_flag, 1) != hipSuccess || dalloc(&c->d_queue, 1) != hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void**>(&c->h_flag), sizeof(int), hipHostMallocCoherent) != hipSuccess ||
+      dalloc(&c->d_queue, 1) != hipSuccess ||
       dalloc(&c->d_chunks, static_cast<size_t>(c->nchunks)) != hipSuccess ||
       dalloc(&c->d_src32, n) != hipSuccess) {
     free_buffers(c);  // the stream stays: the context remains usable
@@ -240,10 +246,7 @@ int ensure_built(pw_ctx* c) {
                         c->h_lin_items.size() * sizeof(WorkItem), hipMemcpyHostToDevice,
                         c->stream));
   // rates start at zero (a calloc'd rate vector in the reference)
-  std::vector<Rate64> zero(n);
-  std::memset(zero.data(), 0, n * sizeof(Rate64));
-  PW_HIP(hipMemcpyAsync(c->k[0], zero.data(), n * sizeof(Rate64), hipMemcpyHostToDevice,
-                        c->stream));
+  PW_HIP(pw::launch_zero_doubles(reinterpret_cast<double*>(c->k[0]), 6 * c->n, c->stream));
   PW_HIP(hipStreamSynchronize(c->stream));
   c->rates = c->k[0];
   c->zc.assign(c->nsys(), 0.0);
@@ -542,7 +545,7 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp&
       PW_HIP(hipEventRecord(e1, c->stream));
       c->ev_used.emplace_back(e0, e1);
     }
-    PW_HIP(pw::launch_finish(pw::SumForm{}, out, n, c->d_flag, op, c->stream));
+    PW_HIP(pw::launch_finish(pw::SumForm{}, out, n, c->h_flag, op, c->stream));
     return PW_OK;
   }
   if (kind == pw::kPairFP32C && !c->compensated && c->smoothing == PW_KERNEL_GAUSSIAN) {
@@ -550,7 +553,7 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp&
     pw::PairArgs args{state, c->pair_items, c->npair, n, out, nullptr, c->d_queue, c->nu,
                       c->d_chunks, c->d_src32, nullptr, c->nchunks};
     PW_HIP(pw::launch_pair(pw::kPairFP32CPlain, pw::PairConfig{}, args, c->npair, c->stream));
-    PW_HIP(pw::launch_finish(pw::SumForm{}, out, n, c->d_flag, op, c->stream));
+    PW_HIP(pw::launch_finish(pw::SumForm{}, out, n, c->h_flag, op, c->stream));
     return PW_OK;
   }
   PW_TRY(ensure_kind(c, kind));
@@ -589,16 +592,22 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp&
     PW_HIP(hipEventRecord(e1, c->stream));
     c->ev_used.emplace_back(e0, e1);
   }
-  PW_HIP(pw::launch_finish(sum, out, n, c->d_flag, op, c->stream));
+  PW_HIP(pw::launch_finish(sum, out, n, c->h_flag, op, c->stream));
+  return PW_OK;
+}
+
+// The flag is host memory the kernels write: cleared once nothing queued can
+// still write it.
+int clear_flag(pw_ctx* c) {
+  PW_HIP(hipStreamSynchronize(c->stream));
+  *static_cast<volatile int*>(c->h_flag) = 0;
   return PW_OK;
 }
 
 int check_flag(pw_ctx* c, const char* what) {
   PW_TRY(pwi::ff_check(c));
-  int flag = 0;
-  PW_HIP(hipMemcpyAsync(&flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   PW_HIP(hipStreamSynchronize(c->stream));
-  if (flag) return fail(PW_ERR_NONFINITE, std::string(what) + ": non-finite rate (coincident particles?)");
+  if (*static_cast<volatile int*>(c->h_flag)) return fail(PW_ERR_NONFINITE, std::string(what) + ": non-finite rate (coincident particles?)");
   return PW_OK;
 }
 
@@ -645,15 +654,97 @@ int upload_state(pw_ctx* c, const std::vector<Rec64>& h) {
   return PW_OK;
 }
 
-int download_rates(pw_ctx* c, std::vector<Rate64>& h) {
-  h.resize(static_cast<size_t>(c->n));
-  if (!c->built) {
-    std::memset(h.data(), 0, h.size() * sizeof(Rate64));
-    return PW_OK;
+// Copies between caller memory and the pinned staging.  A caller's fresh pages
+// fault on their first write, which bounds one thread at 5 GB/s (8 threads: 17
+// GB/s), so large copies are spread over threads.
+struct Segment {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+
+void copy_range(const std::vector<Segment>& segs, size_t from, size_t to) {
+  size_t at = 0;
+  for (const Segment& s : segs) {
+    const size_t a = std::max(from, at), b = std::min(to, at + s.bytes);
+    if (a < b) std::memcpy(static_cast<char*>(s.dst) + (a - at), static_cast<const char*>(s.src) + (a - at), b - a);
+    at += s.bytes;
   }
-  PW_HIP(hipMemcpyAsync(h.data(), c->rates, h.size() * sizeof(Rate64), hipMemcpyDeviceToHost,
-                        c->stream));
+}
+
+void copy_segments(const std::vector<Segment>& segs) {
+  size_t total = 0;
+  for (const Segment& s : segs) total += s.bytes;
+  constexpr size_t kPerThread = size_t(1) << 20;  // a thread costs about what it copies in 30 us
+  const size_t nt = std::min<size_t>(8, total / kPerThread);
+  if (nt < 2) {
+    copy_range(segs, 0, total);
+    return;
+  }
+  const size_t step = (total / nt + 4095) / 4096 * 4096;
+  std::vector<std::thread> th;
+  size_t done = step;  // this thread takes the first range
+  try {
+    th.reserve(nt);
+    for (; done < total; done += step) th.emplace_back(copy_range, std::cref(segs), done, std::min(total, done + step));
+  } catch (...) {  // no more threads: the rest here
+    copy_range(segs, done, total);
+  }
+  copy_range(segs, 0, std::min(step, total));
+  for (auto& t : th) t.join();
+}
+
+// Pinned staging for up to `count` particles (6 doubles each, 256 MB at most:
+// longer transfers go in pieces).  The stream is idle when it returns, so the
+// staging is free.
+int ensure_stage(pw_ctx* c, int64_t count) {
+  constexpr int64_t kMaxParticles = (int64_t(256) << 20) / 48;
+  const int64_t want = std::min(count, kMaxParticles);
   PW_HIP(hipStreamSynchronize(c->stream));
+  if (static_cast<size_t>(want) <= c->stage_particles) return PW_OK;
+  (void)hipHostFree(c->h_stage);
+  c->h_stage = nullptr;
+  c->stage_particles = 0;
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), 48 * static_cast<size_t>(want), hipHostMallocCoherent) !=
+      hipSuccess) {
+    (void)hipGetLastError();
+    c->h_stage = nullptr;
+    return fail(PW_ERR_NOMEM, "pinned staging");
+  }
+  c->stage_particles = static_cast<size_t>(want);
+  return PW_OK;
+}
+
+// positions and strengths (or, rates, velocities and vorticity rates) of
+// particles [first, first + count) into a and b (either may be null)
+int read_particles(pw_ctx* c, bool rates, int64_t first, int64_t count, double* a, double* b) {
+  if (count <= 0) return PW_OK;
+  PW_TRY(ensure_stage(c, count));
+  for (int64_t p = 0; p < count; p += static_cast<int64_t>(c->stage_particles)) {
+    const int64_t m = std::min<int64_t>(count - p, static_cast<int64_t>(c->stage_particles));
+    if (rates) PW_HIP(pw::launch_pack_rates(c->rates, first + p, m, c->h_stage, c->stream));
+    else PW_HIP(pw::launch_pack_state(c->y, first + p, m, c->h_stage, false, c->stream));
+    PW_HIP(hipStreamSynchronize(c->stream));
+    const size_t bytes = 24 * static_cast<size_t>(m);
+    std::vector<Segment> segs;
+    if (a) segs.push_back({a + 3 * p, c->h_stage, bytes});
+    if (b) segs.push_back({b + 3 * p, c->h_stage + 3 * m, bytes});
+    copy_segments(segs);
+  }
+  return PW_OK;
+}
+
+// positions and strengths of particles [first, first + count) from x and a
+int write_particles(pw_ctx* c, int64_t first, int64_t count, const double* x, const double* a) {
+  if (count <= 0) return PW_OK;
+  PW_TRY(ensure_stage(c, count));
+  for (int64_t p = 0; p < count; p += static_cast<int64_t>(c->stage_particles)) {
+    const int64_t m = std::min<int64_t>(count - p, static_cast<int64_t>(c->stage_particles));
+    if (p > 0) PW_HIP(hipStreamSynchronize(c->stream));  // the previous piece has been read
+    const size_t bytes = 24 * static_cast<size_t>(m);
+    copy_segments({{c->h_stage, x + 3 * p, bytes}, {c->h_stage + 3 * m, a + 3 * p, bytes}});
+    PW_HIP(pw::launch_pack_state(c->y, first + p, m, c->h_stage, true, c->stream));
+  }
   return PW_OK;
 }
 
@@ -828,14 +919,13 @@ int pw_set_wake_state(pw_ctx* c, int w, const double* pos, const double* alpha) 
   PW_CTX(c);
   if (w < 0 || w >= static_cast<int>(c->wn.size())) return fail(PW_ERR_ARG, "wake index out of range");
   if (c->wn[w] > 0 && (!pos || !alpha)) return fail(PW_ERR_ARG, "null array");
-  std::vector<Rec64> h;
-  PW_TRY(download_state(c, h));
+  if (c->built) return write_particles(c, c->woff[w], c->wn[w], pos, alpha);
   for (int64_t i = 0; i < c->wn[w]; ++i) {
-    Rec64& r = h[c->woff[w] + i];
+    Rec64& r = c->pending[c->woff[w] + i];
     r.x = pos[3 * i]; r.y = pos[3 * i + 1]; r.z = pos[3 * i + 2];
     r.ax = alpha[3 * i]; r.ay = alpha[3 * i + 1]; r.az = alpha[3 * i + 2];
   }
-  return upload_state(c, h);
+  return PW_OK;
 }
 
 int pw_set_wake_volume(pw_ctx* c, int w, const double* volume) {
@@ -854,10 +944,9 @@ int pw_set_wake_volume(pw_ctx* c, int w, const double* volume) {
 int pw_get_wake_state(pw_ctx* c, int w, double* pos, double* alpha) {
   PW_CTX(c);
   if (w < 0 || w >= static_cast<int>(c->wn.size())) return fail(PW_ERR_ARG, "wake index out of range");
-  std::vector<Rec64> h;
-  PW_TRY(download_state(c, h));
+  if (c->built) return read_particles(c, false, c->woff[w], c->wn[w], pos, alpha);
   for (int64_t i = 0; i < c->wn[w]; ++i) {
-    const Rec64& r = h[c->woff[w] + i];
+    const Rec64& r = c->pending[c->woff[w] + i];
     if (pos) { pos[3 * i] = r.x; pos[3 * i + 1] = r.y; pos[3 * i + 2] = r.z; }
     if (alpha) { alpha[3 * i] = r.ax; alpha[3 * i + 1] = r.ay; alpha[3 * i + 2] = r.az; }
   }
@@ -867,13 +956,10 @@ int pw_get_wake_state(pw_ctx* c, int w, double* pos, double* alpha) {
 int pw_get_wake_rates(pw_ctx* c, int w, double* vel, double* retvor) {
   PW_CTX(c);
   if (w < 0 || w >= static_cast<int>(c->wn.size())) return fail(PW_ERR_ARG, "wake index out of range");
-  std::vector<Rate64> h;
-  PW_TRY(download_rates(c, h));
-  for (int64_t i = 0; i < c->wn[w]; ++i) {
-    const Rate64& r = h[c->woff[w] + i];
-    if (vel) { vel[3 * i] = r.ux; vel[3 * i + 1] = r.uy; vel[3 * i + 2] = r.uz; }
-    if (retvor) { retvor[3 * i] = r.wx; retvor[3 * i + 1] = r.wy; retvor[3 * i + 2] = r.wz; }
-  }
+  if (c->built) return read_particles(c, true, c->woff[w], c->wn[w], vel, retvor);
+  const size_t bytes = 24 * static_cast<size_t>(c->wn[w]);
+  if (vel) std::memset(vel, 0, bytes);
+  if (retvor) std::memset(retvor, 0, bytes);
   return PW_OK;
 }
 
@@ -881,39 +967,25 @@ int pw_set_states(pw_ctx* c, const double* state, int64_t len) {
   PW_CTX(c);
   if (!state) return fail(PW_ERR_ARG, "null state");
   if (len != total_maxsize(c)) return fail(PW_ERR_ARG, "state length != sum of 6*maxn");
-  std::vector<Rec64> h;
-  PW_TRY(download_state(c, h));
-  int64_t base = 0;
+  // per wake the pos block, maxn x 3, then the alpha block (wake.cpp:860-866)
   for (size_t w = 0; w < c->wn.size(); ++w) {
-    const double* p = state + base;                 // pos block, maxn x 3
-    const double* a = state + base + 3 * c->wmax[w];  // alpha block (wake.cpp:860-866)
-    for (int64_t i = 0; i < c->wn[w]; ++i) {
-      Rec64& r = h[c->woff[w] + i];
-      r.x = p[3 * i]; r.y = p[3 * i + 1]; r.z = p[3 * i + 2];
-      r.ax = a[3 * i]; r.ay = a[3 * i + 1]; r.az = a[3 * i + 2];
-    }
-    base += 6 * c->wmax[w];
+    PW_TRY(pw_set_wake_state(c, static_cast<int>(w), state, state + 3 * c->wmax[w]));
+    state += 6 * c->wmax[w];
   }
-  return upload_state(c, h);
+  return PW_OK;
 }
 
 int pw_get_states(pw_ctx* c, double* state, int64_t len) {
   PW_CTX(c);
   if (!state) return fail(PW_ERR_ARG, "null state");
   if (len != total_maxsize(c)) return fail(PW_ERR_ARG, "state length != sum of 6*maxn");
-  std::vector<Rec64> h;
-  PW_TRY(download_state(c, h));
-  std::memset(state, 0, sizeof(double) * static_cast<size_t>(len));
-  int64_t base = 0;
   for (size_t w = 0; w < c->wn.size(); ++w) {
-    double* p = state + base;
-    double* a = state + base + 3 * c->wmax[w];
-    for (int64_t i = 0; i < c->wn[w]; ++i) {
-      const Rec64& r = h[c->woff[w] + i];
-      p[3 * i] = r.x; p[3 * i + 1] = r.y; p[3 * i + 2] = r.z;
-      a[3 * i] = r.ax; a[3 * i + 1] = r.ay; a[3 * i + 2] = r.az;
-    }
-    base += 6 * c->wmax[w];
+    double *p = state, *a = state + 3 * c->wmax[w];
+    PW_TRY(pw_get_wake_state(c, static_cast<int>(w), p, a));
+    const size_t pad = 24 * static_cast<size_t>(c->wmax[w] - c->wn[w]);
+    std::memset(p + 3 * c->wn[w], 0, pad);
+    std::memset(a + 3 * c->wn[w], 0, pad);
+    state += 6 * c->wmax[w];
   }
   return PW_OK;
 }
@@ -922,19 +994,13 @@ int pw_get_rates(pw_ctx* c, double* rate, int64_t len) {
   PW_CTX(c);
   if (!rate) return fail(PW_ERR_ARG, "null rate");
   if (len != total_maxsize(c)) return fail(PW_ERR_ARG, "rate length != sum of 6*maxn");
-  std::vector<Rate64> h;
-  PW_TRY(download_rates(c, h));
-  std::memset(rate, 0, sizeof(double) * static_cast<size_t>(len));
-  int64_t base = 0;
   for (size_t w = 0; w < c->wn.size(); ++w) {
-    double* u = rate + base;
-    double* q = rate + base + 3 * c->wmax[w];  // wake.cpp:876
-    for (int64_t i = 0; i < c->wn[w]; ++i) {
-      const Rate64& r = h[c->woff[w] + i];
-      u[3 * i] = r.ux; u[3 * i + 1] = r.uy; u[3 * i + 2] = r.uz;
-      q[3 * i] = r.wx; q[3 * i + 1] = r.wy; q[3 * i + 2] = r.wz;
-    }
-    base += 6 * c->wmax[w];
+    double *u = rate, *q = rate + 3 * c->wmax[w];  // wake.cpp:876
+    PW_TRY(pw_get_wake_rates(c, static_cast<int>(w), u, q));
+    const size_t pad = 24 * static_cast<size_t>(c->wmax[w] - c->wn[w]);
+    std::memset(u + 3 * c->wn[w], 0, pad);
+    std::memset(q + 3 * c->wn[w], 0, pad);
+    rate += 6 * c->wmax[w];
   }
   return PW_OK;
 }
@@ -1106,7 +1172,7 @@ int pw_solve(pw_ctx* c, int precision) {
   int kind = 0;
   PW_TRY(kind_of(precision, &kind));
   PW_TRY(ensure_built(c));
-  PW_HIP(pw::launch_fill_int(c->d_flag, 1, 0, c->stream));
+  PW_TRY(clear_flag(c));
   PW_TRY(rhs(c, kind, c->y, c->k[0]));
   c->rates = c->k[0];
   return check_flag(c, "pw_solve");
@@ -1215,7 +1281,7 @@ int pw_step(pw_ctx* c, int scheme, double dt, int precision, int64_t nsteps) {
   if (nsteps < 0) return fail(PW_ERR_ARG, "nsteps must be >= 0");
   PW_TRY(ensure_built(c));
   PW_TRY(ensure_kind(c, kind));
-  PW_HIP(pw::launch_fill_int(c->d_flag, 1, 0, c->stream));
+  PW_TRY(clear_flag(c));
   // the tree path re-sorts the particles every stage (host-side sort
   // set-up), so its steps are launched eagerly
   if (c->use_graph && !c->profiling && nsteps > 0 && kind != kKindLearned) {
@@ -1247,7 +1313,7 @@ int pw_interact_wakes(pw_ctx* c, int precision, const int* pairs, int npairs) {
   const int n = static_cast<int>(c->n);
   Rate64* acc = c->k[0];
   Rate64* blk = c->k[1];
-  PW_HIP(pw::launch_fill_int(c->d_flag, 1, 0, c->stream));
+  PW_TRY(clear_flag(c));
   PW_HIP(pw::launch_zero_doubles(reinterpret_cast<double*>(acc), 6 * static_cast<int64_t>(n), c->stream));
   WorkItem* d_items = nullptr;
   if (!items.empty() && dalloc(&d_items, items.size()) != hipSuccess) {
@@ -1270,7 +1336,7 @@ int pw_interact_wakes(pw_ctx* c, int precision, const int* pairs, int npairs) {
     if (e == hipSuccess && a != b)
       e = pw::launch_add_rates(acc, blk, static_cast<int>(c->woff[b]), static_cast<int>(c->woff[b + 1]), c->stream);
   }
-  if (e == hipSuccess) e = pw::launch_check_finite(acc, n, c->d_flag, c->stream);
+  if (e == hipSuccess) e = pw::launch_check_finite(acc, n, c->h_flag, c->stream);
   (void)hipStreamSynchronize(c->stream);  // the items are freed below
   (void)hipFree(d_items);
   if (e != hipSuccess) return fail(PW_ERR_HIP, std::string("pw_interact_wakes: ") + hipGetErrorString(e));

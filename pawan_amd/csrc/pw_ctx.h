@@ -111,7 +111,9 @@ struct pw_ctx {
   int ndiag = 0;
   int* d_diag_first = nullptr;
   double* d_quad = nullptr;
-  int* d_flag = nullptr;
+  int* h_flag = nullptr;        // non-finite rates seen (pinned, written by the kernels)
+  double* h_stage = nullptr;    // pinned staging of state and rate transfers
+  size_t stage_particles = 0;
 
   // per pair-kernel kind: launch configuration and its work items
   struct KindState {

@@ -154,11 +154,18 @@ struct SumForm {
   int ngroups = 0;
 };
 // Sum of the partial rates into `rates` (in order), flag |= any non-finite
-// rate, and the stage arithmetic, in one pass.
+// rate, and the stage arithmetic, in one pass.  flag: a word of pinned host
+// memory.
 hipError_t launch_finish(const SumForm& sum, Rate64* rates, int n, int* flag, const StageOp& op, hipStream_t st);
 // count of non-finite entries of the rates -> *flag (device int)
 hipError_t launch_check_finite(const Rate64* k, int n, int* flag,
                                hipStream_t st);
+
+// particles [first, first + count): positions then strengths (or velocities
+// then vorticity rates) to `host` (6 count doubles of pinned memory), or, with
+// store, positions and strengths from it
+hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* host, bool store, hipStream_t st);
+hipError_t launch_pack_rates(const Rate64* k, int64_t first, int64_t count, double* host, hipStream_t st);
 
 // zero-fill of a small int buffer (a kernel, not hipMemsetAsync, so that
 // the step sequence can be captured into a HIP graph)

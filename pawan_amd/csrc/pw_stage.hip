@@ -93,7 +93,7 @@ __global__ __launch_bounds__(Sum == 2 ? kGroupThreads : kEW) void k_finish(Finis
       k = f.rates[e];
     }
   }
-  if (!isfinite(k)) atomicOr(f.flag, 1);
+  if (!isfinite(k)) *f.flag = 1;  // (host memory: every writer stores the same word)
   stage_component<Op>(f.op, e, k);
 }
 
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kEW) void k_check_finite(
   if (i >= n) return;
   const Rate64 r = k[i];
   const double s = r.ux + r.uy + r.uz + r.wx + r.wy + r.wz;
-  if (!isfinite(s) || !isfinite(r.ux) || !isfinite(r.wx)) atomicOr(flag, 1);
+  if (!isfinite(s) || !isfinite(r.ux) || !isfinite(r.wx)) *flag = 1;
 }
 
 __global__ void k_fill_int(int* __restrict__ p, int n, int value) {
@@ -125,6 +125,27 @@ __global__ __launch_bounds__(kEW) void k_add_rates(Rate64* __restrict__ acc, con
   a.ux += b.ux; a.uy += b.uy; a.uz += b.uz;
   a.wx += b.wx; a.wy += b.wy; a.wz += b.wz;
   acc[i] = a;
+}
+
+// Particles [first, first + count) of the state or the rates to and from the
+// two 3-vectors per particle that callers hold: xyz and alpha (or u and dalpha)
+// of all the particles, one after the other, one thread per double.  The
+// packed side is pinned host memory, read and written by the kernel itself
+// (coalesced 8-byte accesses over the bus), so a transfer is one launch and
+// moves 48 bytes per particle; copying the records both ways and converting
+// them on one host thread took 20 ms of a 1M right-hand side.
+template <bool State, bool Store>
+__global__ __launch_bounds__(kEW) void k_pack(double* __restrict__ dev, int64_t first, int64_t count,
+                                              double* __restrict__ host) {
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * kEW + threadIdx.x;
+  if (e >= 6 * count) return;
+  const int half = e >= 3 * count ? 1 : 0;
+  const int64_t v = e - 3 * count * half;
+  const int64_t i = v / 3;
+  const int c = static_cast<int>(v - 3 * i);
+  double* d = dev + (State ? 8 * (first + i) + 4 * half : 6 * (first + i) + 3 * half) + c;
+  if (Store) *d = host[e];
+  else host[e] = *d;
 }
 
 inline int ew_blocks(int n) { return (n + kEW - 1) / kEW; }
@@ -167,6 +188,22 @@ hipError_t launch_finish(const SumForm& sum, Rate64* rates, int n, int* flag, co
     case kStageEuler: finish_kernel<kStageEuler>(sum, f, st); break;
     default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* host, bool store, hipStream_t st) {
+  if (count <= 0) return hipSuccess;
+  const dim3 g(static_cast<unsigned>((6 * count + kEW - 1) / kEW)), b(kEW);
+  double* d = reinterpret_cast<double*>(y);
+  if (store) hipLaunchKernelGGL((k_pack<true, true>), g, b, 0, st, d, first, count, host);
+  else hipLaunchKernelGGL((k_pack<true, false>), g, b, 0, st, d, first, count, host);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_rates(const Rate64* k, int64_t first, int64_t count, double* host, hipStream_t st) {
+  if (count <= 0) return hipSuccess;
+  hipLaunchKernelGGL((k_pack<false, false>), dim3(static_cast<unsigned>((6 * count + kEW - 1) / kEW)), dim3(kEW), 0, st,
+                     reinterpret_cast<double*>(const_cast<Rate64*>(k)), first, count, host);
   return hipGetLastError();
 }
 
