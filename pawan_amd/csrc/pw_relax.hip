@@ -16,12 +16,14 @@
 //     state.  The first merge of i needs such a neighbour (x_i is unmoved
 //     until then, and strengths only ever drop to zero), so an i with none
 //     does nothing and is left out.
-//  2. One block then visits the flagged i in order and replays the
-//     reference's inner loop: the next j > (last j seen) within the merge
-//     distance of the current x_i, found among the 27 cells around x_i, with
-//     the current strengths.  Later particles have not moved (only the outer
-//     particle of an iteration moves), so the cell list of the original
-//     positions still finds them.
+//  2. The flagged i are visited in order and the reference's inner loop is
+//     replayed: the next j > (last j seen) within the merge distance of the
+//     current x_i, found among the 27 cells around x_i, with the current
+//     strengths.  Later particles have not moved (only the outer particle of
+//     an iteration moves), so the cell list of the original positions still
+//     finds them.  Flagged particles far enough apart cannot touch the same
+//     particles, so they are first gathered into groups (k_group_link) and
+//     every group is replayed by a block of its own.
 // The arithmetic is the reference's (GSL's dnrm2 and ddot, dscal by the
 // reciprocal, no contraction), so the result is bit-for-bit the
 // sequential one.
@@ -33,6 +35,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "pw_ctx.h"
@@ -194,6 +197,29 @@ __device__ __forceinline__ void equal_range(const uint64_t* __restrict__ keys, i
   *hi = c;
 }
 
+// first of the sorted keys not below k (upper: above k)
+__device__ __forceinline__ int bound_of(const uint64_t* __restrict__ keys, int n, uint64_t k, bool upper) {
+  int a = 0, b = n;
+  while (a < b) {
+    const int m = (a + b) >> 1;
+    if (upper ? keys[m] <= k : keys[m] < k) a = m + 1;
+    else b = m;
+  }
+  return a;
+}
+
+// the cells of row r = 0 .. 8 about cell c (y, z offsets r % 3 - 1, r / 3 - 1):
+// x is the lowest part of a key, so its three cells are one range of the
+// sorted keys, from the first not below `first` to the first above `last`;
+// false if the row is outside the grid
+__device__ __forceinline__ bool cell_row(const int64_t* c, int r, uint64_t* first, uint64_t* last) {
+  const int64_t y = c[1] + r % 3 - 1, z = c[2] + r / 3 - 1;
+  if (y < 0 || z < 0 || y > kCellMax || z > kCellMax) return false;
+  *first = cell_key(max(c[0] - 1, int64_t(0)), y, z);
+  *last = cell_key(min(c[0] + 1, kCellMax), y, z);
+  return true;
+}
+
 // can pair (i, j) merge (wake.cpp:129-135), for positions xi, xj and
 // strengths ai, aj with norms mi, mj
 __device__ __forceinline__ bool in_reach(const double* xi, const double* xj, double ri, double rj) {
@@ -223,67 +249,155 @@ __global__ void k_merge_flags(int n, const int* __restrict__ prefix, Grid g, con
   int64_t c[3];
   if (i < *prefix && mi != 0.0 && cell_of(g, xi[0], xi[1], xi[2], c)) {
     const double ri = radius[i];
-    for (int dz = -1; dz <= 1 && !f; ++dz)
-      for (int dy = -1; dy <= 1 && !f; ++dy)
-        for (int dx = -1; dx <= 1 && !f; ++dx) {
-          const int64_t x = c[0] + dx, y = c[1] + dy, z = c[2] + dz;
-          if (x < 0 || y < 0 || z < 0 || x > kCellMax || y > kCellMax || z > kCellMax) continue;
-          int lo, hi;
-          equal_range(keys, n, cell_key(x, y, z), &lo, &hi);
-          for (int e = lo; e < hi && !f; ++e) {
-            const int j = sidx[e];
-            if (j <= i) continue;
-            const double* aj = alpha + 3 * static_cast<int64_t>(j);
-            const double mj = dnrm2_3(aj[0], aj[1], aj[2]);
-            if (mj == 0.0 || !in_reach(xi, pos + 3 * static_cast<int64_t>(j), ri, radius[j])) continue;
-            if (misalignment(ai, aj, mi, mj) >= 0.0001) f = 1;
-          }
-        }
+    for (int r = 0; r < 9 && !f; ++r) {
+      uint64_t first, last;
+      if (!cell_row(c, r, &first, &last)) continue;
+      const int lo = bound_of(keys, n, first, false), hi = bound_of(keys, n, last, true);
+      for (int e = lo; e < hi && !f; ++e) {
+        const int j = sidx[e];
+        if (j <= i) continue;
+        const double* aj = alpha + 3 * static_cast<int64_t>(j);
+        const double mj = dnrm2_3(aj[0], aj[1], aj[2]);
+        if (mj == 0.0 || !in_reach(xi, pos + 3 * static_cast<int64_t>(j), ri, radius[j])) continue;
+        if (misalignment(ai, aj, mi, mj) >= 0.0001) f = 1;
+      }
+    }
   }
   flag[i] = f;
 }
 
-constexpr int kRT = 256;    // threads of the replaying block
-constexpr int kCap = 1024;  // later neighbours of one outer particle kept in LDS
+// ---- groups of flagged particles ------------------------------------------
+// While x_i stays within kTravel cells' width h of where it started, iteration
+// i touches (merges, or tests as in reach) only particles within (kTravel + 1)
+// h of that point: a merge distance is at most h.  Another group's flagged
+// particle p stays as near to its own start, so at any time (its coordinates
+// read one by one, each old or new: at most sqrt(3) kTravel h from the start)
+// it is out of reach of x_i if the starts are more than
+//   (1 + kTravel + sqrt(3) kTravel) h = 5.1 h
+// apart, and so are the particles it absorbs ((2 kTravel + 2) h = 5 h).
+// Particles within kLink h are put into one group; an x_i that leaves its range
+// stops the replay, which then starts over with everything in one group.
+constexpr double kTravel = 1.5, kLink = 6.25;
+constexpr int kExactLinks = 32;  // cells with more flagged particles are linked whole
 
-// the smallest of the block's values (all threads call it)
-__device__ __forceinline__ int block_min_int(int v, int* red) {
-  for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  int m = red[0];
-  for (int w = 1; w < kRT / 64; ++w) m = min(m, red[w]);
-  __syncthreads();
-  return m;
+__device__ __forceinline__ int group_root(int* parent, int x) {
+  for (;;) {
+    const int p = __hip_atomic_load(parent + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (p == x) return x;
+    x = p;  // parents only decrease: the walk ends
+  }
 }
 
-// step 2: one block replays the reference's loops over the flagged
-// particles.  For the current outer particle the later particles of the 27
-// cells around it (index, position, radius, |a| at that time) are gathered
+__device__ __forceinline__ void group_unite(int* parent, int a, int b) {
+  for (;;) {
+    a = group_root(parent, a);
+    b = group_root(parent, b);
+    if (a == b) return;
+    if (a < b) {
+      const int t = a;
+      a = b;
+      b = t;
+    }
+    // the larger root under the smaller; if a got a parent meanwhile, again
+    // from there (a strictly smaller index)
+    const int old = atomicCAS(parent + a, a, b);
+    if (old == a) return;
+    a = old;
+  }
+}
+
+// coarse cells (width kLink h) of the flagged particles
+__global__ void k_group_keys(const double* __restrict__ pos, const int* __restrict__ list, int count, Grid g,
+                             uint64_t* __restrict__ key, int* __restrict__ idx, int* __restrict__ parent) {
+  const int k = blockIdx.x * kB + static_cast<int>(threadIdx.x);
+  if (k >= count) return;
+  int64_t c[3];
+  const double* x = pos + 3 * static_cast<int64_t>(list[k]);
+  g.h *= kLink;
+  key[k] = cell_of(g, x[0], x[1], x[2], c) ? cell_key(c[0], c[1], c[2]) : kNoCell;
+  idx[k] = k;
+  parent[k] = k;
+}
+
+// flagged particle e (in the order of the coarse cells) with those within
+// kLink h in its own cell and in the 13 neighbour cells after it
+__global__ void k_group_link(const double* __restrict__ pos, const int* __restrict__ list,
+                             const uint64_t* __restrict__ keys, const int* __restrict__ sidx, int count, Grid g,
+                             int* parent) {
+  const int e = blockIdx.x * kB + static_cast<int>(threadIdx.x);
+  if (e >= count || keys[e] == kNoCell) return;
+  const double* x = pos + 3 * static_cast<int64_t>(list[sidx[e]]);
+  const double reach = kLink * g.h;
+  const uint64_t key = keys[e], mask = static_cast<uint64_t>(kCellMax);
+  const int64_t c[3] = {static_cast<int64_t>(key & mask), static_cast<int64_t>((key >> kCellBits) & mask),
+                        static_cast<int64_t>(key >> (2 * kCellBits))};
+  for (int q = 13; q < 27; ++q) {  // the cell itself, then the 13 after it in z, y, x order
+    const int64_t nx = c[0] + q % 3 - 1, ny = c[1] + (q / 3) % 3 - 1, nz = c[2] + q / 9 - 1;
+    if (nx < 0 || ny < 0 || nz < 0 || nx > kCellMax || ny > kCellMax || nz > kCellMax) continue;
+    int lo, hi;
+    equal_range(keys, count, cell_key(nx, ny, nz), &lo, &hi);
+    if (lo == hi) continue;
+    if (hi - lo > kExactLinks) {
+      // a crowded cell is one group: each of its particles joins the first
+      group_unite(parent, sidx[e], sidx[lo]);
+      continue;
+    }
+    for (int f = lo; f < hi; ++f) {
+      if (q == 13 && f >= e) break;
+      const double* y = pos + 3 * static_cast<int64_t>(list[sidx[f]]);
+      const double dx = x[0] - y[0], dy = x[1] - y[1], dz = x[2] - y[2];
+      if (dx * dx + dy * dy + dz * dz <= reach * reach) group_unite(parent, sidx[e], sidx[f]);
+    }
+  }
+}
+
+__global__ void k_group_roots(int count, int* parent, int* __restrict__ root) {
+  const int k = blockIdx.x * kB + static_cast<int>(threadIdx.x);
+  if (k < count) root[k] = group_root(parent, k);
+}
+
+// ---- replay ----------------------------------------------------------------
+constexpr int kRT = 64;     // threads of a replaying block: one wave, no other to wait for
+constexpr int kCap = 1024;  // later neighbours of one outer particle kept in LDS
+
+__device__ __forceinline__ int wave_min_int(int v) {
+  for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
+  return v;
+}
+
+// step 2: a block replays the reference's loops over one group: the particles
+// list[k] of one root (consecutive, ascending particles), the block of the
+// first of them doing the work.  For the current outer particle the later
+// particles of the 27 cells around it (index, position, radius) are gathered
 // into LDS, again when x_i moves to another cell; each step then takes the
 // smallest j past the last one seen that is within reach of the current x_i.
 // More than kCap of them: the step scans the cells in memory instead.
+//
+// A replay is a chain of dependent memory reads, so it is bound by latency:
+// one block over all flagged particles took 9.2 ms for a 98,304-particle wake
+// with one particle in 200 turned; by groups the same replay takes 0.09 ms,
+// the linking 0.06.
 __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restrict__ list,
-                                                       const int* __restrict__ count, Grid g,
+                                                       const int* __restrict__ root, int count, Grid g,
                                                        const uint64_t* __restrict__ keys,
                                                        const int* __restrict__ sidx, double* pos, double* alpha,
                                                        const double* __restrict__ radius, double* volume,
-                                                       int64_t* __restrict__ merges) {
-  __shared__ int s_lo[27], s_hi[27];
+                                                       unsigned long long* merges, int* left) {
+  const int k0 = static_cast<int>(blockIdx.x);
+  if (k0 > 0 && (!root || root[k0] == root[k0 - 1])) return;
+  const int group = root ? root[k0] : 0;
+  __shared__ int s_lo[9], s_hi[9];
   __shared__ int s_cnt;
   __shared__ int s_j[kCap];
   __shared__ double s_x[3 * kCap];
   __shared__ double s_r[kCap];
-  __shared__ int s_red[kRT / 64];
   const int tid = static_cast<int>(threadIdx.x);
-  const int K = *count;
-  int64_t done = 0;
-  for (int k = 0; k < K; ++k) {
+  unsigned long long done = 0;
+  for (int k = k0; k < count && (!root || root[k] == group); ++k) {
     const int i = list[k];
-    double xi[3], ai[3];
+    double xi[3], x0[3], ai[3];
     for (int c = 0; c < 3; ++c) {
-      xi[c] = pos[3 * static_cast<int64_t>(i) + c];
+      xi[c] = x0[c] = pos[3 * static_cast<int64_t>(i) + c];
       ai[c] = alpha[3 * static_cast<int64_t>(i) + c];
     }
     const double mi = dnrm2_3(ai[0], ai[1], ai[2]);  // once per i, as the reference takes it
@@ -297,28 +411,34 @@ __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restr
       const bool in_grid = cell_of(g, xi[0], xi[1], xi[2], c);
       if (!in_grid) break;  // a non-finite position reaches nothing
       if (!have || c[0] != cur[0] || c[1] != cur[1] || c[2] != cur[2]) {
-        // the cell ranges, then the later particles of those cells
-        if (tid < 27) {
-          const int64_t x = c[0] + tid % 3 - 1, y = c[1] + (tid / 3) % 3 - 1, z = c[2] + tid / 9 - 1;
-          if (x < 0 || y < 0 || z < 0 || x > kCellMax || y > kCellMax || z > kCellMax) {
-            s_lo[tid] = s_hi[tid] = 0;
-          } else {
-            equal_range(keys, n, cell_key(x, y, z), &s_lo[tid], &s_hi[tid]);
-          }
+        // the ranges of the 27 cells, then the later particles in them
+        __syncthreads();
+        int edge = 0;  // lanes 0-8: first entries of the nine rows, 9-17: their ends
+        if (tid < 18) {
+          uint64_t first, last;
+          if (cell_row(c, tid % 9, &first, &last)) edge = bound_of(keys, n, tid < 9 ? first : last, tid >= 9);
+        }
+        const int end = __shfl(edge, tid + 9, 64);
+        if (tid < 9) {
+          s_lo[tid] = edge;
+          s_hi[tid] = end;
         }
         if (tid == 0) s_cnt = 0;
         __syncthreads();
-        for (int q = 0; q < 27; ++q)
-          for (int e = s_lo[q] + tid; e < s_hi[q]; e += kRT) {
-            const int j = sidx[e];
-            if (j <= jlast) continue;
-            const int slot = atomicAdd(&s_cnt, 1);
-            if (slot < kCap) {
-              s_j[slot] = j;
-              for (int c2 = 0; c2 < 3; ++c2) s_x[3 * slot + c2] = pos[3 * static_cast<int64_t>(j) + c2];
-              s_r[slot] = radius[j];
-            }
+        int total = 0;
+        for (int q = 0; q < 9; ++q) total += s_hi[q] - s_lo[q];
+        for (int f = tid; f < total; f += kRT) {
+          int e = f, q = 0;  // entry f of the nine rows together
+          while (e >= s_hi[q] - s_lo[q]) e -= s_hi[q] - s_lo[q], ++q;
+          const int j = sidx[s_lo[q] + e];
+          if (j <= jlast) continue;
+          const int slot = atomicAdd(&s_cnt, 1);
+          if (slot < kCap) {
+            s_j[slot] = j;
+            for (int c2 = 0; c2 < 3; ++c2) s_x[3 * slot + c2] = pos[3 * static_cast<int64_t>(j) + c2];
+            s_r[slot] = radius[j];
           }
+        }
         __syncthreads();
         for (int c2 = 0; c2 < 3; ++c2) cur[c2] = c[c2];
         have = true;
@@ -336,7 +456,7 @@ __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restr
           if (dnrm2_3(aj[0], aj[1], aj[2]) != 0.0) best = j;
         }
       } else {
-        for (int q = 0; q < 27; ++q)
+        for (int q = 0; q < 9; ++q)
           for (int e = s_lo[q] + tid; e < s_hi[q]; e += kRT) {
             const int j = sidx[e];
             if (j <= jlast || j >= best) continue;
@@ -345,7 +465,7 @@ __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restr
             if (dnrm2_3(aj[0], aj[1], aj[2]) != 0.0) best = j;
           }
       }
-      const int j = block_min_int(best, s_red);
+      const int j = wave_min_int(best);
       if (j == INT_MAX) break;
       double xj[3], aj[3];
       for (int c2 = 0; c2 < 3; ++c2) {
@@ -367,6 +487,16 @@ __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restr
         __threadfence_block();
         __syncthreads();
         ++done;
+        if (root) {
+          // out of the range that keeps the groups apart (or not a number):
+          // the caller starts over with one group
+          const double dx = xi[0] - x0[0], dy = xi[1] - x0[1], dz = xi[2] - x0[2];
+          const double t = kTravel * g.h;
+          if (!(dx * dx + dy * dy + dz * dz <= t * t)) {
+            if (tid == 0) *left = 1;
+            return;  // the same for every thread
+          }
+        }
       }
       jlast = j;
     }
@@ -379,20 +509,36 @@ __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restr
     __threadfence_block();
     __syncthreads();
   }
-  if (tid == 0) *merges = done;
+  if (tid == 0 && done) atomicAdd(merges, done);
 }
 
 #pragma clang fp contract(on)
 
-// device buffers of one call, freed on every path
+// device buffers of one call, parts of one allocation, freed on every path
 struct Buffers {
   std::vector<void*> p;
   hipStream_t st = nullptr;
+  std::vector<std::pair<void**, size_t>> parts;
+  // `count` elements at *out once allocate() has run
   template <typename T>
-  bool get(T** out, size_t count) {
+  void add(T** out, size_t count) {
     *out = nullptr;
-    if (pwi::dalloc(out, count) != hipSuccess) return false;
-    p.push_back(*out);
+    parts.emplace_back(reinterpret_cast<void**>(out), std::max<size_t>(count, 1) * sizeof(T));
+  }
+  bool allocate() {
+    size_t total = 0;
+    for (const auto& q : parts) total += (q.second + 255) / 256 * 256;
+    char* base = nullptr;
+    if (pwi::dalloc(&base, total) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    p.push_back(base);
+    for (const auto& q : parts) {
+      *q.first = base;
+      base += (q.second + 255) / 256 * 256;
+    }
+    parts.clear();
     return true;
   }
   ~Buffers() {
@@ -447,11 +593,21 @@ int pw_wake_split(int device, double stepnum, int64_t maxn, int64_t* num_particl
   const size_t m = static_cast<size_t>(maxn);
   double *d_pos, *d_alpha, *d_rad, *d_vol, *d_birth, *d_act;
   int *d_prefix, *d_flag, *d_off;
-  if (!b.get(&d_pos, 3 * m) || !b.get(&d_alpha, 3 * m) || !b.get(&d_rad, m) || !b.get(&d_vol, m) ||
-      !b.get(&d_birth, m) || !b.get(&d_act, m) || !b.get(&d_prefix, 1) || !b.get(&d_flag, n) || !b.get(&d_off, n)) {
-    (void)hipGetLastError();
-    return fail(PW_ERR_NOMEM, "device buffers");
-  }
+  const int ni = static_cast<int>(n);
+  size_t tb = 0;
+  RX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, static_cast<int*>(nullptr), static_cast<int*>(nullptr), ni, b.st));
+  char* d_temp;
+  b.add(&d_pos, 3 * m);
+  b.add(&d_alpha, 3 * m);
+  b.add(&d_rad, m);
+  b.add(&d_vol, m);
+  b.add(&d_birth, m);
+  b.add(&d_act, m);
+  b.add(&d_prefix, 1);
+  b.add(&d_flag, n);
+  b.add(&d_off, n);
+  b.add(&d_temp, tb);
+  if (!b.allocate()) return fail(PW_ERR_NOMEM, "device buffers");
   const size_t nn = static_cast<size_t>(n);
   RX_HIP(up(d_pos, pos, 3 * nn, b.st));
   RX_HIP(up(d_alpha, alpha, 3 * nn, b.st));
@@ -459,17 +615,12 @@ int pw_wake_split(int device, double stepnum, int64_t maxn, int64_t* num_particl
   RX_HIP(up(d_vol, volume, nn, b.st));
   RX_HIP(up(d_birth, birthstrength, nn, b.st));
   RX_HIP(up(d_act, active, nn, b.st));
-  const int ni = static_cast<int>(n);
   const dim3 grid((ni + kB - 1) / kB);
   RX_HIP(pw::launch_fill_int(d_prefix, 1, ni, b.st));
   hipLaunchKernelGGL(k_age_prefix, grid, dim3(kB), 0, b.st, d_act, ni, stepnum, d_prefix);
   RX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_split_flags, grid, dim3(kB), 0, b.st, ni, d_prefix, d_alpha, d_birth, d_flag);
   RX_HIP(hipGetLastError());
-  size_t tb = 0;
-  RX_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, d_flag, d_off, ni, b.st));
-  void* d_temp = nullptr;
-  if (!b.get(reinterpret_cast<char**>(&d_temp), tb)) return fail(PW_ERR_NOMEM, "scan buffer");
   RX_HIP(hipcub::DeviceScan::ExclusiveSum(d_temp, tb, d_flag, d_off, ni, b.st));
   int last_off = 0, last_flag = 0;
   RX_HIP(down(&last_off, d_off + (ni - 1), 1, b.st));
@@ -511,15 +662,35 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   const int ni = static_cast<int>(n);
   double *d_pos, *d_alpha, *d_rad, *d_vol, *d_act, *d_ext;
   int *d_prefix, *d_flag, *d_idx, *d_sidx, *d_list, *d_count;
-  uint64_t *d_key, *d_skey;
-  int64_t* d_merges;
-  if (!b.get(&d_pos, 3 * nn) || !b.get(&d_alpha, 3 * nn) || !b.get(&d_rad, nn) || !b.get(&d_vol, nn) ||
-      !b.get(&d_act, nn) || !b.get(&d_ext, 7) || !b.get(&d_prefix, 1) || !b.get(&d_flag, nn) ||
-      !b.get(&d_idx, nn) || !b.get(&d_sidx, nn) || !b.get(&d_list, nn) || !b.get(&d_count, 1) ||
-      !b.get(&d_key, nn) || !b.get(&d_skey, nn) || !b.get(&d_merges, 1)) {
-    (void)hipGetLastError();
-    return fail(PW_ERR_NOMEM, "device buffers");
+  int *d_parent, *d_root, *d_sroot, *d_slist, *d_left;
+  uint64_t *d_key, *d_skey, *d_gkey, *d_sgkey;
+  unsigned long long* d_merges;
+  char* d_temp;
+  size_t t1 = 0, t2 = 0;
+  {
+    uint64_t* k0 = nullptr;
+    int* i0 = nullptr;
+    RX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t1, k0, k0, i0, i0, ni, 0, 64, b.st));
+    RX_HIP(hipcub::DeviceSelect::Flagged(nullptr, t2, i0, i0, i0, i0, ni, b.st));
   }
+  b.add(&d_pos, 3 * nn);
+  b.add(&d_alpha, 3 * nn);
+  b.add(&d_rad, nn);
+  b.add(&d_vol, nn);
+  b.add(&d_act, nn);
+  b.add(&d_ext, 7);
+  b.add(&d_prefix, 1);
+  b.add(&d_flag, nn);
+  b.add(&d_idx, nn);
+  b.add(&d_sidx, nn);
+  b.add(&d_list, nn);
+  b.add(&d_count, 1);
+  b.add(&d_key, nn);
+  b.add(&d_skey, nn);
+  b.add(&d_merges, 1);
+  b.add(&d_left, 1);
+  b.add(&d_temp, std::max(t1, t2));
+  if (!b.allocate()) return fail(PW_ERR_NOMEM, "device buffers");
   RX_HIP(up(d_pos, pos, 3 * nn, b.st));
   RX_HIP(up(d_alpha, alpha, 3 * nn, b.st));
   RX_HIP(up(d_rad, radius, nn, b.st));
@@ -546,30 +717,71 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   RX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_cell_keys, grid, dim3(kB), 0, b.st, d_pos, ni, g, d_key, d_idx);
   RX_HIP(hipGetLastError());
-  size_t t1 = 0, t2 = 0;
-  RX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t1, d_key, d_skey, d_idx, d_sidx, ni, 0, 64, b.st));
-  RX_HIP(hipcub::DeviceSelect::Flagged(nullptr, t2, d_idx, d_flag, d_list, d_count, ni, b.st));
-  char* d_temp = nullptr;
-  if (!b.get(&d_temp, std::max(t1, t2))) return fail(PW_ERR_NOMEM, "sort buffer");
   RX_HIP(hipcub::DeviceRadixSort::SortPairs(d_temp, t1, d_key, d_skey, d_idx, d_sidx, ni, 0, 64, b.st));
   hipLaunchKernelGGL(k_merge_flags, grid, dim3(kB), 0, b.st, ni, d_prefix, g, d_skey, d_sidx, d_pos, d_alpha, d_rad,
                      d_flag);
   RX_HIP(hipGetLastError());
   // the flagged particles in ascending order (the sort left d_idx = 0..n-1)
   RX_HIP(hipcub::DeviceSelect::Flagged(d_temp, t2, d_idx, d_flag, d_list, d_count, ni, b.st));
-  hipLaunchKernelGGL(k_merge_resolve, dim3(1), dim3(kRT), 0, b.st, ni, d_list, d_count, g, d_skey, d_sidx, d_pos,
-                     d_alpha, d_rad, d_vol, d_merges);
-  RX_HIP(hipGetLastError());
-  int64_t merges = 0;
-  RX_HIP(down(&merges, d_merges, 1, b.st));
+  int count = 0;
+  RX_HIP(down(&count, d_count, 1, b.st));
   RX_HIP(hipStreamSynchronize(b.st));
+  if (count == 0) return PW_OK;
+  // groups of flagged particles that cannot reach each other's, each
+  // replayed by a block of its own
+  b.add(&d_parent, count);
+  b.add(&d_root, count);
+  b.add(&d_sroot, count);
+  b.add(&d_slist, count);
+  b.add(&d_gkey, count);
+  b.add(&d_sgkey, count);
+  char* d_temp2;
+  size_t t4 = 0, t5 = 0;
+  RX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t4, d_key, d_skey, d_flag, d_sidx, count, 0, 64, b.st));
+  RX_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, t5, d_flag, d_sidx, d_flag, d_sidx, count, 0, 32, b.st));
+  b.add(&d_temp2, std::max(t4, t5));
+  if (!b.allocate()) return fail(PW_ERR_NOMEM, "merge groups");
+  const dim3 lgrid((count + kB - 1) / kB);
+  RX_HIP(pw::launch_fill_int(reinterpret_cast<int*>(d_merges), 2, 0, b.st));
+  RX_HIP(pw::launch_fill_int(d_left, 1, 0, b.st));
+  hipLaunchKernelGGL(k_group_keys, lgrid, dim3(kB), 0, b.st, d_pos, d_list, count, g, d_gkey, d_flag, d_parent);
+  RX_HIP(hipGetLastError());
+  // (d_flag and d_slist are free: indices before and after the sort)
+  RX_HIP(hipcub::DeviceRadixSort::SortPairs(d_temp2, t4, d_gkey, d_sgkey, d_flag, d_slist, count, 0, 64, b.st));
+  hipLaunchKernelGGL(k_group_link, lgrid, dim3(kB), 0, b.st, d_pos, d_list, d_sgkey, d_slist, count, g, d_parent);
+  RX_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_group_roots, lgrid, dim3(kB), 0, b.st, count, d_parent, d_root);
+  RX_HIP(hipGetLastError());
+  // a stable sort: ascending particles within a group
+  RX_HIP(hipcub::DeviceRadixSort::SortPairs(d_temp2, t5, d_root, d_sroot, d_list, d_slist, count, 0, 32, b.st));
+  hipLaunchKernelGGL(k_merge_resolve, dim3(count), dim3(kRT), 0, b.st, ni, d_slist, d_sroot, count, g, d_skey, d_sidx,
+                     d_pos, d_alpha, d_rad, d_vol, d_merges, d_left);
+  RX_HIP(hipGetLastError());
+  unsigned long long merges = 0;
+  int left = 0;
+  RX_HIP(down(&merges, d_merges, 1, b.st));
+  RX_HIP(down(&left, d_left, 1, b.st));
+  RX_HIP(hipStreamSynchronize(b.st));
+  if (left) {
+    // a particle travelled further than the groups are apart: from the start,
+    // one block over all of them
+    RX_HIP(up(d_pos, pos, 3 * nn, b.st));
+    RX_HIP(up(d_alpha, alpha, 3 * nn, b.st));
+    RX_HIP(up(d_vol, volume, nn, b.st));
+    RX_HIP(pw::launch_fill_int(reinterpret_cast<int*>(d_merges), 2, 0, b.st));
+    hipLaunchKernelGGL(k_merge_resolve, dim3(1), dim3(kRT), 0, b.st, ni, d_list, static_cast<const int*>(nullptr), count,
+                       g, d_skey, d_sidx, d_pos, d_alpha, d_rad, d_vol, d_merges, d_left);
+    RX_HIP(hipGetLastError());
+    RX_HIP(down(&merges, d_merges, 1, b.st));
+    RX_HIP(hipStreamSynchronize(b.st));
+  }
   if (merges > 0) {
     RX_HIP(down(pos, d_pos, 3 * nn, b.st));
     RX_HIP(down(alpha, d_alpha, 3 * nn, b.st));
     RX_HIP(down(volume, d_vol, nn, b.st));
     RX_HIP(hipStreamSynchronize(b.st));
   }
-  if (nmerged) *nmerged = merges;
+  if (nmerged) *nmerged = static_cast<int64_t>(merges);
   return PW_OK;
 }
 
