@@ -761,6 +761,13 @@ namespace pwi {
 
 int ensure_built(pw_ctx* c) { return ::ensure_built(c); }
 
+int staging(pw_ctx* c, size_t bytes, void** out) {
+  PW_TRY(ensure_stage(c, static_cast<int64_t>((bytes + 47) / 48)));
+  if (bytes > 48 * c->stage_particles) return fail(PW_ERR_UNSUPPORTED, "staging beyond 256 MB");
+  *out = c->h_stage;
+  return PW_OK;
+}
+
 int prof_begin(pw_ctx* c, hipEvent_t* e0, hipEvent_t* e1) {
   if (c->ev_free.empty()) {
     PW_HIP(hipEventCreate(e0));

@@ -59,6 +59,9 @@ struct FarField {
   uint16_t* d_frag = nullptr;
   float* d_bias = nullptr;
   int adam_step = 0;
+  // samples, partial gradients and results of pw_ff_mlp_grad, kept between calls
+  float* d_work = nullptr;
+  size_t work_floats = 0;
   // training samples
   float *d_X = nullptr, *d_Y = nullptr;
   double* d_aux = nullptr;
@@ -168,6 +171,9 @@ struct pw_ctx {
 namespace pwi {
 
 int ensure_built(pw_ctx* c);
+// at least `bytes` (256 MB at most) of the context's pinned staging, the stream
+// idle
+int staging(pw_ctx* c, size_t bytes, void** out);
 // event pair for one profiled launch (recycled)
 int prof_begin(pw_ctx* c, hipEvent_t* e0, hipEvent_t* e1);
 // learned far field: one right-hand side, list-overflow check, release

@@ -307,6 +307,7 @@ void ff_release(pw_ctx* c) {
   (void)hipFree(f.d_X);
   (void)hipFree(f.d_Y);
   (void)hipFree(f.d_aux);
+  (void)hipFree(f.d_work);
   const FarField fresh;
   std::vector<float> keep = std::move(f.h_params);
   f = fresh;
@@ -840,30 +841,71 @@ int pw_ff_mlp_grad(pw_ctx* c, const float* X, const float* Y, int64_t n, float* 
   PW_CTX(c);
   if (!X || !Y || !grad || n <= 0 || n > (int64_t(1) << 22)) return fail(PW_ERR_ARG, "bad arrays");
   if (!c->ff.have_weights) return fail(PW_ERR_STATE, "no weights");
-  const int blocks = pw::train_blocks(static_cast<int>(n));
-  float *dX = nullptr, *dY = nullptr, *gp = nullptr, *lp = nullptr, *g = nullptr, *l = nullptr;
-  int* idx = nullptr;
-  std::vector<int> h_idx(static_cast<size_t>(n));
-  std::iota(h_idx.begin(), h_idx.end(), 0);
+  auto& f = c->ff;
+  const size_t m = static_cast<size_t>(n), blocks = static_cast<size_t>(pw::train_blocks(static_cast<int>(n)));
+  // samples | gradient, loss | partial gradients | partial losses, one buffer
+  constexpr size_t kKeep = size_t(64) << 20;  // floats: larger calls get a buffer of their own
+  const size_t in = 28 * m, res = pw::kMlpParams + 4, need = in + res + blocks * pw::kMlpParams + blocks;
+  float* own = nullptr;
+  float* w = f.d_work;
+  if (need > f.work_floats) {
+    PW_HIP(hipStreamSynchronize(c->stream));
+    float* fresh = nullptr;
+    if (dalloc(&fresh, need) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(PW_ERR_NOMEM, "gradient buffers");
+    }
+    w = fresh;
+    if (need <= kKeep) {
+      (void)hipFree(f.d_work);
+      f.d_work = fresh;
+      f.work_floats = need;
+    } else {
+      own = fresh;
+    }
+  }
+  float *dX = w, *dY = w + 16 * m, *g = w + in, *l = g + pw::kMlpParams, *gp = g + res, *lp = gp + blocks * pw::kMlpParams;
+  // the samples and the result pass through pinned memory (copies from and to
+  // pageable memory cost more than the kernels); batches too large for it go
+  // straight
+  void* st = nullptr;
+  const bool pinned = in * sizeof(float) <= (size_t(64) << 20);
+  if (pinned) {
+    const int rc = pwi::staging(c, std::max(in, res) * sizeof(float), &st);
+    if (rc != PW_OK) {
+      (void)hipFree(own);
+      return rc;
+    }
+  }
   hipError_t e = hipSuccess;
-  if (dalloc(&dX, 16 * n) != hipSuccess || dalloc(&dY, 12 * n) != hipSuccess ||
-      dalloc(&gp, static_cast<size_t>(blocks) * pw::kMlpParams) != hipSuccess || dalloc(&lp, blocks) != hipSuccess ||
-      dalloc(&g, pw::kMlpParams) != hipSuccess || dalloc(&l, 1) != hipSuccess || dalloc(&idx, n) != hipSuccess)
-    e = hipErrorOutOfMemory;
-  float lh = 0.0f;
-  if (e == hipSuccess) e = hipMemcpyAsync(dX, X, sizeof(float) * 16 * n, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(dY, Y, sizeof(float) * 12 * n, hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(idx, h_idx.data(), sizeof(int) * n, hipMemcpyHostToDevice, c->stream);
+  if (pinned) {
+    std::memcpy(st, X, sizeof(float) * 16 * m);
+    std::memcpy(static_cast<float*>(st) + 16 * m, Y, sizeof(float) * 12 * m);
+    e = hipMemcpyAsync(dX, st, sizeof(float) * in, hipMemcpyHostToDevice, c->stream);
+  } else {
+    e = hipMemcpyAsync(dX, X, sizeof(float) * 16 * m, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(dY, Y, sizeof(float) * 12 * m, hipMemcpyHostToDevice, c->stream);
+  }
   if (e == hipSuccess)
-    e = pw::launch_mlp_grad(c->ff.d_params, dX, dY, idx, static_cast<int>(n), gp, lp, g, l, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(grad, g, sizeof(float) * pw::kMlpParams, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(&lh, l, sizeof(float), hipMemcpyDeviceToHost, c->stream);
+    e = pw::launch_mlp_grad(f.d_params, dX, dY, nullptr, static_cast<int>(n), gp, lp, g, l, c->stream);
+  float lh = 0.0f;
+  if (pinned) {
+    if (e == hipSuccess) e = hipMemcpyAsync(st, g, sizeof(float) * res, hipMemcpyDeviceToHost, c->stream);
+  } else {
+    if (e == hipSuccess) e = hipMemcpyAsync(grad, g, sizeof(float) * pw::kMlpParams, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(&lh, l, sizeof(float), hipMemcpyDeviceToHost, c->stream);
+  }
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  for (void* p : {static_cast<void*>(dX), static_cast<void*>(dY), static_cast<void*>(gp), static_cast<void*>(lp),
-                  static_cast<void*>(g), static_cast<void*>(l), static_cast<void*>(idx)})
-    (void)hipFree(p);
-  (void)hipGetLastError();
-  if (e != hipSuccess) return fail(PW_ERR_HIP, std::string("mlp grad: ") + hipGetErrorString(e));
+  else (void)hipStreamSynchronize(c->stream);  // nothing queued may still use the buffers
+  (void)hipFree(own);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(PW_ERR_HIP, std::string("mlp grad: ") + hipGetErrorString(e));
+  }
+  if (pinned) {
+    std::memcpy(grad, st, sizeof(float) * pw::kMlpParams);
+    lh = static_cast<float*>(st)[pw::kMlpParams];
+  }
   if (loss) *loss = lh;
   return PW_OK;
 }

@@ -58,11 +58,11 @@ hipError_t launch_ff_samples(const Rec64* sorted, const NodeRec* nodes, const No
 
 // Training (FP32).  One call = loss and gradient of
 //   L = (1/n) sum_s sum_o (f(x_s)_o - y_so)^2
-// over the samples idx[0..n) of (X, Y): per-block partial gradients into
+// over the samples idx[0..n) of (X, Y), the first n if idx is null: per-block partial gradients into
 // gpart (blocks x kMlpParams), per-block loss sums into lpart, then the
 // ordered reduction into grad (and *loss_dev = L).
-constexpr int kTrainRows = 32;  // samples per block
-int train_blocks(int n);
+constexpr int kTrainRows = 16;  // samples per tile
+int train_blocks(int n);        // blocks (partial rows) of a batch of n
 hipError_t launch_mlp_grad(const float* params, const float* X, const float* Y, const int* idx, int n,
                            float* gpart, float* lpart, float* grad, float* loss_dev, hipStream_t st);
 // Adam step on params with the gradient in grad.
