@@ -350,9 +350,12 @@ int64_t split_items(const pw_ctx* c, int split) {
 //   particles.  Its source ranges are the longest of 64, 128 and 256 that
 //   leave kSplitItems items, ten blocks per CU: shorter ones add partial sums
 //   (N = 10,000 FP64: 247 at 64, 238 at 128, 248 at 256, 301 at 1,024), longer
-//   ones leave the chip idle (N = 1,000: 15 at 64, 21 at 128, 96 at 1,024, 347
-//   in one part).  Beyond kSplitItemsMax items (403 MB of partial rates) the
-//   ranges double.
+//   ones leave the chip idle (N = 1,000: 15.7 at 64, 21 at 128, 96 at 1,024,
+//   347 in one part).  Where that is 64 and half of it leaves no more than
+//   kSplitItemsFew items, the chain of a wave is what is left to cut: 32 and
+//   16 (N = 1,000: 14.3 at 32, 17.0 at 16; N = 400: 14.5 at 64, 11.5, 10.0;
+//   N = 2,000: 23.9 at 64, 27.8 at 32).  Beyond kSplitItemsMax items (403 MB
+//   of partial rates) the ranges double.
 // * Beyond, the scalar-fed kernels, whose separated loops are shorter, over 64
 //   source parts and a persistent queue (32 from 196,608 particles: there 32
 //   are 3% faster in FP64 and level in FP32C at half the partial rates).
@@ -365,7 +368,7 @@ int64_t split_items(const pw_ctx* c, int split) {
 // Systems of a batch are far below these sizes: split wins there by the same
 // rule (48 rings of 512-16,384, FP64 4.1 ms against 5.4 over 64 parts).
 constexpr int64_t kSplitUpTo64 = 32768, kSplitUpTo32 = 45056;
-constexpr int64_t kSplitItems = 2560, kSplitItemsMax = 131072;
+constexpr int64_t kSplitItems = 2560, kSplitItemsFew = 640, kSplitItemsMax = 131072;
 
 pw::PairConfig auto_config(const pw_ctx* c, int launch_kind) {
   pw::PairConfig p;
@@ -375,6 +378,7 @@ pw::PairConfig auto_config(const pw_ctx* c, int launch_kind) {
   if (launch_kind == pw::kPairFP64HO || largest <= (f32 ? kSplitUpTo32 : kSplitUpTo64)) {
     p.split = 64;
     while (p.split < 256 && split_items(c, 2 * p.split) >= kSplitItems) p.split *= 2;
+    while (p.split > 16 && p.split <= 64 && split_items(c, p.split / 2) <= kSplitItemsFew) p.split /= 2;
     while (split_items(c, p.split) > kSplitItemsMax && p.split < largest) p.split *= 2;
     return p;
   }

@@ -2053,10 +2053,10 @@ __global__ __launch_bounds__(kTB) void k_pair_fp32c_plain(PairArgs a) { pair_ent
 // For wakes whose targets alone do not fill the chip.  One lane per target
 // against all sources (the LDS-tiled and scalar-fed kernels with one part)
 // leaves 4 blocks for 1,000 particles and runs at the latency of one pair
-// after another.  Here the source range of an item shrinks until about a
-// thousand blocks exist (auto_config in pw_capi.hip), down to 64 sources, 16
+// after another.  Here the source range of an item shrinks until hundreds of
+// blocks exist (auto_config in pw_capi.hip), down to 16 sources, 4
 // per wave.  Measured per right-hand side, one part LDS-tiled against this:
-// ring of 1,000 FP64 347 -> 15 us, two rings of 4,816 1,155 -> 74 us (FP64),
+// ring of 1,000 FP64 347 -> 14 us, two rings of 4,816 1,155 -> 74 us (FP64),
 // 1,017 -> 63 us (high-order), 728 -> 42 us (FP32C); at 24,000 FP64 it runs
 // 481 G pairs/s, bound by its instructions per pair (52 beyond the core, 98 in
 // it), no longer by waves in flight.
