@@ -210,7 +210,7 @@ int ensure_built(pw_ctx* c) {
   build_items(c);
   const size_t n = static_cast<size_t>(c->n);
   if (dalloc(&c->y, n) != hipSuccess || dalloc(&c->ys, n) != hipSuccess ||
-      dalloc(&c->k[0], n) != hipSuccess || dalloc(&c->k[1], n) != hipSuccess ||
+      dalloc(&c->k[0], n) != hipSuccess || dalloc(&c->k[1], std::max<size_t>(n, pw::kPointScratchRows)) != hipSuccess ||
       dalloc(&c->k[2], n) != hipSuccess || dalloc(&c->k[3], n) != hipSuccess ||
       dalloc(&c->d_radius, n) != hipSuccess ||
       dalloc(&c->pair_items, c->h_pair_items.size()) != hipSuccess ||
@@ -753,10 +753,11 @@ int write_particles(pw_ctx* c, int64_t first, int64_t count, const double* x, co
 }
 
 // velocities at m points on the device; the partial sums go to the second
-// rate array, which holds no result between calls
+// rate array, which holds no result between calls (and has room for every
+// split of up to kPointBlocks blocks, however few particles there are)
 hipError_t point_velocity(pw_ctx* c, const double* d_pts, int m, double* d_u) {
   return pw::launch_point_velocity(c->y, static_cast<int>(c->n), d_pts, m, d_u, reinterpret_cast<double*>(c->k[1]),
-                                   6 * static_cast<size_t>(c->n), c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
+                                   6 * std::max(static_cast<size_t>(c->n), pw::kPointScratchRows), c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
 }
 
 }  // namespace

@@ -387,7 +387,10 @@ hipError_t launch_vring_resolve(Rec64* y, int off, int m, int nazi, bool high_or
 
 // velocity at m points (AoS doubles, device) from the n particles of state;
 // scratch: partial sums of split sources (as many splits as it holds, none if
-// null)
+// null; kPointScratchRows 48-byte rows hold every split it would choose for up
+// to 16,384 points)
+constexpr int kPointBlocks = 4096;
+constexpr size_t kPointScratchRows = size_t(32) * (kPointBlocks + 256);
 hipError_t launch_point_velocity(const Rec64* state, int n, const double* pts, int m, double* u, double* scratch,
                                  size_t scratch_doubles, bool high_order, hipStream_t st);
 // near field of the tree path (highorder: the algebraic kernel's pairs)

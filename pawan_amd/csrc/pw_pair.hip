@@ -236,6 +236,15 @@ __device__ __forceinline__ double uniform(double v) {
   return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
 }
 
+// Read-only data of a launch seen through the constant address space: loads
+// at wave-uniform addresses then become scalar loads.
+template <typename T>
+using ConstPtr = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ ConstPtr<T> as_const(const T* p) {
+  return (ConstPtr<T>)(p);
+}
+
 // Separated source ranges of the FP64 kernel.  Positions relative to the
 // block's targets' centre c_T (t' = x_t - c_T, r_s = x_s - c_T, FP64), with
 // m_s = a_s x r_s staged with each source and c_t = t' x a_t per target:
@@ -508,17 +517,22 @@ __device__ __forceinline__ void item_fp64_ho(const PairArgs& pa, const WorkItem&
 // src/interaction/interaction.cpp:453-476): the velocity at m arbitrary
 // points from every particle, with each particle's own radius as sigma,
 // in FP64 with the closed far form beyond 90 sigma^2.  One block per (64
-// points, source range): its four waves hold the same points, one per lane,
-// and take a quarter of every 256-source LDS tile each; their sums are added
-// in wave order and, when the sources are split over several blocks, leave as
-// a 64-row slab that k_point_sum adds in order.  A point that coincides with a
-// particle gets no contribution from it (a_s x d = 0).
+// points, particle range).  The particles sit in the lanes, P per lane in
+// registers, and the points are walked one after another, the same for every
+// lane; a lane's three sums go to LDS, where four lanes per component add the
+// wave's 64 for a batch of four points at a time.  The waves' sums are added
+// in wave order and, when the particles are split over several blocks, leave
+// as a 64-row slab that k_point_sum adds in order.  A point that coincides
+// with a particle gets no contribution from it.
 // HighOrder: the algebraic kernel's q (highorder.h:31-39) instead.
 //
-// Few points against a large wake were the case to fix: with one lane per
-// point against every source, 1,200 points ran on 5 blocks, 105 ms a call
-// against 262,144 particles.  Split (launch_point_velocity), the same runs on
-// 2,052 blocks, 0.75 ms a call with its copies, FP64 issue-bound.
+// Points come in any order (a disk sampled at random), particles along their
+// filaments.  With the points in the lanes, some lane is in the core of most
+// particles, and the wave pays for the core for all of them; 64 consecutive
+// particles are in reach of one point for about 6% of (point, wave) pairs, and
+// a single point still fills the lanes.  1,200 points against 262,144
+// particles: 0.77 ms with the points in the lanes (407 G pairs/s), 0.364 ms so
+// (864 G pairs/s of about 1,150 at the FP64 issue rate), 3 waves per SIMD.
 // ---------------------------------------------------------------------
 struct PointArgs {
   const Rec64* state;
@@ -527,79 +541,140 @@ struct PointArgs {
   int m;
   double* u;        // splits == 1
   double* partial;  // (group, split) slabs of 64 x 3
-  int splits, range;  // source ranges, particles per range
+  int splits, range;  // particle ranges, particles per range
 };
 
-template <bool HighOrder>
-__global__ __launch_bounds__(kTB) void k_point_velocity(PointArgs a) {
-  constexpr int kWaves = kTB / 64;
-  __shared__ Rec64 tile[kTB];
-  __shared__ double red[kWaves - 1][3][64];
-  __shared__ __align__(16) double tab[HighOrder ? 2 : kCore64Pieces * kCore64Row];
-  if (!HighOrder) stage_core64(tab);  // (synchronised with the first tile)
-  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
-  const int g = static_cast<int>(blockIdx.x) / a.splits, part = static_cast<int>(blockIdx.x) % a.splits;
-  const int k = 64 * g + lane;
-  const bool active = k < a.m;
-  const size_t kp = 3 * static_cast<size_t>(active ? k : 64 * g);
-  const double px = a.pts[kp], py = a.pts[kp + 1], pz = a.pts[kp + 2];
-  const int s0 = part * a.range, s1 = min(a.n, s0 + a.range);
-  double u[3] = {0.0, 0.0, 0.0};
-  for (int base = s0; base < s1; base += kTB) {
-    const int cnt = min(kTB, s1 - base);
-    __syncthreads();
-    if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = a.state[base + threadIdx.x];
-    __syncthreads();
-    const int l1 = cnt * (wave + 1) / kWaves;
-#pragma unroll 2
-    for (int l = cnt * wave / kWaves; l < l1; ++l) {
-      const Rec64& s = tile[l];
-      const double dx = px - s.x, dy = py - s.y, dz = pz - s.z;
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      if (r2 == 0.0) continue;
-      double q;
-      if (HighOrder) {
-        const double ib = rsqrt_pos(r2 + s.s2);
-        const double ib2 = ib * ib;
-        q = kQ * fma(2.5, s.s2, r2) * (ib2 * ib2 * ib);
-      } else {
-        const double ir = rsqrt_pos(r2);
-        q = kQ * (ir * (ir * ir));
-        if (r2 <= kFar64 * s.s2) {
-          const double isg = rsqrt_pos(s.s2);
-          const double isg2 = isg * isg;
-          const double sb = r2 * isg2;
-          double e, gg;
-          core64(sb, tab, e, gg);
-          q = kCore64K * (isg2 * isg) * fma(sb, gg, e * (1.0 / 3.0));
-        }
-      }
-      u[0] += q * (s.ay * dz - s.az * dy);
-      u[1] += q * (s.az * dx - s.ax * dz);
-      u[2] += q * (s.ax * dy - s.ay * dx);
-    }
-  }
-  if (wave > 0)
-    for (int c = 0; c < 3; ++c) red[wave - 1][c][lane] = u[c];
-  __syncthreads();
-  if (wave > 0 || !active) return;
-  for (int w = 0; w < kWaves - 1; ++w)
-    for (int c = 0; c < 3; ++c) u[c] += red[w][c][lane];
-  double* out = a.splits > 1 ? a.partial + 192 * static_cast<size_t>(blockIdx.x) + 3 * lane
-                             : a.u + 3 * static_cast<size_t>(k);
-  for (int c = 0; c < 3; ++c) out[c] = u[c];
+// LDS written by one lane of a wave before this is read by another after it
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// u of a point group: its slabs added in order, one thread per component
-__global__ __launch_bounds__(192) void k_point_sum(const double* __restrict__ partial, int splits, int m,
-                                                   double* __restrict__ u) {
-  const int g = static_cast<int>(blockIdx.x), e = static_cast<int>(threadIdx.x);
-  if (64 * g + e / 3 >= m) return;
+constexpr int kPointBatch = 4;   // points whose lane sums are in LDS at once
+constexpr int kPointQuarter = 17;  // a component's 64 lane sums, 16 in each quarter of a row: the four
+constexpr int kPointRow = 68;      // lanes of each row then read different banks
+constexpr int kPointRows = 3 * kPointBatch;
+static_assert(4 * kPointRows <= 64, "four lanes per row");
+
+// Share: the block's waves share out the points and each walks the whole range;
+// otherwise they share out the range and each walks every point.
+template <bool HighOrder, int P, bool Share>
+__global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_point_velocity(PointArgs a) {
+  constexpr int kWaves = kTB / 64;
+  __shared__ double rows[kWaves][kPointRows * kPointRow];
+  __shared__ double acc[kWaves][3 * 64];
+  __shared__ __align__(16) double tab[HighOrder ? 2 : kCore64Pieces * kCore64Row];
+  if (!HighOrder) stage_core64(tab);
+  const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+  const int g = static_cast<int>(blockIdx.x) / a.splits, part = static_cast<int>(blockIdx.x) % a.splits;
+  const int npts = min(64, a.m - 64 * g);
+  const ConstPtr<double> pts = as_const(a.pts + 192 * static_cast<size_t>(g));
+  const int s0 = part * a.range, s1 = min(a.n, s0 + a.range);
+  for (int e = lane; e < 3 * 64; e += 64) acc[wave][e] = 0.0;
+  __syncthreads();
+  double* __restrict__ row = rows[wave];
+  const int slot = lane + (lane >> 4) * (kPointQuarter - 16);
+  const int quarter = (lane >> 2) * kPointRow + (lane & 3) * kPointQuarter;  // what this lane adds
+  const int pbegin = Share ? 64 / kWaves * wave : 0;
+  const int pend = Share ? min(pbegin + 64 / kWaves, npts) : npts;
+  for (int base = Share ? s0 : s0 + 64 * P * wave; base < s1; base += Share ? 64 * P : 64 * P * kWaves) {
+    // lanes past the range hold a particle without strength, far from everything
+    double x[P], y[P], z[P], s2[P], ax[P], ay[P], az[P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      const int l = base + 64 * j + lane;
+      const bool on = l < s1;
+      const Rec64 r = a.state[on ? l : s0];
+      x[j] = on ? r.x : 1e100;
+      y[j] = r.y; z[j] = r.z;
+      s2[j] = r.s2;
+      ax[j] = on ? r.ax : 0.0;
+      ay[j] = on ? r.ay : 0.0;
+      az[j] = on ? r.az : 0.0;
+    }
+    for (int p0 = pbegin; p0 < pend; p0 += kPointBatch) {
+      const int pn = min(kPointBatch, pend - p0);
+#pragma unroll 1
+      for (int p = 0; p < pn; ++p) {
+        const double px = pts[3 * (p0 + p)], py = pts[3 * (p0 + p) + 1], pz = pts[3 * (p0 + p) + 2];
+        double ux = 0.0, uy = 0.0, uz = 0.0;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+          const double dx = px - x[j], dy = py - y[j], dz = pz - z[j];
+          const double r2 = dx * dx + dy * dy + dz * dz;
+          double q;
+          if (HighOrder) {
+            const double ib = rsqrt_pos(r2 + s2[j]);
+            const double ib2 = ib * ib;
+            q = fma(2.5, s2[j], r2) * (ib2 * ib2 * ib);
+            if (r2 == 0.0) q = 0.0;
+          } else {
+            const double ir = rsqrt_pos(r2);
+            q = ir * (ir * ir);
+            if (r2 <= kFar64 * s2[j]) {
+              const double isg = rsqrt_pos(s2[j]);
+              const double isg2 = isg * isg;
+              const double sb = r2 * isg2;
+              double e, gg;
+              core64(sb, tab, e, gg);
+              q = (kCore64K / kQ) * (isg2 * isg) * fma(sb, gg, e * (1.0 / 3.0));
+              if (r2 == 0.0) q = 0.0;
+            }
+          }
+          ux += q * (ay[j] * dz - az[j] * dy);
+          uy += q * (az[j] * dx - ax[j] * dz);
+          uz += q * (ax[j] * dy - ay[j] * dx);
+        }
+        row[(3 * p) * kPointRow + slot] = ux;
+        row[(3 * p + 1) * kPointRow + slot] = uy;
+        row[(3 * p + 2) * kPointRow + slot] = uz;
+      }
+      wave_lds_sync();
+      double v = 0.0, w = 0.0;
+      if (lane < 12 * pn) {
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+          v += row[quarter + i];
+          w += row[quarter + i + 1];
+        }
+      }
+      v += w;
+      v += __shfl_xor(v, 1, 64);
+      v += __shfl_xor(v, 2, 64);
+      if (lane < 12 * pn && (lane & 3) == 0) acc[wave][3 * p0 + (lane >> 2)] += v;
+      wave_lds_sync();
+    }
+  }
+  __syncthreads();
+  const int e = static_cast<int>(threadIdx.x);
+  if (e >= 3 * npts) return;
+  double v = acc[0][e];
+  for (int w = 1; w < kWaves; ++w) v += acc[w][e];
+  v *= kQ;
+  if (a.splits > 1) a.partial[192 * static_cast<size_t>(blockIdx.x) + e] = v;
+  else a.u[192 * static_cast<size_t>(g) + e] = v;
+}
+
+// u of a point group: its slabs added in order, each quarter of them by a
+// thread per component (the chain of one group's 256 slabs is what a call with
+// few points waits for: 15 us with one thread per component, 8 with four)
+__global__ __launch_bounds__(4 * 192) void k_point_sum(const double* __restrict__ partial, int splits, int m,
+                                                       double* __restrict__ u) {
+  __shared__ double sum[3][192];
+  const int g = static_cast<int>(blockIdx.x), e = static_cast<int>(threadIdx.x) % 192;
+  const int quarter = static_cast<int>(threadIdx.x) / 192;
+  const bool on = 64 * g + e / 3 < m;
   const double* p = partial + 192 * static_cast<size_t>(g) * splits + e;
-  double v = p[0];
+  double v = 0.0;
+  if (on) {
+    const int i1 = splits * (quarter + 1) / 4;
 #pragma unroll 8
-  for (int i = 1; i < splits; ++i) v += p[192 * static_cast<size_t>(i)];
-  u[192 * static_cast<size_t>(g) + e] = v;
+    for (int i = splits * quarter / 4; i < i1; ++i) v += p[192 * static_cast<size_t>(i)];
+  }
+  if (quarter > 0) sum[quarter - 1][e] = v;
+  __syncthreads();
+  if (quarter == 0 && on) u[192 * static_cast<size_t>(g) + e] = ((v + sum[0][e]) + sum[1][e]) + sum[2][e];
 }
 
 // ---------------------------------------------------------------------
@@ -1050,14 +1125,6 @@ __device__ __forceinline__ void fold_s(const P32S& p, float tx, float ty, float 
   two_sum(hi[5], lo[5], fmaf(tax, p.ay, fmaf(-tay, p.ax, -3.0f * p.bz)));
 }
 
-// Read-only data of a launch seen through the constant address space: loads
-// at wave-uniform addresses then become scalar loads.
-template <typename T>
-using ConstPtr = const __attribute__((address_space(4))) T*;
-template <typename T>
-__device__ __forceinline__ ConstPtr<T> as_const(const T* p) {
-  return (ConstPtr<T>)(p);
-}
 // field by field (a struct copy out of that address space has no constructor)
 __device__ __forceinline__ Chunk32 load(ConstPtr<Chunk32> p, int i) {
   Chunk32 h;
@@ -2340,21 +2407,39 @@ hipError_t launch_point_velocity(const Rec64* state, int n, const double* pts, i
   if (m <= 0) return hipSuccess;
   PointArgs a{state, n, pts, m, u, scratch, 1, n};
   const int groups = (m + 63) / 64;
-  // source ranges until about 2,048 blocks exist (two full rounds of 4 blocks
-  // per CU), whole 256-source tiles each, as far as the scratch holds the slabs
-  const int64_t want = std::min<int64_t>((2048 + groups - 1) / groups, (n + kTB - 1) / kTB);
+  // Four particles per lane (the walk over the points and the sums across
+  // lanes are paid once for four) where that leaves a block for every CU;
+  // otherwise one, and the block's waves share out the points, which makes a
+  // wave's chain 16 points long: 100 points against 1,024 particles 39 us a
+  // call, with the range shared out 51.  Where the points alone fill the chip,
+  // few particles fill the lanes only if every wave has all of them: 100,000
+  // points against 128 particles 275 us a call, with the range shared out 358.
+  // Particle ranges of whole lanes, until about 4,096 blocks exist (five
+  // rounds of 3 blocks per CU: the last one, partly empty, weighs little; at
+  // 2,048 the 262,144-particle case takes 429 instead of 402 us), at most 256
+  // (k_point_sum walks them), as far as the scratch holds the slabs.
+  const int per = static_cast<int64_t>(groups) * ((n + 4 * kTB - 1) / (4 * kTB)) < 256 ? 1 : n < 4 * kTB ? 2 : 4;
+  const int set = per == 4 ? 4 * kTB : 64 * per;  // particles a block's lanes hold
+  const int64_t want = std::min<int64_t>(std::min((kPointBlocks + groups - 1) / groups, 256), (n + set - 1) / set);
   const int64_t fits = scratch ? static_cast<int64_t>(scratch_doubles / (192 * static_cast<size_t>(groups))) : 0;
   const int64_t splits = std::min(want, fits);
   if (splits > 1) {
-    a.range = static_cast<int>((n + splits * kTB - 1) / (splits * kTB)) * kTB;
+    a.range = static_cast<int>((n + splits * set - 1) / (splits * set)) * set;
     a.splits = (n + a.range - 1) / a.range;
   }
-  const dim3 grid(static_cast<unsigned>(groups) * a.splits);
-  if (high_order) hipLaunchKernelGGL(k_point_velocity<true>, grid, dim3(kTB), 0, st, a);
-  else hipLaunchKernelGGL(k_point_velocity<false>, grid, dim3(kTB), 0, st, a);
+  const dim3 grid(static_cast<unsigned>(groups) * a.splits), block(kTB);
+  if (high_order) {
+    if (per == 1) hipLaunchKernelGGL((k_point_velocity<true, 1, true>), grid, block, 0, st, a);
+    else if (per == 2) hipLaunchKernelGGL((k_point_velocity<true, 2, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_point_velocity<true, 4, false>), grid, block, 0, st, a);
+  } else {
+    if (per == 1) hipLaunchKernelGGL((k_point_velocity<false, 1, true>), grid, block, 0, st, a);
+    else if (per == 2) hipLaunchKernelGGL((k_point_velocity<false, 2, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_point_velocity<false, 4, false>), grid, block, 0, st, a);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.splits == 1) return e;
-  hipLaunchKernelGGL(k_point_sum, dim3(groups), dim3(192), 0, st, scratch, a.splits, m, u);
+  hipLaunchKernelGGL(k_point_sum, dim3(groups), dim3(4 * 192), 0, st, scratch, a.splits, m, u);
   return hipGetLastError();
 }
 
