@@ -331,7 +331,7 @@ void make_split(const pw_ctx* c, int split, std::vector<WorkItem>& items, std::v
       for (int64_t a = s.a; a < s.b; a += split, ++g.count)
         items.push_back({static_cast<int32_t>(t0), t1, static_cast<int32_t>(a),
                          static_cast<int32_t>(std::min<int64_t>(a + split, s.b)),
-                         static_cast<int32_t>(items.size()), 0, 0, 0});
+                         static_cast<int32_t>(items.size()), 0, chunk_of(c, a), chunk_of(c, t0)});
       groups.push_back(g);
     }
 }
@@ -355,20 +355,27 @@ int64_t split_items(const pw_ctx* c, int split) {
 //   kSplitItemsFew items, the chain of a wave is what is left to cut: 32 and
 //   16 (N = 1,000: 14.3 at 32, 17.0 at 16; N = 400: 14.5 at 64, 11.5, 10.0;
 //   N = 2,000: 23.9 at 64, 27.8 at 32).  Beyond kSplitItemsMax items (403 MB
-//   of partial rates) the ranges double.
-// * Beyond, the scalar-fed kernels, whose separated loops are shorter, over 64
-//   source parts and a persistent queue (32 from 196,608 particles: there 32
-//   are 3% faster in FP64 and level in FP32C at half the partial rates).
-//   FP64, split against scalar-fed: 24,000 particles 1,197 against 1,431,
-//   32,768 2,149 against 2,023, 65,536 8,088 against 6,955; FP32C: 32,000
-//   938 against 1,045, 49,152 2,062 against 2,031, 131,072 14,200 against
-//   11,216.  The high-order FP64 kernel has no scalar-fed form: split at every
-//   size (131,072: 33.8 ms against 34.7 LDS-tiled in 16 parts, 39.7 in one).
+//   of partial rates) the ranges double.  From kSplitSepItems items of whole
+//   256-source tiles, the 64-particle chunks' spheres are formed first (one
+//   launch, about 5 us) and chunks separated from an item's targets take the
+//   separated sums: two rings of 32,000 FP64 2,100 -> 1,825, FP32C 947 -> 757;
+//   48 rings of 512-16,384 FP64 4,158 -> 3,650, FP32C 1,807 -> 1,485; helix
+//   16,384 FP64 563 -> 534, FP32C 265 -> 257; at 6,400 items a coarse helix,
+//   which separates little, is still up to 4% slower with them.
+// * Beyond, the scalar-fed kernels, one persistent wave per 64 targets, over 64
+//   source parts (32 from 196,608 particles: there 32 are 3% faster in FP64 and
+//   level in FP32C at half the partial rates).  Split against scalar-fed, rings
+//   and helix: FP64 32,000 1,825 and 1,997 against 2,059 and 2,007, 48,000
+//   3,945 and 4,090 against 4,324 and 3,995, 64,000 7,465 and 6,632 against
+//   7,370 and 6,596; FP32C 64,000 2,862 and 3,087 against 3,393 and 3,267,
+//   96,000 7,232 and 6,940 against 7,155 and 6,627.  The high-order FP64 kernel
+//   has no scalar-fed form: split at every size (131,072: 33.8 ms against 34.7
+//   LDS-tiled in 16 parts, 39.7 in one).
 //
 // Systems of a batch are far below these sizes: split wins there by the same
-// rule (48 rings of 512-16,384, FP64 4.1 ms against 5.4 over 64 parts).
-constexpr int64_t kSplitUpTo64 = 32768, kSplitUpTo32 = 45056;
-constexpr int64_t kSplitItems = 2560, kSplitItemsFew = 640, kSplitItemsMax = 131072;
+// rule (48 rings of 512-16,384, FP64 3.65 ms against 5.4 over 64 parts).
+constexpr int64_t kSplitUpTo64 = 40960, kSplitUpTo32 = 65536;
+constexpr int64_t kSplitItems = 2560, kSplitItemsFew = 640, kSplitItemsMax = 131072, kSplitSepItems = 8192;
 
 pw::PairConfig auto_config(const pw_ctx* c, int launch_kind) {
   pw::PairConfig p;
@@ -380,6 +387,7 @@ pw::PairConfig auto_config(const pw_ctx* c, int launch_kind) {
     while (p.split < 256 && split_items(c, 2 * p.split) >= kSplitItems) p.split *= 2;
     while (p.split > 16 && p.split <= 64 && split_items(c, p.split / 2) <= kSplitItemsFew) p.split /= 2;
     while (split_items(c, p.split) > kSplitItemsMax && p.split < largest) p.split *= 2;
+    p.split_sep = launch_kind != pw::kPairFP64HO && p.split >= 256 && split_items(c, p.split) >= kSplitSepItems;
     return p;
   }
   p.parts = c->n < 196608 ? 64 : 32;
@@ -442,7 +450,7 @@ int ensure_kind(pw_ctx* c, int kind) {
     // the scalar-fed FP64 kernel's source records, allocated before any
     // step is captured (no allocation may happen inside a capture)
     int rc = PW_OK;
-    if (k.run.scalar_feed && kind == pw::kPairFP64 && !c->d_src64 && dalloc(&c->d_src64, c->n) != hipSuccess) {
+    if ((k.run.scalar_feed || k.run.split_sep) && kind == pw::kPairFP64 && !c->d_src64 && dalloc(&c->d_src64, c->n) != hipSuccess) {
       (void)hipGetLastError();
       rc = fail(PW_ERR_NOMEM, "scalar-fed FP64 source records");
     }
@@ -577,7 +585,7 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp&
   args.nchunks = c->nchunks;
   // the high-order kernel replaces the Gaussian kinds (pw_set_kernel)
   const int launch_kind = launch_kind_of(c, kind);
-  if (k.run.scalar_feed && launch_kind == pw::kPairFP64) args.src64 = c->d_src64;  // ensure_kind made it
+  if ((k.run.scalar_feed || k.run.split_sep) && launch_kind == pw::kPairFP64) args.src64 = c->d_src64;  // ensure_kind made it
   const int grid = c->num_cus * pw::pair_kernel_waves(launch_kind, k.run);
   pw::SumForm sum;
   sum.partial = c->partial;

@@ -35,7 +35,7 @@ struct WorkItem {
   int32_t t0, t1, s0, s1;
   int32_t part, nself;
   int32_t chunk0;  // source chunk (Chunk32) holding s0, for the scalar-fed FP32C kernel
-  int32_t pad2;
+  int32_t tchunk;  // split: the chunk of the targets [t0, t1)
 };
 
 // One group of at most 64 targets [t0, t1) of the split kernel: its items'
@@ -95,6 +95,8 @@ struct PairConfig {
   bool two_per_lane = false;// FP32C scalar-fed: two targets per lane
   int split = 0;           // sources per item of the split kernel (one block
                            // per 64 targets and source range); 0: not used
+  bool split_sep = false;  // split in ranges of whole 256-source tiles: chunks separated from
+                           // an item's targets take the separated sums
 };
 
 // Pair-kernel variants.

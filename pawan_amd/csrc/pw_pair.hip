@@ -1394,6 +1394,23 @@ __global__ __launch_bounds__(64) void k_src_chunks(const Rec64* __restrict__ sta
   }
 }
 
+// sources [l0, l1) of a chunk separated from every target of the wave, one
+// target per lane
+template <bool HighOrder>
+__device__ __forceinline__ void separated32(const T32& me, const Chunk32& h, ConstPtr<Src32> src, int l0, int l1,
+                                            float* hi, float* lo) {
+  const float tx = static_cast<float>(me.x - h.cx), ty = static_cast<float>(me.y - h.cy),
+              tz = static_cast<float>(me.z - h.cz);
+  const float cx = ty * me.az - tz * me.ay, cy = tz * me.ax - tx * me.az, cz = tx * me.ay - ty * me.ax;
+  P32S p;
+#pragma unroll 4
+  for (int l = l0; l < l1; ++l) {
+    const Src32 sr = load(src, l);
+    pair32s<HighOrder>(tx, ty, tz, me.hs2, me.ax, me.ay, me.az, cx, cy, cz, sr, p);
+  }
+  fold_s(p, tx, ty, tz, me.ax, me.ay, me.az, hi, lo);
+}
+
 // Targets [tb, tb + 64 TPL) of item it (a 64-lane wave of its own; with
 // TPL = 2 each lane owns targets tb + lane and tb + 64 + lane, and every
 // source record read from scalar registers feeds two pairs).
@@ -1599,6 +1616,28 @@ __device__ __forceinline__ Rec64 load(ConstPtr<Rec64> p, int i) {
   return r;
 }
 
+// sources [l0, l1) of a chunk separated from every target of the wave
+__device__ __forceinline__ void separated64(const T64& me, const Chunk32& h, ConstPtr<Src64> src, int l0, int l1,
+                                            AccF64& a) {
+  const double tx = me.x - h.cx, ty = me.y - h.cy, tz = me.z - h.cz;
+  const double cx = ty * me.az - tz * me.ay, cy = tz * me.ax - tx * me.az, cz = tx * me.ay - ty * me.ax;
+  P64S p;
+#pragma unroll 2
+  for (int l = l0; l < l1; ++l)
+    pair64s(tx, ty, tz, me.ax, me.ay, me.az, cx, cy, cz, src[l].rx, src[l].ry, src[l].rz, src[l].ax,
+            src[l].ay, src[l].az, src[l].mx, src[l].my, src[l].mz, p);
+  // u += (A x t' - M)/4pi; the stretching's A and B join the factored sums
+  a.ux += kQ * ((p.ay * tz - p.az * ty) - p.mx);
+  a.uy += kQ * ((p.az * tx - p.ax * tz) - p.my);
+  a.uz += kQ * ((p.ax * ty - p.ay * tx) - p.mz);
+  a.ax += kQ * p.ax;
+  a.ay += kQ * p.ay;
+  a.az += kQ * p.az;
+  a.bx += (-3.0 * kQ) * p.bx;
+  a.by += (-3.0 * kQ) * p.by;
+  a.bz += (-3.0 * kQ) * p.bz;
+}
+
 // Targets [tb, tb + 64) of item it (a 64-lane wave of its own).
 __device__ __forceinline__ void wave_fp64s(const WorkItem& it, int tb, double nu, const Rec64* state_g,
                                            const Chunk32* chunks_g, int nchunks, const Src64* src_g,
@@ -1636,23 +1675,7 @@ __device__ __forceinline__ void wave_fp64s(const WorkItem& it, int tb, double nu
     const double gap = sqrt(ddx * ddx + ddy * ddy + ddz * ddz) * 0.999999 - rW - h.r;
     const bool sep = gap > 0.0 && gap * gap > kFar64 * (h2W + h.h2) * 1.0001 && h.r <= gap;
     if (sep) {
-      const double tx = me.x - h.cx, ty = me.y - h.cy, tz = me.z - h.cz;
-      const double cx = ty * me.az - tz * me.ay, cy = tz * me.ax - tx * me.az, cz = tx * me.ay - ty * me.ax;
-      P64S p;
-#pragma unroll 2
-      for (int l = l0; l < l1; ++l)
-        pair64s(tx, ty, tz, me.ax, me.ay, me.az, cx, cy, cz, src[l].rx, src[l].ry, src[l].rz, src[l].ax,
-                src[l].ay, src[l].az, src[l].mx, src[l].my, src[l].mz, p);
-      // u += (A x t' - M)/4pi; the stretching's A and B join the factored sums
-      a.ux += kQ * ((p.ay * tz - p.az * ty) - p.mx);
-      a.uy += kQ * ((p.az * tx - p.ax * tz) - p.my);
-      a.uz += kQ * ((p.ax * ty - p.ay * tx) - p.mz);
-      a.ax += kQ * p.ax;
-      a.ay += kQ * p.ay;
-      a.az += kQ * p.az;
-      a.bx += (-3.0 * kQ) * p.bx;
-      a.by += (-3.0 * kQ) * p.by;
-      a.bz += (-3.0 * kQ) * p.bz;
+      separated64(me, h, src, l0, l1, a);
     } else {
 #pragma unroll 1
       for (int l = l0; l < l1; ++l)
@@ -2124,9 +2147,18 @@ __global__ __launch_bounds__(kTB) void k_pair_fp32c_plain(PairArgs a) { pair_ent
 // blocks exist (auto_config in pw_capi.hip), down to 16 sources, 4
 // per wave.  Measured per right-hand side, one part LDS-tiled against this:
 // ring of 1,000 FP64 347 -> 14 us, two rings of 4,816 1,155 -> 74 us (FP64),
-// 1,017 -> 63 us (high-order), 728 -> 42 us (FP32C); at 24,000 FP64 it runs
-// 481 G pairs/s, bound by its instructions per pair (52 beyond the core, 98 in
-// it), no longer by waves in flight.
+// 1,017 -> 63 us (high-order), 728 -> 42 us (FP32C).
+//
+// Sep: where the launch is large enough to pay for the chunks' spheres, the
+// chunks of a whole tile that are separated from the item's targets take the
+// scalar-fed kernels' separated sums (32 instructions a pair in FP64, 26 in
+// FP32C, against 52 and 38 beyond the core and 98 and 60 in it); a tile whose
+// four chunks all are is not staged.  In FP64 a tile with some of them is shared
+// out in quarters of chunks, so that a wave with a separated chunk does not wait
+// for the others (3%; in FP32C the folds per quarter cost more than that).  FP32C
+// is held to 64 registers (8 waves per SIMD): 1% to 4% against the 78 it would
+// take.  Two rings of 16,000: FP64 584 -> 556 us, FP32C 254 -> 213; of 32,000:
+// 2,100 -> 1,825 and 947 -> 757 (561 and 1,353 G pairs/s).
 // ---------------------------------------------------------------------
 template <int Kind>
 struct SplitSum;
@@ -2145,6 +2177,11 @@ struct SplitSum<kPairFP64> {
   static __device__ __forceinline__ Src source(const Rec64& r) { return r; }
   __device__ __forceinline__ void pair(const Src& s, const double* __restrict__ tab) { pair64(me, s, tab, a); }
   __device__ __forceinline__ void chunk_end() {}
+  static constexpr bool kMix = true;
+  static constexpr float kFar = static_cast<float>(kFar64);
+  __device__ __forceinline__ void separated(const PairArgs& pa, const Chunk32& h, int l0, int l1) {
+    separated64(me, h, as_const(pa.src64), h.first + l0, h.first + l1, a);
+  }
   __device__ __forceinline__ void result(double (&r)[6]) const {
     r[0] = a.ux; r[1] = a.uy; r[2] = a.uz;
     r[3] = (me.ay * a.az - me.az * a.ay) + a.bx;
@@ -2165,6 +2202,7 @@ struct SplitSum<kPairFP64HO> {
     me.nu2 = 2.0 * nu;
   }
   static __device__ __forceinline__ Src source(const Rec64& r) { return r; }
+  static constexpr bool kMix = false;
   __device__ __forceinline__ void pair(const Src& s, const double* __restrict__) { pair64_ho(me, s, a); }
   __device__ __forceinline__ void chunk_end() {}
   __device__ __forceinline__ void result(double (&r)[6]) const {
@@ -2215,6 +2253,11 @@ struct SplitSum32 {
     fold(p, me.ax, me.ay, me.az, hi, lo);
     p = P32{};
   }
+  static constexpr bool kMix = false;
+  static constexpr float kFar = kFar32;
+  __device__ __forceinline__ void separated(const PairArgs& pa, const Chunk32& h, int l0, int l1) {
+    separated32<HighOrder>(me, h, as_const(pa.src), h.first + l0, h.first + l1, hi, lo);
+  }
   __device__ __forceinline__ void result(double (&r)[6]) const {
 #pragma unroll
     for (int k = 0; k < kAcc; ++k) r[k] = kQ * (static_cast<double>(hi[k]) + static_cast<double>(lo[k]));
@@ -2228,8 +2271,8 @@ struct SplitSum<kPairFP32C> : SplitSum32<false> {};
 template <>
 struct SplitSum<kPairFP32CHO> : SplitSum32<true> {};
 
-template <int Kind>
-__global__ __launch_bounds__(kTB) void k_pair_split(PairArgs pa) {
+template <int Kind, bool Sep>
+__global__ __launch_bounds__(kTB, Sep&& Kind != kPairFP64 ? 8 : 1) void k_pair_split(PairArgs pa) {
   using Sum = SplitSum<Kind>;
   constexpr int kWaves = kTB / 64;
   constexpr size_t kTileBytes = kTB * sizeof(typename Sum::Src);
@@ -2240,22 +2283,49 @@ __global__ __launch_bounds__(kTB) void k_pair_split(PairArgs pa) {
   const Rec64* __restrict__ state = pa.state;
   const WorkItem it = pa.items[blockIdx.x];
   const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
-  if (Sum::kTable) stage_core64(tab);  // (synchronised with the first tile)
+  bool staged = false;  // the table (synchronised with the first tile)
   const int t = it.t0 + lane;
   const bool active = t < it.t1;
   Sum sum;
   sum.init(state[active ? t : it.t0], pa.nu);
   for (int base = it.s0; base < it.s1; base += kTB) {
     const int cnt = min(kTB, it.s1 - base);
-    __syncthreads();
-    if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = Sum::source(state[base + threadIdx.x]);
-    __syncthreads();
-    const int l0 = cnt * wave / kWaves, l1 = cnt * (wave + 1) / kWaves;
-    if (base + l0 < it.t1 && base + l1 > it.t0) {  // the wave's own targets may be among these sources
-      for (int l = l0; l < l1; ++l)
-        if (base + l != t) sum.pair(tile[l], tab);  // the self pair is never evaluated
-    } else {
-      for (int l = l0; l < l1; ++l) sum.pair(tile[l], tab);
+    unsigned far = 0;  // bit w: the chunk of wave w is separated from the targets (the same in all waves)
+    const int c0 = it.chunk0 + (base - it.s0) / 64;
+    if constexpr (Sep) {
+      if (cnt == kTB) {
+        const Chunk32 h = pa.chunks[c0 + (lane & 3)], w = pa.chunks[it.tchunk];
+        const double dx = h.cx - w.cx, dy = h.cy - w.cy, dz = h.cz - w.cz;
+        const float gap = static_cast<float>(sqrt(fma(dz, dz, fma(dy, dy, dx * dx)))) * 0.99999f - w.r - h.r;
+        const bool sep = gap > 0.0f && gap * gap > Sum::kFar * (w.h2 + h.h2) * 1.0001f && h.r <= gap;
+        far = static_cast<unsigned>(__ballot(sep)) & 15u;
+      }
+    }
+    if (far != 15u) {
+      __syncthreads();
+      if (Sum::kTable && !staged) stage_core64(tab);
+      staged = true;
+      if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = Sum::source(state[base + threadIdx.x]);
+      __syncthreads();
+    }
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    const bool mixed = Sep && Sum::kMix && far != 0 && far != 15u;
+    const int q1 = mixed ? kWaves : w + 1;
+#pragma unroll 1
+    for (int q = mixed ? 0 : w; q < q1; ++q) {
+      const int l0 = mixed ? 64 * q + 16 * w : cnt * w / kWaves, l1 = mixed ? l0 + 16 : cnt * (w + 1) / kWaves;
+      if constexpr (Sep) {
+        if (far >> q & 1u) {
+          sum.separated(pa, load(as_const(pa.chunks), c0 + q), l0 - 64 * q, l1 - 64 * q);
+          continue;
+        }
+      }
+      if (base + l0 < it.t1 && base + l1 > it.t0) {  // the wave's own targets may be among these sources
+        for (int l = l0; l < l1; ++l)
+          if (base + l != t) sum.pair(tile[l], tab);  // the self pair is never evaluated
+      } else {
+        for (int l = l0; l < l1; ++l) sum.pair(tile[l], tab);
+      }
     }
     sum.chunk_end();
   }
@@ -2325,11 +2395,32 @@ hipError_t launch_pair(int kind, const PairConfig& cfg, const PairArgs& args, in
   if (args.nitems <= 0) return hipSuccess;
   if (cfg.split > 0) {
     const dim3 g(static_cast<unsigned>(args.nitems)), block(kTB);
+    const bool sep = cfg.split_sep;
+    if (sep) {
+      if (kind == kPairFP64HO || cfg.split % kTB) return hipErrorInvalidValue;
+      if (!args.chunks || args.nchunks <= 0 || !(kind == kPairFP64 ? static_cast<void*>(args.src64) : args.src))
+        return hipErrorInvalidValue;
+      if (kind == kPairFP64)
+        hipLaunchKernelGGL(k_src_chunks64, dim3(args.nchunks), dim3(64), 0, st, args.state, args.chunks, args.src64);
+      else
+        hipLaunchKernelGGL(k_src_chunks, dim3(args.nchunks), dim3(64), 0, st, args.state, args.chunks, args.src);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
     switch (kind) {
-      case kPairFP64: hipLaunchKernelGGL(k_pair_split<kPairFP64>, g, block, 0, st, args); break;
-      case kPairFP64HO: hipLaunchKernelGGL(k_pair_split<kPairFP64HO>, g, block, 0, st, args); break;
-      case kPairFP32C: hipLaunchKernelGGL(k_pair_split<kPairFP32C>, g, block, 0, st, args); break;
-      case kPairFP32CHO: hipLaunchKernelGGL(k_pair_split<kPairFP32CHO>, g, block, 0, st, args); break;
+      case kPairFP64:
+        if (sep) hipLaunchKernelGGL((k_pair_split<kPairFP64, true>), g, block, 0, st, args);
+        else hipLaunchKernelGGL((k_pair_split<kPairFP64, false>), g, block, 0, st, args);
+        break;
+      case kPairFP64HO: hipLaunchKernelGGL((k_pair_split<kPairFP64HO, false>), g, block, 0, st, args); break;
+      case kPairFP32C:
+        if (sep) hipLaunchKernelGGL((k_pair_split<kPairFP32C, true>), g, block, 0, st, args);
+        else hipLaunchKernelGGL((k_pair_split<kPairFP32C, false>), g, block, 0, st, args);
+        break;
+      case kPairFP32CHO:
+        if (sep) hipLaunchKernelGGL((k_pair_split<kPairFP32CHO, true>), g, block, 0, st, args);
+        else hipLaunchKernelGGL((k_pair_split<kPairFP32CHO, false>), g, block, 0, st, args);
+        break;
       default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
