@@ -1891,6 +1891,17 @@ __device__ __forceinline__ void pair32_rel_core(float tx, float ty, float tz, co
   else accumulate32_pair_n3(dx, dy, dz, q, f, t.ax, t.ay, t.az, s, p);
 }
 
+// A run that is not separated from the slice as a whole is sorted while it is
+// staged: the sources beyond the core of every target of the slice first (each
+// lane tests the one it stages against the slice's sphere), which take the
+// separated sums, then the rest.  Both loops stay free of a choice per source: made
+// by a ballot in the loop it cost more (41.7 -> 44.5 ms on the 1M helix) than
+// the instructions it saved.  The kernel is bound by its vector instructions
+// (1.51 per cycle and CU, 46 a pair) with its LDS 76% busy.  Lists, nodes and
+// chunks are read through the constant address space: scalar loads, and the
+// registers their copies took.  1M helix, solve 41.1 -> 38.0 ms; 300,032 with the
+// network 18.8 -> 17.5.
+//
 // Halves: the slice holds at most 32 targets; lanes 32-63 take the same
 // targets as lanes 0-31 and each half every other source of a tile, and
 // the two halves' sums are added at the end (a leaf's last slice is often
@@ -1899,13 +1910,19 @@ template <bool HighOrder, bool Uniform, bool Halves>
 __device__ __forceinline__ void near_slice(const NearArgs& a, const NearItem& it, int slice, SrcRel* tile,
                                            const float4* __restrict__ tab) {
   const int T = it.T;
+  const ConstPtr<NodeRec> nodes = as_const(a.nodes);
+  const ConstPtr<LeafChunk> chunks = as_const(a.chunks);
   const int lane = static_cast<int>(threadIdx.x);
   const int h = Halves ? lane >> 5 : 0;  // this lane's half: sources h, h + 2, ...
   constexpr int kStep = Halves ? 2 : 1;
-  const int t0 = a.nodes[T].first, t1 = a.nodes[T].last;
-  const double tcx = a.nodes[T].cx, tcy = a.nodes[T].cy, tcz = a.nodes[T].cz;
-  const float tr = a.nodes[T].r;
-  const LeafChunk ts = a.chunks[kLeafChunks * T + slice];  // this slice's targets
+  const int t0 = nodes[T].first, t1 = nodes[T].last;
+  const double tcx = nodes[T].cx, tcy = nodes[T].cy, tcz = nodes[T].cz;
+  const float tr = nodes[T].r;
+  const ConstPtr<LeafChunk> ts = chunks + (kLeafChunks * T + slice);  // this slice's targets
+  const double scx = ts->cx, scy = ts->cy, scz = ts->cz;
+  const float sr = ts->r;
+  const float sx = uniform(static_cast<float>(scx - tcx)), sy = uniform(static_cast<float>(scy - tcy)),
+              sz = uniform(static_cast<float>(scz - tcz));
   const int self = kNearSlice * slice + (Halves ? lane & 31 : lane);  // index of this lane's target in T
   const int t = t0 + self;
   const bool active = t < t1;
@@ -1926,22 +1943,30 @@ __device__ __forceinline__ void near_slice(const NearArgs& a, const NearItem& it
 #pragma unroll
   for (int k = 0; k < kAcc; ++k) hi[k] = lo[k] = 0.0f;
   PSE32F pse;
-  const int* __restrict__ L = a.list + static_cast<size_t>(T) * a.cap;
+  const ConstPtr<int> L = as_const(a.list) + static_cast<size_t>(T) * a.cap;
   for (int k = it.k0; k < it.k1; ++k) {
     const int id = L[k];
-    const int base = a.nodes[id].first;
-    const int cnt = a.nodes[id].last - base;
+    const int base = nodes[id].first;
+    const int cnt = nodes[id].last - base;
     // every pair of the two leaves beyond the Gaussian core: no core test
-    const double ddx = a.nodes[id].cx - tcx, ddy = a.nodes[id].cy - tcy, ddz = a.nodes[id].cz - tcz;
-    const float gap = static_cast<float>(sqrt(ddx * ddx + ddy * ddy + ddz * ddz)) - tr - a.nodes[id].r;
+    const double ddx = nodes[id].cx - tcx, ddy = nodes[id].cy - tcy, ddz = nodes[id].cz - tcz;
+    const float gap = static_cast<float>(sqrt(ddx * ddx + ddy * ddy + ddz * ddz)) - tr - nodes[id].r;
     const bool all_far = gap > 0.0f && gap * gap > a.gap2 * 1.0001f;
     const bool diag = id == T;
     for (int c0 = 0; c0 < cnt; c0 += kNearSlice) {
       const int nc = min(kNearSlice, cnt - c0);
-      __syncthreads();  // the previous tile is read
+      // a run of the leaf beyond the core of every target of the slice
+      bool sep = all_far;
+      if (!sep) {
+        const ConstPtr<LeafChunk> cs = chunks + (kLeafChunks * id + (c0 >> 6));
+        const double ex = cs->cx - scx, ey = cs->cy - scy, ez = cs->cz - scz;
+        const float g = static_cast<float>(sqrt(ex * ex + ey * ey + ez * ez)) - sr - cs->r;
+        sep = g > 0.0f && g * g > a.gap2 * 1.0001f;
+      }
+      SrcRel f;
+      bool clear = false;
       if (lane < nc) {
         const Rec64 r = a.sorted[base + c0 + lane];
-        SrcRel f;
         f.rx = static_cast<float>(r.x - tcx);
         f.ry = static_cast<float>(r.y - tcy);
         f.rz = static_cast<float>(r.z - tcz);
@@ -1954,34 +1979,38 @@ __device__ __forceinline__ void near_slice(const NearArgs& a, const NearItem& it
         f.mz = f.ax * f.ry - f.ay * f.rx;
         f.vol = static_cast<float>(r.vol);
         f.pad = 0.0f;
-        tile[lane] = f;
+        // beyond the core of every target by itself
+        const float ex = f.rx - sx, ey = f.ry - sy, ez = f.rz - sz;
+        const float g = sqrtf(fmaf(ez, ez, fmaf(ey, ey, ex * ex))) - sr;
+        clear = sep || (g > 0.0f && g * g > a.gap2 * 1.0001f);
       }
+      uint64_t far = __ballot(clear);
+      if (__popcll(far) < kClearMin && !sep) far = 0;
+      const int nfar = __popcll(far);
+      const uint64_t below = (uint64_t(1) << lane) - 1;  // the clear sources first, each part in order
+      const int slot = far >> lane & 1 ? __popcll(far & below) : nfar + __popcll(~far & below);
+      // this target's slot in the tile, if there (its own source is never clear)
+      const int own = diag && (c0 >> 6) == slice ? (Halves ? __shfl(slot, lane & 31) : slot) : -1;
+      __syncthreads();  // the previous tile is read
+      if (lane < nc) tile[slot] = f;
       __syncthreads();
       if (!active) continue;
-      // a run of the leaf beyond the core of every target of the slice
-      bool sep = all_far;
-      if (!sep) {
-        const LeafChunk& cs = a.chunks[kLeafChunks * id + (c0 >> 6)];
-        const double ex = cs.cx - ts.cx, ey = cs.cy - ts.cy, ez = cs.cz - ts.cz;
-        const float g = static_cast<float>(sqrt(ex * ex + ey * ey + ez * ez)) - ts.r - cs.r;
-        sep = g > 0.0f && g * g > a.gap2 * 1.0001f;
-      }
-      if (sep) {
+      if (nfar) {
         P32S q;
 #pragma unroll 2
-        for (int l = h; l < nc; l += kStep)
+        for (int l = h; l < nfar; l += kStep)
           pair32s<HighOrder>(rx, ry, rz, me.hs2, me.ax, me.ay, me.az, ctx, cty, ctz, tile[l], q);
         fold_s(q, rx, ry, rz, me.ax, me.ay, me.az, hi, lo);
-        continue;
+        if (nfar == nc) continue;
       }
       P32 p;
       if (diag) {
-        const int own = self - c0;  // this target's slot in the tile, if there
-        for (int l = h; l < nc; l += kStep)
+        for (int l = nfar + h; l < nc; l += kStep)
           if (l != own) pair32_rel_core<HighOrder, Uniform>(rx, ry, rz, me, tile[l], tab, a, p, pse);
       } else {
 #pragma unroll 1
-        for (int l = h; l < nc; l += kStep) pair32_rel_core<HighOrder, Uniform>(rx, ry, rz, me, tile[l], tab, a, p, pse);
+        for (int l = nfar + h; l < nc; l += kStep)
+          pair32_rel_core<HighOrder, Uniform>(rx, ry, rz, me, tile[l], tab, a, p, pse);
       }
       if (HighOrder) fold(p, me.ax, me.ay, me.az, hi, lo);
       else fold_n3(p, hi, lo);

@@ -1,0 +1,42 @@
+"""Near field of the tree path with nothing accepted as far, so that it is the
+whole sum: tiles sorted into sources clear of a slice's targets and the rest,
+slices of more and of fewer than 32 targets, the leaf's own run, one radius and
+radii that vary; against the LDS-tiled FP64 kernel at the repository's FP32C
+bars."""
+import numpy as np
+import pytest
+
+from conftest import normwise
+from pawan_amd import capi, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _cut(s, n, varied):
+    r = s.radius[:n] * (np.linspace(0.5, 1.5, n) if varied else 1.0)
+    return W.ParticleSystem(off=np.array([0, n], dtype=np.int64), pos=s.pos[:n].copy(), alpha=s.alpha[:n].copy(),
+                            radius=r, volume=s.volume[:n].copy(), nu=1e-3, coupled=True, name="cut")
+
+
+SYSTEMS = {
+    "ring": lambda: _cut(W.cored_ring(R=1.0, gamma=1.0, sigma=0.1, core=0.1, nst=40, ncs_ring=4), 97, False),
+    "rings": lambda: _cut(W.leapfrog_64k(301), 4801, False),
+    "rings, varied radii": lambda: _cut(W.leapfrog_64k(301), 4801, True),
+    "helix": lambda: _cut(W.helix_wake(16384), 8257, False),
+}
+
+
+@pytest.mark.parametrize("name", SYSTEMS)
+@pytest.mark.parametrize("kernel", [0, 1])
+def test_near_field_alone(name, kernel):
+    s = SYSTEMS[name]()
+    with capi.Solver(s) as g:
+        g.set_kernel(kernel)
+        g.set_pair_config("fp64", 2)
+        ru, rw = g.solve("fp64")
+        g.ff_set_params(1e-6, 0.0, use_mlp=False)
+        u, w = g.solve("learned")
+        assert g.ff_info()["near_pairs"] > 0.98 * s.n * (s.n - 1)
+    eu, ew = normwise(u, ru), normwise(w, rw)
+    print(f"{name} kernel {kernel}: {eu:.2e} {ew:.2e}", flush=True)
+    assert eu < 1e-6 and ew < 1e-5
