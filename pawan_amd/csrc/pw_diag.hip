@@ -162,7 +162,7 @@ __global__ __launch_bounds__(kTB) void k_diag_pairs(
   __shared__ Rec64 tile[kTB];
   __shared__ double red[kWaves * kDiagQuad];
   __shared__ __align__(16) double tab[HighOrder ? 2 : kCore64Pieces * kCore64Row];
-  if (!HighOrder) stage_core64(tab);  // (synchronised with the first tile)
+  if (!HighOrder) stage_core64<kTB>(tab);  // (synchronised with the first tile)
   const WorkItem it = items[blockIdx.x];
   const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
   const int t = it.t0 + lane;

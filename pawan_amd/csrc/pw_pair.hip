@@ -299,7 +299,7 @@ __device__ __forceinline__ void item_fp64(const PairArgs& pa, const WorkItem& it
   __shared__ double s_tb[kTB / 64][6];  // each wave's targets' box
   __shared__ double s_b[kTB / 64][7];   // each staged chunk's box (relative to c_T) and largest sigma^2/2
   __shared__ __align__(16) double tab[kCore64Pieces * kCore64Row];
-  stage_core64(tab);  // (synchronised with the first tile)
+  stage_core64<kTB>(tab);  // (synchronised with the first tile)
   const Rec64* __restrict__ state = pa.state;
   const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
   const int t = it.t0 + static_cast<int>(threadIdx.x);
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
   __shared__ double rows[kWaves][kPointRows * kPointRow];
   __shared__ double acc[kWaves][3 * 64];
   __shared__ __align__(16) double tab[HighOrder ? 2 : kCore64Pieces * kCore64Row];
-  if (!HighOrder) stage_core64(tab);
+  if (!HighOrder) stage_core64<kTB>(tab);
   const int lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
   const int g = static_cast<int>(blockIdx.x) / a.splits, part = static_cast<int>(blockIdx.x) % a.splits;
   const int npts = min(64, a.m - 64 * g);
@@ -1760,7 +1760,7 @@ __device__ __forceinline__ void wave_fp64s(const WorkItem& it, int tb, double nu
 template <bool Persistent>
 __device__ __forceinline__ void fp64s_entry(const PairArgs& a) {
   __shared__ __align__(16) double tab[kCore64Pieces * kCore64Row];
-  stage_core64(tab);
+  stage_core64<64>(tab);
   __syncthreads();
   const int waves = 4 * a.nitems;
   for (int w = Persistent ? -1 : static_cast<int>(blockIdx.x);;) {
@@ -2240,7 +2240,7 @@ __global__ __launch_bounds__(kTB) void k_pair_fp32c_plain(PairArgs a) { pair_ent
 // after another.  Here the source range of an item shrinks until hundreds of
 // blocks exist (auto_config in pw_capi.hip), down to 16 sources, 4
 // per wave.  Measured per right-hand side, one part LDS-tiled against this:
-// ring of 1,000 FP64 347 -> 14 us, two rings of 4,816 1,155 -> 74 us (FP64),
+// ring of 1,000 FP64 347 -> 12.3 us, two rings of 4,816 1,155 -> 74 us (FP64),
 // 1,017 -> 63 us (high-order), 728 -> 42 us (FP32C).
 //
 // Sep: where the launch is large enough to pay for the chunks' spheres, the
@@ -2366,7 +2366,7 @@ template <>
 struct SplitSum<kPairFP32CHO> : SplitSum32<true> {};
 
 template <int Kind, bool Sep>
-__global__ __launch_bounds__(kTB, Sep&& Kind != kPairFP64 ? 8 : 1) void k_pair_split(PairArgs pa) {
+__global__ __launch_bounds__(kTB, !Sep ? 1 : Kind == kPairFP64 ? 4 : 8) void k_pair_split(PairArgs pa) {
   using Sum = SplitSum<Kind>;
   constexpr int kWaves = kTB / 64;
   constexpr size_t kTileBytes = kTB * sizeof(typename Sum::Src);
@@ -2396,10 +2396,12 @@ __global__ __launch_bounds__(kTB, Sep&& Kind != kPairFP64 ? 8 : 1) void k_pair_s
       }
     }
     if (far != 15u) {
+      const bool on = static_cast<int>(threadIdx.x) < cnt;
+      const Rec64 rec = state[base + (on ? static_cast<int>(threadIdx.x) : 0)];  // in flight with the table
       __syncthreads();
-      if (Sum::kTable && !staged) stage_core64(tab);
+      if (Sum::kTable && !staged) stage_core64<kTB>(tab);
       staged = true;
-      if (static_cast<int>(threadIdx.x) < cnt) tile[threadIdx.x] = Sum::source(state[base + threadIdx.x]);
+      if (on) tile[threadIdx.x] = Sum::source(rec);
       __syncthreads();
     }
     const int w = __builtin_amdgcn_readfirstlane(wave);

@@ -24,6 +24,12 @@ constexpr int kEW = 256;
 // The partial rates are summed in order (deterministic).  Sum: 0 none, 1
 // slices of n rows, 2 slabs of 64 rows (k_pair_split).
 constexpr int kGroupThreads = 6 * 64;  // a group's 64 rows
+// Loads of the split sum in flight at a time.  The kernel is a chain of memory
+// latencies (a group's slabs were written through other XCDs' caches): with 8,
+// and the stage's own inputs loaded after the sum, a right-hand side of 1,000
+// particles took 14.5 us (FP64), with 8 and the inputs loaded first 13.1, with
+// 16 12.4, with 32 12.5 (and 200 particles 9.0, 8.8, 9.6).
+constexpr int kSumUnroll = 16;
 
 struct FinishArgs {
   const double* partial;
@@ -35,55 +41,99 @@ struct FinishArgs {
   StageOp op;
 };
 
-template <int Op>
-__device__ __forceinline__ void stage_component(const StageOp& op, int64_t e, double k) {
-#pragma clang fp contract(off)
-  if (Op == kStageNone) return;
+// What a component's stage arithmetic reads besides the rate; loaded before the
+// partial rates are summed, so that the two waits overlap.
+struct StageIn {
+  double y = 0, next = 0, k1 = 0, k2 = 0, k3 = 0;
+};
+
+// the component's place in Rec64: x y z s2 ax ay az vol
+__device__ __forceinline__ int64_t stage_at(int64_t e) {
   const int64_t t = e / 6;
   const int c = static_cast<int>(e - 6 * t);
-  const int64_t at = 8 * t + c + (c >= 3 ? 1 : 0);  // the component in Rec64: x y z s2 ax ay az vol
-  double* y = reinterpret_cast<double*>(op.y);
-  const double yc = y[at];
+  return 8 * t + c + (c >= 3 ? 1 : 0);
+}
+
+template <int Op>
+__device__ __forceinline__ StageIn stage_in(const StageOp& op, int64_t e) {
+  StageIn in;
+  if (Op == kStageNone) return in;
+  const int64_t at = stage_at(e);
+  const double* y = reinterpret_cast<const double*>(op.y);
+  in.y = y[at];
+  if ((Op == kStageLin || Op == kStageRk3Mid) && e % 3 == 2) in.next = y[at + 1];  // s2, vol
+  if (Op == kStageRk3Mid || Op == kStageRk4 || Op == kStageRk3) in.k1 = reinterpret_cast<const double*>(op.k1)[e];
+  if (Op == kStageRk4 || Op == kStageRk3) in.k2 = reinterpret_cast<const double*>(op.k2)[e];
+  if (Op == kStageRk4) in.k3 = reinterpret_cast<const double*>(op.k3)[e];
+  return in;
+}
+
+template <int Op>
+__device__ __forceinline__ void stage_component(const StageOp& op, const StageIn& in, int64_t e, double k) {
+#pragma clang fp contract(off)
+  if (Op == kStageNone) return;
+  const int64_t at = stage_at(e);
   if (Op == kStageLin || Op == kStageRk3Mid) {
     double* out = reinterpret_cast<double*>(op.out);
     if (Op == kStageLin) {
-      out[at] = k * op.a + yc;
+      out[at] = k * op.a + in.y;
     } else {
-      double* k1 = reinterpret_cast<double*>(op.k1);
-      const double b1 = k1[e] * op.a;
-      out[at] = (k * op.b + yc) - b1;
-      k1[e] = b1;
+      const double b1 = in.k1 * op.a;
+      out[at] = (k * op.b + in.y) - b1;
+      reinterpret_cast<double*>(op.k1)[e] = b1;
     }
-    if (c == 2 || c == 5) out[at + 1] = y[at + 1];  // s2, vol
-  } else if (Op == kStageRk4) {
-    const double a1 = reinterpret_cast<const double*>(op.k1)[e], a2 = reinterpret_cast<const double*>(op.k2)[e],
-                 a3 = reinterpret_cast<const double*>(op.k3)[e];
-    y[at] = yc + ((a1 + k) * op.a + (a2 + a3) * op.b);
-  } else if (Op == kStageRk3) {
-    const double b1 = reinterpret_cast<const double*>(op.k1)[e], a2 = reinterpret_cast<const double*>(op.k2)[e];
-    y[at] = yc + ((b1 * (1.0 / 6.0) + k * op.a) + a2 * op.b);
-  } else {
-    y[at] = yc + k * op.a;
+    if (e % 3 == 2) out[at + 1] = in.next;
+    return;
   }
+  double* y = reinterpret_cast<double*>(op.y);
+  if (Op == kStageRk4)
+    y[at] = in.y + ((in.k1 + k) * op.a + (in.k2 + in.k3) * op.b);
+  else if (Op == kStageRk3)
+    y[at] = in.y + ((in.k1 * (1.0 / 6.0) + k * op.a) + in.k2 * op.b);
+  else
+    y[at] = in.y + k * op.a;
+}
+
+// p[0] + p[stride] + ... in that order, UNROLL loads in flight at a time
+template <int kUnroll>
+__device__ __forceinline__ double sum_slices(const double* __restrict__ p, size_t stride, int count) {
+  double k = p[0];
+  int i = 1;
+  for (; i + kUnroll <= count; i += kUnroll) {
+    double v[kUnroll];
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) v[j] = p[(i + j) * stride];
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) k += v[j];
+  }
+  if (i < count) {
+    double v[kUnroll];  // the rest: loads past the end repeat the last slice and are not added
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) v[j] = p[min(i + j, count - 1) * stride];
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j)
+      if (i + j < count) k += v[j];
+  }
+  return k;
 }
 
 template <int Sum, int Op>
 __global__ __launch_bounds__(Sum == 2 ? kGroupThreads : kEW) void k_finish(FinishArgs f) {
   int64_t e;
   double k;
+  StageIn in;
   if (Sum == 2) {
     const SplitGroup g = f.groups[blockIdx.x];
     if (static_cast<int>(threadIdx.x) >= 6 * (g.t1 - g.t0)) return;
     e = 6 * static_cast<int64_t>(g.t0) + threadIdx.x;
-    const double* p = f.partial + static_cast<size_t>(g.first) * kGroupThreads + threadIdx.x;
-    k = p[0];
-#pragma unroll 8
-    for (int i = 1; i < g.count; ++i) k += p[static_cast<size_t>(i) * kGroupThreads];
+    in = stage_in<Op>(f.op, e);
+    k = sum_slices<kSumUnroll>(f.partial + static_cast<size_t>(g.first) * kGroupThreads + threadIdx.x, kGroupThreads, g.count);
     f.rates[e] = k;
   } else {
     e = static_cast<int64_t>(blockIdx.x) * kEW + threadIdx.x;
     const int64_t total = 6 * static_cast<int64_t>(f.n);
     if (e >= total) return;
+    in = stage_in<Op>(f.op, e);
     if (Sum == 1) {
       k = f.partial[e];
 #pragma unroll 8
@@ -94,7 +144,7 @@ __global__ __launch_bounds__(Sum == 2 ? kGroupThreads : kEW) void k_finish(Finis
     }
   }
   if (!isfinite(k)) *f.flag = 1;  // (host memory: every writer stores the same word)
-  stage_component<Op>(f.op, e, k);
+  stage_component<Op>(f.op, in, e, k);
 }
 
 __global__ __launch_bounds__(kEW) void k_check_finite(
