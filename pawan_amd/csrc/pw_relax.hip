@@ -45,6 +45,7 @@ namespace {
 using pwi::fail;
 
 constexpr int kB = 256;
+constexpr int kExtentBlocks = 64;
 constexpr int kCellBits = 21;  // cell coordinate bits per axis of a key
 constexpr int64_t kCellMax = (int64_t(1) << kCellBits) - 1;
 constexpr uint64_t kNoCell = ~uint64_t(0);
@@ -123,14 +124,16 @@ __global__ void k_split_apply(int n, int64_t first, const int* __restrict__ flag
 
 // ---- merge ----------------------------------------------------------------
 
-// bounding box and largest radius, one block (n is at most 2^31)
-__global__ __launch_bounds__(1024) void k_extent(const double* __restrict__ pos, const double* __restrict__ radius,
-                                                 int n, double* __restrict__ out) {
-  __shared__ double red[7][1024];
+// bounding box and largest radius, a row of seven per block (the host takes
+// the rest; one block of 1,024 threads read 98,304 particles in 67 us, 64 blocks
+// in 9)
+__global__ __launch_bounds__(kB) void k_extent(const double* __restrict__ pos, const double* __restrict__ radius,
+                                               int n, double* __restrict__ out) {
+  __shared__ double red[7][kB];
   double v[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0};
-  for (int i = static_cast<int>(threadIdx.x); i < n; i += 1024) {
+  for (int64_t i = blockIdx.x * kB + threadIdx.x; i < n; i += kExtentBlocks * kB) {
     for (int c = 0; c < 3; ++c) {
-      const double x = pos[3 * static_cast<int64_t>(i) + c];
+      const double x = pos[3 * i + c];
       if (isfinite(x)) {
         v[c] = fmin(v[c], x);
         v[3 + c] = fmax(v[3 + c], x);
@@ -141,14 +144,14 @@ __global__ __launch_bounds__(1024) void k_extent(const double* __restrict__ pos,
   }
   for (int k = 0; k < 7; ++k) red[k][threadIdx.x] = v[k];
   __syncthreads();
-  for (int s = 512; s > 0; s >>= 1) {
+  for (int s = kB / 2; s > 0; s >>= 1) {
     if (static_cast<int>(threadIdx.x) < s)
       for (int k = 0; k < 7; ++k)
         red[k][threadIdx.x] = k < 3 ? fmin(red[k][threadIdx.x], red[k][threadIdx.x + s])
                                     : fmax(red[k][threadIdx.x], red[k][threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x < 7) out[threadIdx.x] = red[threadIdx.x][0];
+  if (threadIdx.x < 7) out[7 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
 struct Grid {
@@ -235,35 +238,35 @@ __device__ __forceinline__ double misalignment(const double* ai, const double* a
 }
 
 // step 1: particles of the age prefix that have a later neighbour they
-// would merge with in the original state
+// would merge with in the original state.  One thread per particle and row of
+// cells (a search is a chain of 17 reads; nine rows of two searches one after
+// another took 81 us for 98,304 particles, this 39); flag is zero before.
 __global__ void k_merge_flags(int n, const int* __restrict__ prefix, Grid g, const uint64_t* __restrict__ keys,
                               const int* __restrict__ sidx, const double* __restrict__ pos,
                               const double* __restrict__ alpha, const double* __restrict__ radius,
                               int* __restrict__ flag) {
-  const int i = blockIdx.x * kB + static_cast<int>(threadIdx.x);
-  if (i >= n) return;
-  int f = 0;
+  const int64_t t = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x;
+  const int i = static_cast<int>(t / 9), r = static_cast<int>(t % 9);
+  if (i >= n || i >= *prefix) return;
   const double* xi = pos + 3 * static_cast<int64_t>(i);
   const double* ai = alpha + 3 * static_cast<int64_t>(i);
-  const double mi = dnrm2_3(ai[0], ai[1], ai[2]);
   int64_t c[3];
-  if (i < *prefix && mi != 0.0 && cell_of(g, xi[0], xi[1], xi[2], c)) {
-    const double ri = radius[i];
-    for (int r = 0; r < 9 && !f; ++r) {
-      uint64_t first, last;
-      if (!cell_row(c, r, &first, &last)) continue;
-      const int lo = bound_of(keys, n, first, false), hi = bound_of(keys, n, last, true);
-      for (int e = lo; e < hi && !f; ++e) {
-        const int j = sidx[e];
-        if (j <= i) continue;
-        const double* aj = alpha + 3 * static_cast<int64_t>(j);
-        const double mj = dnrm2_3(aj[0], aj[1], aj[2]);
-        if (mj == 0.0 || !in_reach(xi, pos + 3 * static_cast<int64_t>(j), ri, radius[j])) continue;
-        if (misalignment(ai, aj, mi, mj) >= 0.0001) f = 1;
-      }
+  uint64_t first, last;
+  if (!cell_of(g, xi[0], xi[1], xi[2], c) || !cell_row(c, r, &first, &last)) return;
+  const double mi = dnrm2_3(ai[0], ai[1], ai[2]);
+  if (mi == 0.0) return;
+  const double ri = radius[i];
+  for (int e = bound_of(keys, n, first, false); e < n && keys[e] <= last; ++e) {
+    const int j = sidx[e];
+    if (j <= i) continue;
+    const double* aj = alpha + 3 * static_cast<int64_t>(j);
+    const double mj = dnrm2_3(aj[0], aj[1], aj[2]);
+    if (mj == 0.0 || !in_reach(xi, pos + 3 * static_cast<int64_t>(j), ri, radius[j])) continue;
+    if (misalignment(ai, aj, mi, mj) >= 0.0001) {
+      flag[i] = 1;  // (any row's thread may store it)
+      return;
     }
   }
-  flag[i] = f;
 }
 
 // ---- groups of flagged particles ------------------------------------------
@@ -320,34 +323,35 @@ __global__ void k_group_keys(const double* __restrict__ pos, const int* __restri
 }
 
 // flagged particle e (in the order of the coarse cells) with those within
-// kLink h in its own cell and in the 13 neighbour cells after it
+// kLink h in its own cell and in the 13 neighbour cells after it; one thread per
+// particle and cell (one per particle: 67 us for 930 of them, this 11)
 __global__ void k_group_link(const double* __restrict__ pos, const int* __restrict__ list,
                              const uint64_t* __restrict__ keys, const int* __restrict__ sidx, int count, Grid g,
                              int* parent) {
-  const int e = blockIdx.x * kB + static_cast<int>(threadIdx.x);
+  const int64_t t = blockIdx.x * static_cast<int64_t>(kB) + threadIdx.x;
+  const int e = static_cast<int>(t / 14);
+  const int q = 13 + static_cast<int>(t % 14);  // the cell itself, then the 13 after it in z, y, x order
   if (e >= count || keys[e] == kNoCell) return;
   const double* x = pos + 3 * static_cast<int64_t>(list[sidx[e]]);
   const double reach = kLink * g.h;
   const uint64_t key = keys[e], mask = static_cast<uint64_t>(kCellMax);
-  const int64_t c[3] = {static_cast<int64_t>(key & mask), static_cast<int64_t>((key >> kCellBits) & mask),
-                        static_cast<int64_t>(key >> (2 * kCellBits))};
-  for (int q = 13; q < 27; ++q) {  // the cell itself, then the 13 after it in z, y, x order
-    const int64_t nx = c[0] + q % 3 - 1, ny = c[1] + (q / 3) % 3 - 1, nz = c[2] + q / 9 - 1;
-    if (nx < 0 || ny < 0 || nz < 0 || nx > kCellMax || ny > kCellMax || nz > kCellMax) continue;
-    int lo, hi;
-    equal_range(keys, count, cell_key(nx, ny, nz), &lo, &hi);
-    if (lo == hi) continue;
-    if (hi - lo > kExactLinks) {
-      // a crowded cell is one group: each of its particles joins the first
-      group_unite(parent, sidx[e], sidx[lo]);
-      continue;
-    }
-    for (int f = lo; f < hi; ++f) {
-      if (q == 13 && f >= e) break;
-      const double* y = pos + 3 * static_cast<int64_t>(list[sidx[f]]);
-      const double dx = x[0] - y[0], dy = x[1] - y[1], dz = x[2] - y[2];
-      if (dx * dx + dy * dy + dz * dz <= reach * reach) group_unite(parent, sidx[e], sidx[f]);
-    }
+  const int64_t nx = static_cast<int64_t>(key & mask) + q % 3 - 1,
+                ny = static_cast<int64_t>((key >> kCellBits) & mask) + (q / 3) % 3 - 1,
+                nz = static_cast<int64_t>(key >> (2 * kCellBits)) + q / 9 - 1;
+  if (nx < 0 || ny < 0 || nz < 0 || nx > kCellMax || ny > kCellMax || nz > kCellMax) return;
+  int lo, hi;
+  equal_range(keys, count, cell_key(nx, ny, nz), &lo, &hi);
+  if (lo == hi) return;
+  if (hi - lo > kExactLinks) {
+    // a crowded cell is one group: each of its particles joins the first
+    group_unite(parent, sidx[e], sidx[lo]);
+    return;
+  }
+  for (int f = lo; f < hi; ++f) {
+    if (q == 13 && f >= e) break;
+    const double* y = pos + 3 * static_cast<int64_t>(list[sidx[f]]);
+    const double dx = x[0] - y[0], dy = x[1] - y[1], dz = x[2] - y[2];
+    if (dx * dx + dy * dy + dz * dz <= reach * reach) group_unite(parent, sidx[e], sidx[f]);
   }
 }
 
@@ -376,7 +380,7 @@ __device__ __forceinline__ int wave_min_int(int v) {
 // A replay is a chain of dependent memory reads, so it is bound by latency:
 // one block over all flagged particles took 9.2 ms for a 98,304-particle wake
 // with one particle in 200 turned; by groups the same replay takes 0.09 ms,
-// the linking 0.06.
+// the linking 0.01.
 __global__ __launch_bounds__(kRT) void k_merge_resolve(int n, const int* __restrict__ list,
                                                        const int* __restrict__ root, int count, Grid g,
                                                        const uint64_t* __restrict__ keys,
@@ -678,7 +682,7 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   b.add(&d_rad, nn);
   b.add(&d_vol, nn);
   b.add(&d_act, nn);
-  b.add(&d_ext, 7);
+  b.add(&d_ext, 7 * kExtentBlocks);
   b.add(&d_prefix, 1);
   b.add(&d_flag, nn);
   b.add(&d_idx, nn);
@@ -697,11 +701,12 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   RX_HIP(up(d_vol, volume, nn, b.st));
   RX_HIP(up(d_act, active, nn, b.st));
   // the cell size: the largest merge distance, with room for rounding
-  hipLaunchKernelGGL(k_extent, dim3(1), dim3(1024), 0, b.st, d_pos, d_rad, ni, d_ext);
+  hipLaunchKernelGGL(k_extent, dim3(kExtentBlocks), dim3(kB), 0, b.st, d_pos, d_rad, ni, d_ext);
   RX_HIP(hipGetLastError());
-  double ext[7];
-  RX_HIP(down(ext, d_ext, 7, b.st));
+  double ext[7 * kExtentBlocks];
+  RX_HIP(down(ext, d_ext, 7 * kExtentBlocks, b.st));
   RX_HIP(hipStreamSynchronize(b.st));
+  for (int k = 7; k < 7 * kExtentBlocks; ++k) ext[k % 7] = k % 7 < 3 ? std::min(ext[k % 7], ext[k]) : std::max(ext[k % 7], ext[k]);
   if (!(ext[6] > 0.0)) return PW_OK;  // no radius: nothing is within reach
   Grid g;
   g.x0 = std::isfinite(ext[0]) ? ext[0] : 0.0;
@@ -718,7 +723,9 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   hipLaunchKernelGGL(k_cell_keys, grid, dim3(kB), 0, b.st, d_pos, ni, g, d_key, d_idx);
   RX_HIP(hipGetLastError());
   RX_HIP(hipcub::DeviceRadixSort::SortPairs(d_temp, t1, d_key, d_skey, d_idx, d_sidx, ni, 0, 64, b.st));
-  hipLaunchKernelGGL(k_merge_flags, grid, dim3(kB), 0, b.st, ni, d_prefix, g, d_skey, d_sidx, d_pos, d_alpha, d_rad,
+  RX_HIP(pw::launch_fill_int(d_flag, ni, 0, b.st));
+  const dim3 rgrid(static_cast<unsigned>((9 * static_cast<int64_t>(ni) + kB - 1) / kB));
+  hipLaunchKernelGGL(k_merge_flags, rgrid, dim3(kB), 0, b.st, ni, d_prefix, g, d_skey, d_sidx, d_pos, d_alpha, d_rad,
                      d_flag);
   RX_HIP(hipGetLastError());
   // the flagged particles in ascending order (the sort left d_idx = 0..n-1)
@@ -748,7 +755,7 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   RX_HIP(hipGetLastError());
   // (d_flag and d_slist are free: indices before and after the sort)
   RX_HIP(hipcub::DeviceRadixSort::SortPairs(d_temp2, t4, d_gkey, d_sgkey, d_flag, d_slist, count, 0, 64, b.st));
-  hipLaunchKernelGGL(k_group_link, lgrid, dim3(kB), 0, b.st, d_pos, d_list, d_sgkey, d_slist, count, g, d_parent);
+  hipLaunchKernelGGL(k_group_link, dim3(static_cast<unsigned>((14 * static_cast<int64_t>(count) + kB - 1) / kB)), dim3(kB), 0, b.st, d_pos, d_list, d_sgkey, d_slist, count, g, d_parent);
   RX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_group_roots, lgrid, dim3(kB), 0, b.st, count, d_parent, d_root);
   RX_HIP(hipGetLastError());
