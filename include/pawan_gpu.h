@@ -165,6 +165,10 @@ int pw_set_wake_state(pw_ctx *ctx, int wake, const double *pos,
 int pw_set_wake_volume(pw_ctx *ctx, int wake, const double *volume);
 int pw_get_wake_state(pw_ctx *ctx, int wake, double *pos, double *alpha);
 int pw_get_wake_rates(pw_ctx *ctx, int wake, double *vel, double *retvor);
+/* The same rows of every wake, one wake after the other (N x 3 each, N the
+ * particles of all wakes; either may be null). */
+int pw_get_all_state(pw_ctx *ctx, double *pos, double *alpha);
+int pw_get_all_rates(pw_ctx *ctx, double *vel, double *retvor);
 
 /* Whole-system state / rate vectors in the reference layout: wakes
  * concatenated, wake w occupying 6*maxn_w doubles [pos ; alpha] or

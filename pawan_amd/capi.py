@@ -29,7 +29,8 @@ SCHEMES = {"euler": PW_EULER, "rk3": PW_RK3, "rk4": PW_RK4}
 EXPORTS = [
     "pw_version", "pw_last_error", "pw_device_count", "pw_create", "pw_destroy",
     "pw_add_wake", "pw_set_nu", "pw_get_nu", "pw_set_coupled", "pw_get_size",
-    "pw_set_wake_state", "pw_get_wake_state", "pw_get_wake_rates", "pw_set_states",
+    "pw_set_wake_state", "pw_get_wake_state", "pw_get_wake_rates", "pw_get_all_state",
+    "pw_get_all_rates", "pw_set_states",
     "pw_get_states", "pw_get_rates", "pw_solve", "pw_step", "pw_diagnose",
     "pw_synchronize", "pw_set_profiling", "pw_get_pair_timing",
     "pw_set_pair_config", "pw_get_pair_config", "pw_autotune", "pw_set_graph",
@@ -99,6 +100,8 @@ def load(path: str | None = None) -> C.CDLL:
         "pw_set_wake_volume": ([vp, i, _dp], i),
         "pw_get_wake_state": ([vp, i, _dp, _dp], i),
         "pw_get_wake_rates": ([vp, i, _dp, _dp], i),
+        "pw_get_all_state": ([vp, _dp, _dp], i),
+        "pw_get_all_rates": ([vp, _dp, _dp], i),
         "pw_set_states": ([vp, _dp, i64], i),
         "pw_get_states": ([vp, _dp, i64], i),
         "pw_get_rates": ([vp, _dp, i64], i),
@@ -300,21 +303,18 @@ class Solver:
         return vel, ret
 
     def _all_wakes(self, get):
-        """Two N x 3 arrays, wake after wake, filled by get(ctx, wake, a, b)."""
+        """Two N x 3 arrays, wake after wake, filled by get(ctx, a, b)."""
         first, second = np.empty((self.n, 3)), np.empty((self.n, 3))
-        at = 0
-        for w, n in enumerate(self.wake_sizes):
-            _check(get(self._h, w, first[at:at + n], second[at:at + n]))
-            at += n
+        _check(get(self._h, first, second))
         return first, second
 
     def state(self):
         """(pos, alpha) of all particles, wakes concatenated."""
-        return self._all_wakes(self._lib.pw_get_wake_state)
+        return self._all_wakes(self._lib.pw_get_all_state)
 
     def rates(self):
         """(vel, retvor) of all particles from the last right-hand side."""
-        return self._all_wakes(self._lib.pw_get_wake_rates)
+        return self._all_wakes(self._lib.pw_get_all_rates)
 
     def set_states(self, state: np.ndarray) -> None:
         state = np.ascontiguousarray(state, dtype=np.float64)
