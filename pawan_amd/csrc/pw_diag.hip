@@ -152,7 +152,7 @@ __device__ __forceinline__ void diag_pair(const Rec64& me, const Rec64& s, const
 //
 // The ordered pairs of 94 blocks, each with an exp, an erf, two square roots
 // and seven divisions, took 18.7 ms for 24,000 particles; unordered, split
-// over 9,000 blocks and with the divisions taken out (about 60 instructions a
+// over 4,600 blocks and with the divisions taken out (about 60 instructions a
 // pair, the core from pw_core64.h) FP64 issue bounds it.
 template <bool HighOrder>
 __global__ __launch_bounds__(kTB) void k_diag_pairs(
