@@ -56,48 +56,45 @@ __device__ __forceinline__ v4f mfma(float a, float b, v4f c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// acc[t] += in (16 x 128, LDS) times B, for the wave's two column tiles;
-// b(t, s) loads this lane's B value of step s
-template <typename LoadB>
-__device__ __forceinline__ void product128(const float (*in)[kLd], LoadB b, v4f (&acc)[2]) {
-  const int lane = static_cast<int>(threadIdx.x) & 63, c = lane & 15, g = lane >> 4;
+// This lane's 64 B values of a 128-long product, for the wave's two column
+// tiles: value s of tile t.  Loaded a product ahead of their use, so that a
+// wave, alone on its SIMD, does not wait for them (registers are there: 512).
+struct Weights {
+  float v[2][32];
+};
+
+// W[k][j] row-major 128 x 128: columns j of the forward product;
+// w = W + 32 wave + c + 128 * 32 g
+__device__ __forceinline__ void load_forward(const float* __restrict__ w, Weights& b) {
 #pragma unroll
-  for (int s0 = 0; s0 < 32; s0 += 16) {
-    // 32 weights and 16 inputs in flight: one wave per SIMD has only these
-    // loads to hide their latency behind
-    float w[2][16];
+  for (int s = 0; s < 32; ++s)
 #pragma unroll
-    for (int t = 0; t < 2; ++t) b(t, s0, w[t]);
-    v4f a[4];
+    for (int t = 0; t < 2; ++t) b.v[t][s] = w[H * s + 16 * t];
+}
+// the transposed product: column n of W^T is row n of W;
+// w = W + 128 (32 wave + c) + 32 g
+__device__ __forceinline__ void load_backward(const float* __restrict__ w, Weights& b) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = *reinterpret_cast<const v4f*>(&in[c][32 * g + s0 + 4 * q]);
+  for (int q = 0; q < 8; ++q)
 #pragma unroll
-    for (int s = 0; s < 16; ++s)
+    for (int t = 0; t < 2; ++t) {
+      const v4f x = *reinterpret_cast<const v4f*>(w + 16 * H * t + 4 * q);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) acc[t] = mfma(a[s >> 2][s & 3], w[t][s], acc[t]);
-  }
+      for (int i = 0; i < 4; ++i) b.v[t][4 * q + i] = x[i];
+    }
 }
 
-// W[k][j] row-major 128 x 128: columns j of the forward product
-struct ForwardB {
-  const float* w;  // W + 32 wave + c + 128 * 32 g
-  __device__ __forceinline__ void operator()(int t, int s0, float (&v)[16]) const {
+// acc[t] += in (16 x 128, LDS) times B, for the wave's two column tiles
+__device__ __forceinline__ void product128(const float (*in)[kLd], const Weights& b, v4f (&acc)[2]) {
+  const int lane = static_cast<int>(threadIdx.x) & 63, c = lane & 15, g = lane >> 4;
+  v4f a[8];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) v[s] = w[H * (s0 + s) + 16 * t];
-  }
-};
-// the transposed product: column n of W^T is row n of W
-struct BackwardB {
-  const float* w;  // W + 128 (32 wave + c) + 32 g
-  __device__ __forceinline__ void operator()(int t, int s0, float (&v)[16]) const {
+  for (int q = 0; q < 8; ++q) a[q] = *reinterpret_cast<const v4f*>(&in[c][32 * g + 4 * q]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const v4f x = *reinterpret_cast<const v4f*>(w + 16 * H * t + s0 + 4 * q);
+  for (int s = 0; s < 32; ++s)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[4 * q + i] = x[i];
-    }
-  }
-};
+    for (int t = 0; t < 2; ++t) acc[t] = mfma(a[s >> 2][s & 3], b.v[t][s], acc[t]);
+}
 
 // acc[a][b] += in^T d over the tile's 16 samples: rows 16 (NA wave + a) of the
 // weights, columns 16 b
@@ -132,7 +129,10 @@ __device__ __forceinline__ void store_tiles(const v4f (&a)[2], float (*out)[kLd]
 // Each wave owns 32 of the 128 units: forward and backward products write its
 // columns, so its pre-activations stay in its registers for gelu'; activations
 // and deltas pass to the other waves through LDS.  Weights are read straight
-// from memory, each by the one wave that uses it.
+// from memory, each by the one wave that uses it, a phase ahead of their use:
+// the block is nine phases between barriers, and with the loads inside them each
+// waited for memory (42.6 us a batch of 4,096, now 32.3, of which the matrix
+// cores work 6 and the partial rows take about 9 to write).
 //
 // The products were FP32 vector instructions fed one LDS read each, over 32
 // samples per block: 144 us for a batch of 4,096 on 128 CUs (164 us a training
@@ -154,12 +154,12 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ para
     // hoisting 147 KB of loads out of the loop into (spilled) registers
     const float* P = params;
     asm volatile("" : "+s"(P));
-    // inputs (rows beyond n are zero and carry zero error)
-    {
-      const int r = tid >> 4, k = tid & 15;
-      s.x[r][k] = row0 + r < n ? X[sample(row0 + r) * kMlpIn + k] : 0.0f;
-    }
-    __syncthreads();
+    // what the first phases read, in flight together: inputs (rows beyond n are
+    // zero and carry zero error), biases, first and second layer
+    const int er = tid >> 4, ej = tid & 15;  // this thread's input, and its output's error
+    const bool has = row0 + er < n;
+    const size_t at = sample(has ? row0 + er : row0);
+    const float xin = X[at * kMlpIn + ej];
     v4f a1[2], a2[2], a3[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -170,38 +170,54 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ para
         a3[t][r] = P[kOffB3 + col + 16 * t];
       }
     static_assert(kMlpIn == 16 && R == 16, "one 16x16 tile of inputs");
+    float w1[4][2];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) a1[t] = mfma(s.x[c][4 * q + g], P[kOffW1 + H * (4 * q + g) + col + 16 * t], a1[t]);
+      for (int t = 0; t < 2; ++t) w1[q][t] = P[kOffW1 + H * (4 * q + g) + col + 16 * t];
+    Weights wa, wb;
+    load_forward(P + kOffW2 + 32 * H * g + col, wa);
+    s.x[er][ej] = has ? xin : 0.0f;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) a1[t] = mfma(s.x[c][4 * q + g], w1[q][t], a1[t]);
     const auto act = [](float v, int, int) { return gelu_f(v); };
     store_tiles(a1, s.h1, act);
+    load_forward(P + kOffW3 + 32 * H * g + col, wb);
     __syncthreads();
-    product128(s.h1, ForwardB{P + kOffW2 + 32 * H * g + col}, a2);
+    product128(s.h1, wa, a2);
     store_tiles(a2, s.h2, act);
+    load_backward(P + kOffW3 + H * col + 32 * g, wa);
+    // the output layer's weights both ways, its bias and the target
+    float w4[8], w4t[3][2];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) w4[q] = c < kMlpOut ? P[kOffW4 + (32 * wave + 4 * q + g) * kMlpOut + c] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) w4t[q][t] = P[kOffW4 + (col + 16 * t) * kMlpOut + 4 * q + g];
+    const bool out_on = ej < kMlpOut && has;
+    const float b4 = out_on ? P[kOffB4 + ej] : 0.0f, target = out_on ? Y[at * kMlpOut + ej] : 0.0f;
     __syncthreads();
-    product128(s.h2, ForwardB{P + kOffW3 + 32 * H * g + col}, a3);
+    product128(s.h2, wb, a3);
     store_tiles(a3, s.h3, act);
     __syncthreads();
     // output layer: 12 columns of one tile, a K quarter per wave
     {
       v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int k = 32 * wave + 4 * q + g;
-        acc = mfma(s.h3[c][k], c < kMlpOut ? P[kOffW4 + k * kMlpOut + c] : 0.0f, acc);
-      }
+      for (int q = 0; q < 8; ++q) acc = mfma(s.h3[c][32 * wave + 4 * q + g], w4[q], acc);
 #pragma unroll
       for (int r = 0; r < 4; ++r) s.part[wave][4 * g + r][c] = acc[r];
     }
     __syncthreads();
     {
-      const int r = tid >> 4, j = tid & 15;
       float err = 0.0f;
-      if (j < kMlpOut && row0 + r < n)
-        err = (((s.part[0][r][j] + s.part[1][r][j]) + (s.part[2][r][j] + s.part[3][r][j])) + P[kOffB4 + j]) -
-              Y[sample(row0 + r) * kMlpOut + j];
-      s.o[r][j] = 2.0f * err;
+      if (out_on)
+        err = (((s.part[0][er][ej] + s.part[1][er][ej]) + (s.part[2][er][ej] + s.part[3][er][ej])) + b4) - target;
+      s.o[er][ej] = 2.0f * err;
       lsum = fmaf(err, err, lsum);
     }
     __syncthreads();
@@ -211,7 +227,8 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ para
     for (int q = 0; q < 3; ++q)
 #pragma unroll
       for (int t = 0; t < 2; ++t)
-        d[t] = mfma(s.o[c][4 * q + g], P[kOffW4 + (col + 16 * t) * kMlpOut + 4 * q + g], d[t]);
+        d[t] = mfma(s.o[c][4 * q + g], w4t[q][t], d[t]);
+    load_backward(P + kOffW2 + H * col + 32 * g, wb);
     store_tiles(d, s.d[0], [&](float v, int t, int r) { return v * gelu_d(a3[t][r]); });
     wgrad<2, 1>(s.h3, 32 * wave, s.o, 0, g4);
     if (tid < kMlpOut)
@@ -219,7 +236,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ para
     __syncthreads();
     // delta2, and the third layer's gradient
     d[0] = d[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    product128(s.d[0], BackwardB{P + kOffW3 + H * col + 32 * g}, d);
+    product128(s.d[0], wa, d);
     store_tiles(d, s.d[1], [&](float v, int t, int r) { return v * gelu_d(a2[t][r]); });
     wgrad<2, 8>(s.h2, 32 * wave, s.d[0], 0, g3);
     if (tid < H)
@@ -227,7 +244,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float* __restrict__ para
     __syncthreads();
     // delta1, and the second layer's
     d[0] = d[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    product128(s.d[1], BackwardB{P + kOffW2 + H * col + 32 * g}, d);
+    product128(s.d[1], wb, d);
     store_tiles(d, s.d[0], [&](float v, int t, int r) { return v * gelu_d(a1[t][r]); });
     wgrad<2, 8>(s.h1, 32 * wave, s.d[1], 0, g2);
     if (tid < H)
@@ -313,7 +330,7 @@ uint64_t splitmix(uint64_t& s) {
 
 }  // namespace
 
-// One block per tile up to one per CU (302 registers: one wave per SIMD), then
+// One block per tile up to one per CU (413 registers: one wave per SIMD), then
 // several tiles per block: the partial rows, 147 KB each, stay below 38 MB.
 int train_blocks(int n) {
   const int tiles = (n + R - 1) / R;
