@@ -431,13 +431,18 @@ __device__ __forceinline__ void item_fp64(const PairArgs& pa, const WorkItem& it
 // adds them factored, A += q a_s, C += c a_s, D += c V_s, and the item ends
 // with w = a_t x A + B + V_t C - D a_t.
 // ---------------------------------------------------------------------
-constexpr double kHoF = -0x1.e8ec8a4aeacc4p-4;   // -3/(8 pi)
-constexpr double kHoEta = 0x1.0b615ba0f867bp+2;  // 105/(8 pi)
+// All sums carry 4 pi, B also -1/3: q' = 4 pi q, F = -(3/4pi) f with f = (rho^2 +
+// 7/2 sigma^2) b^-7/2, and 4 pi x 2 nu eta / sigma^2 = 105 nu sigma^4 b^-9/2 (nu2
+// holds 105 nu); the results are scaled once.  That is 52 vector instructions a
+// factored pair, 55 with the constants in it (per right-hand side: two rings of
+// 4,816 61.2 -> 60.3 us, of 16,000 516 -> 505).
+constexpr double kHoNu = 105.0;
+constexpr double kThird = 1.0 / 3.0;
 
 struct AccHO {
   double ux = 0, uy = 0, uz = 0;  // sum q v
   double ax = 0, ay = 0, az = 0;  // A = sum q a_s (factored sources)
-  double bx = 0, by = 0, bz = 0;  // B
+  double bx = 0, by = 0, bz = 0;  // -B/3
   double cx = 0, cy = 0, cz = 0;  // C = sum c a_s (factored sources)
   double d = 0;                   // D = sum c V_s (factored sources)
 };
@@ -450,20 +455,21 @@ __device__ __forceinline__ void pair64_ho(const T64& t, const Rec64& s, AccHO& a
   const double ib2 = ib * ib;
   const double ib5 = ib2 * ib2 * ib;
   const double ib7 = ib5 * ib2;
-  const double q = kQ * fma(2.5, sig2, r2) * ib5;
-  const double F = kHoF * fma(7.0, sig2, 2.0 * r2) * ib7;
-  const double c = t.nu2 * kHoEta * (sig2 * sig2) * (ib7 * ib2);  // 2 nu eta / sigma^2
+  const double q = fma(2.5, sig2, r2) * ib5;
+  const double f = fma(3.5, sig2, r2) * ib7;
+  const double c = t.nu2 * (sig2 * sig2) * (ib7 * ib2);
   const double vx = s.ay * dz - s.az * dy;
   const double vy = s.az * dx - s.ax * dz;
   const double vz = s.ax * dy - s.ay * dx;
   a.ux += q * vx;
   a.uy += q * vy;
   a.uz += q * vz;
-  const double fr = F * (t.ax * vx + t.ay * vy + t.az * vz);
+  const double fr = f * (t.ax * vx + t.ay * vy + t.az * vz);
   if (__ballot(r2 <= kFar64 * sig2)) {
-    a.bx += q * (t.ay * s.az - t.az * s.ay) + fr * dx + c * (t.vol * s.ax - s.vol * t.ax);
-    a.by += q * (t.az * s.ax - t.ax * s.az) + fr * dy + c * (t.vol * s.ay - s.vol * t.ay);
-    a.bz += q * (t.ax * s.ay - t.ay * s.ax) + fr * dz + c * (t.vol * s.az - s.vol * t.az);
+    const double q3 = -kThird * q, c3 = -kThird * c;
+    a.bx += q3 * (t.ay * s.az - t.az * s.ay) + fr * dx + c3 * (t.vol * s.ax - s.vol * t.ax);
+    a.by += q3 * (t.az * s.ax - t.ax * s.az) + fr * dy + c3 * (t.vol * s.ay - s.vol * t.ay);
+    a.bz += q3 * (t.ax * s.ay - t.ay * s.ax) + fr * dz + c3 * (t.vol * s.az - s.vol * t.az);
   } else {
     a.ax += q * s.ax;
     a.ay += q * s.ay;
@@ -486,7 +492,7 @@ __device__ __forceinline__ void item_fp64_ho(const PairArgs& pa, const WorkItem&
   T64 me;
   me.x = m.x; me.y = m.y; me.z = m.z; me.hs2 = 0.5 * m.s2;
   me.ax = m.ax; me.ay = m.ay; me.az = m.az; me.vol = m.vol;
-  me.nu2 = 2.0 * pa.nu;
+  me.nu2 = kHoNu * pa.nu;
   AccHO a;
   for (int base = it.s0; base < it.s1; base += kTB) {
     const int cnt = min(kTB, it.s1 - base);
@@ -504,10 +510,12 @@ __device__ __forceinline__ void item_fp64_ho(const PairArgs& pa, const WorkItem&
   }
   if (active) {
     Rate64 r;
-    r.ux = a.ux; r.uy = a.uy; r.uz = a.uz;
-    r.wx = ((me.ay * a.az - me.az * a.ay) + a.bx) + (me.vol * a.cx - a.d * me.ax);
-    r.wy = ((me.az * a.ax - me.ax * a.az) + a.by) + (me.vol * a.cy - a.d * me.ay);
-    r.wz = ((me.ax * a.ay - me.ay * a.ax) + a.bz) + (me.vol * a.cz - a.d * me.az);
+    r.ux = kQ * a.ux;
+    r.uy = kQ * a.uy;
+    r.uz = kQ * a.uz;
+    r.wx = kQ * (((me.ay * a.az - me.az * a.ay) - 3.0 * a.bx) + (me.vol * a.cx - a.d * me.ax));
+    r.wy = kQ * (((me.az * a.ax - me.ax * a.az) - 3.0 * a.by) + (me.vol * a.cy - a.d * me.ay));
+    r.wz = kQ * (((me.ax * a.ay - me.ay * a.ax) - 3.0 * a.bz) + (me.vol * a.cz - a.d * me.az));
     out_rates(pa, it)[t] = r;
   }
 }
@@ -2288,22 +2296,22 @@ template <>
 struct SplitSum<kPairFP64HO> {
   using Src = Rec64;
   static constexpr bool kTable = false;
+  static constexpr bool kMix = false;
   T64 me;
   AccHO a;
   __device__ __forceinline__ void init(const Rec64& m, double nu) {
     me.x = m.x; me.y = m.y; me.z = m.z; me.hs2 = 0.5 * m.s2;
     me.ax = m.ax; me.ay = m.ay; me.az = m.az; me.vol = m.vol;
-    me.nu2 = 2.0 * nu;
+    me.nu2 = kHoNu * nu;
   }
   static __device__ __forceinline__ Src source(const Rec64& r) { return r; }
-  static constexpr bool kMix = false;
   __device__ __forceinline__ void pair(const Src& s, const double* __restrict__) { pair64_ho(me, s, a); }
   __device__ __forceinline__ void chunk_end() {}
   __device__ __forceinline__ void result(double (&r)[6]) const {
-    r[0] = a.ux; r[1] = a.uy; r[2] = a.uz;
-    r[3] = ((me.ay * a.az - me.az * a.ay) + a.bx) + (me.vol * a.cx - a.d * me.ax);
-    r[4] = ((me.az * a.ax - me.ax * a.az) + a.by) + (me.vol * a.cy - a.d * me.ay);
-    r[5] = ((me.ax * a.ay - me.ay * a.ax) + a.bz) + (me.vol * a.cz - a.d * me.az);
+    r[0] = kQ * a.ux; r[1] = kQ * a.uy; r[2] = kQ * a.uz;
+    r[3] = kQ * (((me.ay * a.az - me.az * a.ay) - 3.0 * a.bx) + (me.vol * a.cx - a.d * me.ax));
+    r[4] = kQ * (((me.az * a.ax - me.ax * a.az) - 3.0 * a.by) + (me.vol * a.cy - a.d * me.ay));
+    r[5] = kQ * (((me.ax * a.ay - me.ay * a.ax) - 3.0 * a.bz) + (me.vol * a.cz - a.d * me.az));
   }
 };
 
