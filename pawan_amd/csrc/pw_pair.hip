@@ -1989,8 +1989,10 @@ __device__ __forceinline__ void near_slice(const NearArgs& a, const NearItem& it
         f.pad = 0.0f;
         // beyond the core of every target by itself
         const float ex = f.rx - sx, ey = f.ry - sy, ez = f.rz - sz;
-        const float g = sqrtf(fmaf(ez, ez, fmaf(ey, ey, ex * ex))) - sr;
-        clear = sep || (g > 0.0f && g * g > a.gap2 * 1.0001f);
+        // (by more than the rounding of the positions, also where the radii are
+        // below it: a slice's own particles are never clear)
+        const float d = sqrtf(fmaf(ez, ez, fmaf(ey, ey, ex * ex))), g = d - sr;
+        clear = sep || (g > 1e-5f * (d + tr) && g * g > a.gap2 * 1.0001f);
       }
       uint64_t far = __ballot(clear);
       if (__popcll(far) < kClearMin && !sep) far = 0;

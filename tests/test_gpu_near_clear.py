@@ -40,3 +40,20 @@ def test_near_field_alone(name, kernel):
     eu, ew = normwise(u, ru), normwise(w, rw)
     print(f"{name} kernel {kernel}: {eu:.2e} {ew:.2e}", flush=True)
     assert eu < 1e-6 and ew < 1e-5
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+def test_radii_below_the_rounding_of_positions(uniform):
+    """A slice's own particles lie on its bounding sphere up to rounding and are
+    not to be taken for clear ones, however small the core: each would meet
+    itself.  FP32 positions relative to a leaf of radius 0.5 leave the nearest
+    pairs, 0.005 apart, 1e-5 of their displacement."""
+    s = SYSTEMS["rings"]()
+    s.radius[:] = 1e-9 if uniform else np.linspace(1e-9, 2e-9, s.n)
+    with capi.Solver(s) as g:
+        g.set_pair_config("fp64", 2)
+        ru, rw = g.solve("fp64")
+        g.ff_set_params(1e-6, 0.0, use_mlp=False)
+        u, w = g.solve("learned")
+    assert np.isfinite(u).all() and np.isfinite(w).all()
+    assert normwise(u, ru) < 1e-4 and normwise(w, rw) < 1e-3
