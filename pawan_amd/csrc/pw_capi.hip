@@ -450,7 +450,8 @@ int ensure_kind(pw_ctx* c, int kind) {
     // the scalar-fed FP64 kernel's source records, allocated before any
     // step is captured (no allocation may happen inside a capture)
     int rc = PW_OK;
-    if ((k.run.scalar_feed || k.run.split_sep) && kind == pw::kPairFP64 && !c->d_src64 && dalloc(&c->d_src64, c->n) != hipSuccess) {
+    if ((k.run.scalar_feed || k.run.split_sep) && kind == pw::kPairFP64 && !c->d_src64 &&
+        dalloc(&c->d_src64, c->n) != hipSuccess) {
       (void)hipGetLastError();
       rc = fail(PW_ERR_NOMEM, "scalar-fed FP64 source records");
     }
@@ -585,7 +586,8 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp&
   args.nchunks = c->nchunks;
   // the high-order kernel replaces the Gaussian kinds (pw_set_kernel)
   const int launch_kind = launch_kind_of(c, kind);
-  if ((k.run.scalar_feed || k.run.split_sep) && launch_kind == pw::kPairFP64) args.src64 = c->d_src64;  // ensure_kind made it
+  if ((k.run.scalar_feed || k.run.split_sep) && launch_kind == pw::kPairFP64)
+    args.src64 = c->d_src64;  // ensure_kind made it
   const int grid = c->num_cus * pw::pair_kernel_waves(launch_kind, k.run);
   pw::SumForm sum;
   sum.partial = c->partial;
@@ -765,7 +767,8 @@ int write_particles(pw_ctx* c, int64_t first, int64_t count, const double* x, co
 // split of up to kPointBlocks blocks, however few particles there are)
 hipError_t point_velocity(pw_ctx* c, const double* d_pts, int m, double* d_u) {
   return pw::launch_point_velocity(c->y, static_cast<int>(c->n), d_pts, m, d_u, reinterpret_cast<double*>(c->k[1]),
-                                   6 * std::max(static_cast<size_t>(c->n), pw::kPointScratchRows), c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
+                                   6 * std::max(static_cast<size_t>(c->n), pw::kPointScratchRows),
+                                   c->smoothing == PW_KERNEL_HIGHORDER, c->stream);
 }
 
 }  // namespace

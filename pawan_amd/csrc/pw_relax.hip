@@ -706,7 +706,8 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   double ext[7 * kExtentBlocks];
   RX_HIP(down(ext, d_ext, 7 * kExtentBlocks, b.st));
   RX_HIP(hipStreamSynchronize(b.st));
-  for (int k = 7; k < 7 * kExtentBlocks; ++k) ext[k % 7] = k % 7 < 3 ? std::min(ext[k % 7], ext[k]) : std::max(ext[k % 7], ext[k]);
+  for (int k = 7; k < 7 * kExtentBlocks; ++k)
+    ext[k % 7] = k % 7 < 3 ? std::min(ext[k % 7], ext[k]) : std::max(ext[k % 7], ext[k]);
   if (!(ext[6] > 0.0)) return PW_OK;  // no radius: nothing is within reach
   Grid g;
   g.x0 = std::isfinite(ext[0]) ? ext[0] : 0.0;
@@ -755,7 +756,8 @@ int pw_wake_merge(int device, double stepnum, int64_t num_particles, double* pos
   RX_HIP(hipGetLastError());
   // (d_flag and d_slist are free: indices before and after the sort)
   RX_HIP(hipcub::DeviceRadixSort::SortPairs(d_temp2, t4, d_gkey, d_sgkey, d_flag, d_slist, count, 0, 64, b.st));
-  hipLaunchKernelGGL(k_group_link, dim3(static_cast<unsigned>((14 * static_cast<int64_t>(count) + kB - 1) / kB)), dim3(kB), 0, b.st, d_pos, d_list, d_sgkey, d_slist, count, g, d_parent);
+  const dim3 cgrid(static_cast<unsigned>((14 * static_cast<int64_t>(count) + kB - 1) / kB));
+  hipLaunchKernelGGL(k_group_link, cgrid, dim3(kB), 0, b.st, d_pos, d_list, d_sgkey, d_slist, count, g, d_parent);
   RX_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_group_roots, lgrid, dim3(kB), 0, b.st, count, d_parent, d_root);
   RX_HIP(hipGetLastError());
