@@ -1907,8 +1907,8 @@ __device__ __forceinline__ void pair32_rel_core(float tx, float ty, float tz, co
 // the instructions it saved.  The kernel is bound by its vector instructions
 // (1.51 per cycle and CU, 46 a pair) with its LDS 76% busy.  Lists, nodes and
 // chunks are read through the constant address space: scalar loads, and the
-// registers their copies took.  1M helix, solve 41.1 -> 38.0 ms; 300,032 with the
-// network 18.8 -> 17.5.
+// registers their copies took.  1M helix, solve 41.1 -> 38.5 ms; 300,032 with the
+// network 18.8 -> 17.7.
 //
 // Halves: the slice holds at most 32 targets; lanes 32-63 take the same
 // targets as lanes 0-31 and each half every other source of a tile, and
