@@ -124,6 +124,7 @@ void free_buffers(pw_ctx* c) {
     k.d_groups = nullptr;
     k.nitems = k.ngroups = 0;
     k.built_parts = k.built_split = 0;
+    k.rows = 0;
     k.lean = false;
   }
   c->partial = nullptr;
@@ -397,6 +398,9 @@ pw::PairConfig auto_config(const pw_ctx* c, int launch_kind) {
   return p;
 }
 
+// The buffer is shared by all kinds and freed before a larger one is tried (both
+// need not fit at once): when that fails there is none, and a kind built earlier
+// is built again before its next launch (ensure_kind compares its rows).
 int ensure_partial(pw_ctx* c, size_t rows) {
   if (rows <= c->partial_rows) return PW_OK;
   (void)hipFree(c->partial);
@@ -424,6 +428,7 @@ int build_kind(pw_ctx* c, int kind, const pw::PairConfig& cfg) {
   k.d_items = nullptr;
   k.d_groups = nullptr;
   k.built_parts = k.built_split = 0;
+  k.rows = 0;
   if (dalloc(&k.d_items, items.size()) != hipSuccess ||
       (!groups.empty() && dalloc(&k.d_groups, groups.size()) != hipSuccess)) {
     (void)hipGetLastError();
@@ -432,8 +437,10 @@ int build_kind(pw_ctx* c, int kind, const pw::PairConfig& cfg) {
   PW_HIP(hipMemcpy(k.d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
   if (!groups.empty())
     PW_HIP(hipMemcpy(k.d_groups, groups.data(), groups.size() * sizeof(pw::SplitGroup), hipMemcpyHostToDevice));
-  if (cfg.split > 0) PW_TRY(ensure_partial(c, 64 * items.size()));
-  else if (cfg.parts > 1) PW_TRY(ensure_partial(c, static_cast<size_t>(cfg.parts) * c->n));
+  const size_t rows =
+      cfg.split > 0 ? 64 * items.size() : cfg.parts > 1 ? static_cast<size_t>(cfg.parts) * static_cast<size_t>(c->n) : 0;
+  PW_TRY(ensure_partial(c, rows));
+  k.rows = rows;
   k.nitems = static_cast<int>(items.size());
   k.ngroups = static_cast<int>(groups.size());
   k.built_parts = cfg.parts;
@@ -455,7 +462,10 @@ int ensure_kind(pw_ctx* c, int kind) {
       (void)hipGetLastError();
       rc = fail(PW_ERR_NOMEM, "scalar-fed FP64 source records");
     }
-    if (rc == PW_OK && k.d_items && k.built_parts == k.run.parts && k.built_split == k.run.split) return PW_OK;
+    // (the rows too: another kind's larger buffer may have replaced them by none)
+    if (rc == PW_OK && k.d_items && k.built_parts == k.run.parts && k.built_split == k.run.split &&
+        c->partial_rows >= k.rows)
+      return PW_OK;
     if (rc == PW_OK) rc = build_kind(c, kind, k.run);
     // a launch chosen here that does not fit in memory: the one that needs none
     if (rc != PW_ERR_NOMEM || !chosen || is_default(k.run)) return rc;

@@ -128,6 +128,7 @@ struct pw_ctx {
     int ngroups = 0;
     int built_parts = 0;  // parts and split the items were built for (0: none yet)
     int built_split = 0;
+    size_t rows = 0;      // rows of the partial buffer the built items write
     bool lean = false;    // the chosen launch's buffers did not fit in memory
     bool tuned = false;
   } ks[3];

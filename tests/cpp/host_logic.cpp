@@ -1,0 +1,225 @@
+// Host side of the C API on a stand-in for the HIP runtime: device memory is
+// host memory, allocations can be made to fail, and the kernel launchers check
+// the buffers they are given instead of launching.  Built from pw_capi.hip and
+// pw_ff.hip with the host compiler by tests/test_host_logic.py; runs without a
+// GPU.  Usage: host_logic CHECK
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <limits>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "pw_ctx.h"
+#include "pw_mlp.h"
+
+// ---- the stand-in runtime ---------------------------------------------------
+namespace {
+
+size_t g_device_limit = std::numeric_limits<size_t>::max();  // bytes of device memory
+size_t g_pinned_limit = std::numeric_limits<size_t>::max();  // bytes of pinned memory
+size_t g_device_used = 0;
+std::map<const void*, size_t> g_device, g_pinned;
+std::vector<std::string> g_calls;  // launches and event records, in order
+int g_failures = 0;
+
+void expect(bool ok, const std::string& what) {
+  if (!ok) {
+    ++g_failures;
+    std::printf("FAILED: %s\n", what.c_str());
+  }
+}
+
+// bytes from p to the end of the device allocation that holds it
+size_t room(const void* p) {
+  auto it = g_device.upper_bound(p);
+  if (!p || it == g_device.begin()) return 0;
+  --it;
+  const char *at = static_cast<const char*>(p), *from = static_cast<const char*>(it->first);
+  return at < from + it->second ? static_cast<size_t>(from + it->second - at) : 0;
+}
+
+size_t pinned_used() {
+  size_t s = 0;
+  for (const auto& a : g_pinned) s += a.second;
+  return s;
+}
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t bytes) {
+  *p = nullptr;
+  if (bytes > g_device_limit || g_device_used > g_device_limit - bytes) return hipErrorOutOfMemory;
+  *p = std::malloc(bytes ? bytes : 1);
+  if (!*p) return hipErrorOutOfMemory;
+  g_device[*p] = bytes;
+  g_device_used += bytes;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  if (!p) return hipSuccess;
+  const auto it = g_device.find(p);
+  if (it == g_device.end()) return hipErrorInvalidValue;
+  g_device_used -= it->second;
+  g_device.erase(it);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+  *p = nullptr;
+  if (bytes > g_pinned_limit || pinned_used() > g_pinned_limit - bytes) return hipErrorOutOfMemory;
+  *p = std::malloc(bytes ? bytes : 1);
+  g_pinned[*p] = bytes;
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+  if (p && g_pinned.erase(p)) std::free(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t bytes, hipMemcpyKind) {
+  std::memcpy(d, s, bytes);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t bytes, hipMemcpyKind k, hipStream_t) {
+  return hipMemcpy(d, s, bytes, k);
+}
+hipError_t hipGetDeviceCount(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+  std::memset(p, 0, sizeof *p);
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void* s) {
+  *p = const_cast<void*>(s);
+  return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = reinterpret_cast<hipStream_t>(1);
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) {
+  *e = reinterpret_cast<hipEvent_t>(1);
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) {
+  g_calls.push_back("event");
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 1.0f;
+  return hipSuccess;
+}
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+}
+
+// ---- the launchers ----------------------------------------------------------
+namespace pw {
+
+int pair_kernel_waves(int, const PairConfig&) { return 8; }
+
+hipError_t launch_pair(int, const PairConfig& cfg, const PairArgs& a, int, hipStream_t) {
+  g_calls.push_back("pair");
+  expect(room(a.items) >= a.nitems * sizeof(WorkItem), "pair items hold the launch");
+  const size_t rows = cfg.split > 0 ? 64 * static_cast<size_t>(a.nitems)
+                                    : cfg.parts > 1 ? static_cast<size_t>(cfg.parts) * a.n : 0;
+  expect(room(a.partial) >= rows * sizeof(Rate64), "the partial rows hold the launch");
+  return hipSuccess;
+}
+hipError_t launch_finish(const SumForm&, Rate64*, int, int*, const StageOp&, hipStream_t) {
+  g_calls.push_back("finish");
+  return hipSuccess;
+}
+hipError_t launch_zero_doubles(double*, int64_t, hipStream_t) { return hipSuccess; }
+hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* host, bool store, hipStream_t) {
+  expect(g_pinned.count(host) && g_pinned[host] >= 48 * static_cast<size_t>(count), "staging holds the piece");
+  for (int64_t i = 0; i < count; ++i) {
+    Rec64& r = y[first + i];
+    double *x = host + 3 * i, *a = host + 3 * (count + i);
+    if (store) {
+      r.x = x[0]; r.y = x[1]; r.z = x[2];
+      r.ax = a[0]; r.ay = a[1]; r.az = a[2];
+    } else {
+      x[0] = r.x; x[1] = r.y; x[2] = r.z;
+      a[0] = r.ax; a[1] = r.ay; a[2] = r.az;
+    }
+  }
+  return hipSuccess;
+}
+
+}  // namespace pw
+
+// ---- the checks -------------------------------------------------------------
+namespace {
+
+pw_ctx* context(const std::vector<int64_t>& wakes, bool coupled = true) {
+  pw_ctx* c = nullptr;
+  expect(pw_create(&c, 0) == PW_OK, "create");
+  expect(pw_set_coupled(c, coupled) == PW_OK, "set_coupled");
+  int64_t base = 0;
+  for (const int64_t n : wakes) {
+    std::vector<double> x(3 * n), a(3 * n), r(n, 0.1), v(n, 1.0);
+    for (int64_t i = 0; i < 3 * n; ++i) {
+      x[i] = base + i;
+      a[i] = -(base + i) - 0.5;
+    }
+    base += 3 * n;
+    expect(pw_add_wake(c, n, n, x.data(), a.data(), r.data(), v.data(), nullptr) == PW_OK, "add_wake");
+  }
+  return c;
+}
+
+// One precision's larger partial-sum buffer does not fit: it runs in one part,
+// and what other precisions had built must not be launched without rows.
+void partial_buffer() {
+  for (const size_t left : {size_t(100) << 20, size_t(8) << 20, size_t(1) << 20}) {
+    pw_ctx* c = context({60000});
+    g_device_limit = std::numeric_limits<size_t>::max();
+    expect(pw_solve(c, PW_FP64) == PW_OK, "fp64");  // 64 parts: 184 MB of rows
+    g_device_limit = g_device_used + left;
+    expect(pw_solve(c, PW_FP32C) == PW_OK, "fp32c");  // split: more than that
+    expect(pw_solve(c, PW_FP64) == PW_OK, "fp64 again");
+    expect(pw_step(c, PW_RK4, 1e-3, PW_FP32C, 1) == PW_OK, "fp32c step");
+    expect(pw_step(c, PW_RK4, 1e-3, PW_FP64, 1) == PW_OK, "fp64 step");
+    pw_destroy(c);
+  }
+  // a number of parts that was asked for and does not fit is an error, and
+  // leaves the other precision a launch that has its rows
+  pw_ctx* c = context({60000});
+  g_device_limit = std::numeric_limits<size_t>::max();
+  expect(pw_set_pair_config(c, PW_FP64, 16, 1, 0) == PW_OK, "16 parts");
+  expect(pw_set_pair_config(c, PW_FP32C, 256, 1, 0) == PW_OK, "256 parts");
+  expect(pw_solve(c, PW_FP64) == PW_OK, "fp64 in 16 parts");
+  g_device_limit = g_device_used + (size_t(64) << 20);
+  expect(pw_solve(c, PW_FP32C) == PW_ERR_NOMEM, "256 parts do not fit");
+  expect(pw_solve(c, PW_FP32C) == PW_ERR_NOMEM, "nor the second time");
+  expect(pw_solve(c, PW_FP64) == PW_OK, "fp64 in 16 parts again");
+  pw_destroy(c);
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::map<std::string, void (*)()> checks = {{"partial_buffer", partial_buffer}};
+  if (argc != 2 || !checks.count(argv[1])) {
+    std::fprintf(stderr, "usage: host_logic CHECK\n");
+    return 2;
+  }
+  checks.at(argv[1])();
+  if (g_failures) std::printf("last error: %s\n", pw_last_error());
+  std::printf("%s: %d failures\n", argv[1], g_failures);
+  return g_failures ? 1 : 0;
+}
