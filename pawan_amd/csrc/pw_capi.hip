@@ -495,23 +495,33 @@ void append_items(const pw_ctx* c, int a, int b, int nself, std::vector<WorkItem
                    chunk_of(c, c->woff[b]), 0});
 }
 
-// Source range of the diagnostics' pair items over `systems` ([a, b) each):
-// the longest of 64 ... 1,024 particles that leaves ten blocks per CU (short
-// ranges cost the staging of a block's tiles and table per few pairs), longer
-// where the items would exceed 131,072.
+// Source range of the diagnostics' pair items, count(range) of them: the longest
+// of 64 ... 1,024 particles that leaves ten blocks per CU (short ranges cost the
+// staging of a block's tiles and table per few pairs), longer where the items
+// would exceed 131,072.
+template <typename Count>
+int diag_range(const Count& count) {
+  int range = 64;
+  while (range < 1024 && count(2 * range) >= 2560) range *= 2;
+  while (range < (1 << 28) && count(range) > 131072) range *= 2;
+  return range;
+}
+
+// over the unordered pairs of `systems` ([a, b) each)
 int diag_range(const std::vector<std::pair<int64_t, int64_t>>& systems) {
-  const auto count = [&](int64_t range) {
+  return diag_range([&](int64_t range) {
     int64_t items = 0;
     for (const auto& s : systems) {
       const int64_t len = s.second - s.first;
       items += (len + 63) / 64 * ((len + range - 1) / range + 1) / 2;
     }
     return items;
-  };
-  int range = 64;
-  while (range < 1024 && count(2 * range) >= 2560) range *= 2;
-  while (range < (1 << 28) && count(range) > 131072) range *= 2;
-  return range;
+  });
+}
+
+// over na x nb pairs of two wakes
+int diag_range(int64_t na, int64_t nb) {
+  return diag_range([=](int64_t range) { return (na + 63) / 64 * ((nb + range - 1) / range); });
 }
 
 // pair items of one system's unordered pairs
@@ -1450,14 +1460,15 @@ int pw_diagnose_wakes(pw_ctx* c, int wa, int wb, double* out, int64_t out_len) {
   if (wa == wb) {
     append_diag_items(c->woff[wa], c->woff[wa + 1], diag_range({{c->woff[wa], c->woff[wa + 1]}}), items);
   } else {
-    // every source of wake b, 1,024 at a time, for each 64 targets of wake a
+    // every source of wake b, a range at a time, for each 64 targets of wake a
+    const int range = diag_range(c->wn[wa], c->wn[wb]);
     for (int64_t t0 = c->woff[wa]; t0 < c->woff[wa + 1]; t0 += 64)
-      for (int64_t s0 = c->woff[wb]; s0 < c->woff[wb + 1]; s0 += 1024)
+      for (int64_t s0 = c->woff[wb]; s0 < c->woff[wb + 1]; s0 += range)
         items.push_back({static_cast<int32_t>(t0), static_cast<int32_t>(std::min<int64_t>(t0 + 64, c->woff[wa + 1])),
-                         static_cast<int32_t>(s0), static_cast<int32_t>(std::min<int64_t>(s0 + 1024, c->woff[wb + 1])),
+                         static_cast<int32_t>(s0), static_cast<int32_t>(std::min<int64_t>(s0 + range, c->woff[wb + 1])),
                          -1, 1, 0, 0});
   }
-  constexpr int Q = pw::kDiagQuad;
+  constexpr size_t Q = pw::kDiagQuad;
   const int ni = static_cast<int>(items.size());
   // the wake's linear-sum items are contiguous in the context's list
   int l0 = 0, nl = 0;
@@ -1468,20 +1479,26 @@ int pw_diagnose_wakes(pw_ctx* c, int wa, int wb, double* out, int64_t out_len) {
     }
   WorkItem* d_items = nullptr;
   double* d_q = nullptr;
-  if (ni > 0 && (dalloc(&d_items, items.size()) != hipSuccess || dalloc(&d_q, Q * items.size()) != hipSuccess)) {
+  // each item's sums, the block's, and the items of the block: [0, ni)
+  if (ni > 0 && (dalloc(&d_items, items.size()) != hipSuccess || dalloc(&d_q, Q * (items.size() + 1) + 1) != hipSuccess)) {
     (void)hipGetLastError();
     (void)hipFree(d_items);
     return fail(PW_ERR_NOMEM, "diagnostic buffers");
   }
-  std::vector<double> quad(Q * static_cast<size_t>(ni)), lin(11 * static_cast<size_t>(nl));
+  double q[Q] = {0.0};
+  const int first[2] = {0, ni};
+  std::vector<double> lin(11 * static_cast<size_t>(nl));
   hipError_t e = hipSuccess;
   if (ni > 0) {
+    double* d_sum = d_q + Q * items.size();
+    int* d_first = reinterpret_cast<int*>(d_sum + Q);
     e = hipMemcpyAsync(d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(d_first, first, sizeof first, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess)
       e = pw::launch_diag_pairs(c->y, c->d_radius, d_items, ni, d_q, c->smoothing == PW_KERNEL_HIGHORDER,
                                 c->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(quad.data(), d_q, quad.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = pw::launch_diag_sum(d_q, d_first, 1, d_sum, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(q, d_sum, sizeof q, hipMemcpyDeviceToHost, c->stream);
   }
   if (e == hipSuccess && wa == wb && nl > 0) {
     e = pw::launch_diag_linear(c->y, c->lin_items + l0, nl, c->d_lin + 11 * static_cast<size_t>(l0), c->stream);
@@ -1506,9 +1523,6 @@ int pw_diagnose_wakes(pw_ctx* c, int wa, int wb, double* out, int64_t out_len) {
     out[14] = v[9];
     out[15] = v[10];
   }
-  double q[Q] = {0};
-  for (int b = 0; b < ni; ++b)
-    for (int m = 0; m < Q; ++m) q[m] += quad[Q * b + m];
   // within a wake 2 sum_{i<j} plus the self terms; across wakes one
   // direction, doubled as in calculate*(W1, W2) (interaction.cpp:551-718)
   const double f = wa == wb ? 1.0 : 2.0;

@@ -24,6 +24,7 @@ size_t g_pinned_limit = std::numeric_limits<size_t>::max();  // bytes of pinned 
 size_t g_device_used = 0;
 std::map<const void*, size_t> g_device, g_pinned;
 std::vector<std::string> g_calls;  // launches and event records, in order
+std::vector<pw::WorkItem> g_diag;  // the last diagnostics launch
 int g_failures = 0;
 
 void expect(bool ok, const std::string& what) {
@@ -144,6 +145,30 @@ hipError_t launch_finish(const SumForm&, Rate64*, int, int*, const StageOp&, hip
   return hipSuccess;
 }
 hipError_t launch_zero_doubles(double*, int64_t, hipStream_t) { return hipSuccess; }
+hipError_t launch_diag_linear(const Rec64*, const WorkItem*, int nitems, double* out, hipStream_t) {
+  for (int k = 0; k < 11 * nitems; ++k) out[k] = 0.0;
+  return hipSuccess;
+}
+// every item's sums are its number of pairs
+hipError_t launch_diag_pairs(const Rec64*, const double*, const WorkItem* items, int nitems, double* out, bool,
+                             hipStream_t) {
+  g_diag.assign(items, items + nitems);
+  expect(room(out) >= kDiagQuad * sizeof(double) * nitems, "the sums hold the items");
+  for (int b = 0; b < nitems; ++b)
+    for (int m = 0; m < kDiagQuad; ++m)
+      out[kDiagQuad * b + m] =
+          static_cast<double>(items[b].t1 - items[b].t0) * static_cast<double>(items[b].s1 - items[b].s0);
+  return hipSuccess;
+}
+hipError_t launch_diag_sum(const double* items, const int* first, int nsys, double* out, hipStream_t) {
+  for (int s = 0; s < nsys; ++s)
+    for (int m = 0; m < kDiagQuad; ++m) {
+      double v = 0.0;
+      for (int b = first[s]; b < first[s + 1]; ++b) v += items[kDiagQuad * b + m];
+      out[kDiagQuad * s + m] = v;
+    }
+  return hipSuccess;
+}
 hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* host, bool store, hipStream_t) {
   expect(g_pinned.count(host) && g_pinned[host] >= 48 * static_cast<size_t>(count), "staging holds the piece");
   for (int64_t i = 0; i < count; ++i) {
@@ -210,10 +235,36 @@ void partial_buffer() {
   pw_destroy(c);
 }
 
+// Wake blocks of the diagnostics: at most 131,072 items whatever the sizes, at
+// most 64 targets each, which together cover the block.
+void diagnose_items() {
+  const std::vector<std::vector<int64_t>> sizes = {{500000, 500000}, {1100000, 900000}, {65, 70000}, {70000, 65}, {1, 1}};
+  for (const auto& n : sizes) {
+    pw_ctx* c = context(n);
+    double out[16];
+    expect(pw_diagnose_wakes(c, 0, 1, out, 16) == PW_OK, "cross block");
+    expect(g_diag.size() <= 131072, "items of a cross block: " + std::to_string(g_diag.size()));
+    double pairs = 0.0;
+    for (const auto& it : g_diag) {
+      expect(it.nself == 1 && it.t0 >= 0 && it.t1 <= n[0] && it.s0 >= n[0] && it.s1 <= n[0] + n[1] && it.t0 < it.t1 &&
+                 it.t1 - it.t0 <= 64 && it.s0 < it.s1,
+             "an item of a cross block");
+      pairs += static_cast<double>(it.t1 - it.t0) * static_cast<double>(it.s1 - it.s0);
+    }
+    const double all = static_cast<double>(n[0]) * static_cast<double>(n[1]);
+    expect(pairs == all, "a cross block is covered");
+    expect(out[9] == 2.0 * all, "the sum of a cross block");
+    expect(pw_diagnose_wakes(c, 1, 1, out, 16) == PW_OK && g_diag.size() <= 131072, "a wake's own block");
+    for (const auto& it : g_diag) expect(it.nself == 0 && it.s0 >= n[0] && it.s1 <= it.t1, "an item of a wake");
+    pw_destroy(c);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, void (*)()> checks = {{"partial_buffer", partial_buffer}};
+  const std::map<std::string, void (*)()> checks = {{"partial_buffer", partial_buffer},
+                                                      {"diagnose_items", diagnose_items}};
   if (argc != 2 || !checks.count(argv[1])) {
     std::fprintf(stderr, "usage: host_logic CHECK\n");
     return 2;

@@ -35,3 +35,9 @@ def test_partial_buffer_that_does_not_fit(host_logic):
     """A precision whose partial-sum rows do not fit runs in one part or
     reports it; the other precisions' launches still get rows of their own."""
     _run(host_logic, "partial_buffer")
+
+
+def test_diagnostics_of_wake_blocks_stay_bounded(host_logic):
+    """However large two wakes are, their block is a bounded number of items
+    that cover it, and its sums come from all of them."""
+    _run(host_logic, "diagnose_items")
