@@ -729,24 +729,24 @@ void copy_segments(const std::vector<Segment>& segs) {
 }
 
 // Pinned staging for up to `count` particles (6 doubles each, 256 MB at most:
-// longer transfers go in pieces).  The stream is idle when it returns, so the
-// staging is free.
+// longer transfers go in pieces, and so do those that pinned memory cannot be had
+// for).  The stream is idle when it returns, so the staging is free.
 int ensure_stage(pw_ctx* c, int64_t count) {
   constexpr int64_t kMaxParticles = (int64_t(256) << 20) / 48;
   const int64_t want = std::min(count, kMaxParticles);
   PW_HIP(hipStreamSynchronize(c->stream));
-  if (static_cast<size_t>(want) <= c->stage_particles) return PW_OK;
-  (void)hipHostFree(c->h_stage);
-  c->h_stage = nullptr;
-  c->stage_particles = 0;
-  if (hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), 48 * static_cast<size_t>(want), hipHostMallocCoherent) !=
-      hipSuccess) {
-    (void)hipGetLastError();
-    c->h_stage = nullptr;
-    return fail(PW_ERR_NOMEM, "pinned staging");
+  for (int64_t m = want; m > static_cast<int64_t>(c->stage_particles); m /= 2) {
+    double* fresh = nullptr;
+    if (hipHostMalloc(reinterpret_cast<void**>(&fresh), 48 * static_cast<size_t>(m), hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
+      continue;
+    }
+    (void)hipHostFree(c->h_stage);
+    c->h_stage = fresh;
+    c->stage_particles = static_cast<size_t>(m);
+    return PW_OK;
   }
-  c->stage_particles = static_cast<size_t>(want);
-  return PW_OK;
+  return c->stage_particles > 0 ? PW_OK : fail(PW_ERR_NOMEM, "pinned staging");
 }
 
 // positions and strengths (or, rates, velocities and vorticity rates) of
@@ -799,7 +799,7 @@ int ensure_built(pw_ctx* c) { return ::ensure_built(c); }
 
 int staging(pw_ctx* c, size_t bytes, void** out) {
   PW_TRY(ensure_stage(c, static_cast<int64_t>((bytes + 47) / 48)));
-  if (bytes > 48 * c->stage_particles) return fail(PW_ERR_UNSUPPORTED, "staging beyond 256 MB");
+  if (bytes > 48 * c->stage_particles) return fail(PW_ERR_NOMEM, "pinned staging");
   *out = c->h_stage;
   return PW_OK;
 }

@@ -173,7 +173,7 @@ namespace pwi {
 
 int ensure_built(pw_ctx* c);
 // at least `bytes` (256 MB at most) of the context's pinned staging, the stream
-// idle
+// idle; PW_ERR_NOMEM if there is not so much
 int staging(pw_ctx* c, size_t bytes, void** out);
 // event pair for one profiled launch (recycled)
 int prof_begin(pw_ctx* c, hipEvent_t* e0, hipEvent_t* e1);

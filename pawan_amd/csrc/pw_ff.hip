@@ -866,16 +866,17 @@ int pw_ff_mlp_grad(pw_ctx* c, const float* X, const float* Y, int64_t n, float* 
   }
   float *dX = w, *dY = w + 16 * m, *g = w + in, *l = g + pw::kMlpParams, *gp = g + res, *lp = gp + blocks * pw::kMlpParams;
   // the samples and the result pass through pinned memory (copies from and to
-  // pageable memory cost more than the kernels); batches too large for it go
-  // straight
+  // pageable memory cost more than the kernels); batches too large for it, or
+  // for the pinned memory there is, go straight
   void* st = nullptr;
-  const bool pinned = in * sizeof(float) <= (size_t(64) << 20);
+  bool pinned = in * sizeof(float) <= (size_t(64) << 20);
   if (pinned) {
     const int rc = pwi::staging(c, std::max(in, res) * sizeof(float), &st);
-    if (rc != PW_OK) {
+    if (rc != PW_OK && rc != PW_ERR_NOMEM) {
       (void)hipFree(own);
       return rc;
     }
+    pinned = rc == PW_OK;
   }
   hipError_t e = hipSuccess;
   if (pinned) {

@@ -185,6 +185,30 @@ hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* hos
   return hipSuccess;
 }
 
+hipError_t launch_pack_rates(const Rate64* k, int64_t first, int64_t count, double* host, hipStream_t) {
+  expect(g_pinned.count(host) && g_pinned[host] >= 48 * static_cast<size_t>(count), "staging holds the piece");
+  for (int64_t i = 0; i < count; ++i) {
+    std::memcpy(host + 3 * i, &k[first + i].ux, 24);
+    std::memcpy(host + 3 * (count + i), &k[first + i].wx, 24);
+  }
+  return hipSuccess;
+}
+int train_blocks(int) { return 256; }
+void pack_mlp(const float*, std::vector<uint16_t>& frag, std::vector<float>& bias) {
+  frag.assign(kMlpFragElems, 0);
+  bias.assign(kMlpBiasLen, 0.0f);
+}
+// the gradient is the sum of the inputs, the loss that of the targets
+hipError_t launch_mlp_grad(const float*, const float* X, const float* Y, const int*, int n, float*, float*, float* grad,
+                           float* loss, hipStream_t) {
+  float x = 0.0f, y = 0.0f;
+  for (int i = 0; i < 16 * n; ++i) x += X[i];
+  for (int i = 0; i < 12 * n; ++i) y += Y[i];
+  for (int p = 0; p < kMlpParams; ++p) grad[p] = x;
+  *loss = y;
+  return hipSuccess;
+}
+
 }  // namespace pw
 
 // ---- the checks -------------------------------------------------------------
@@ -260,11 +284,51 @@ void diagnose_items() {
   }
 }
 
+// With little pinned memory to be had, transfers go in smaller pieces and the
+// training samples straight from the caller's memory.
+void little_pinned_memory() {
+  g_pinned_limit = 100000;  // 2,083 particles
+  const std::vector<int64_t> n = {30000, 7, 4001};
+  pw_ctx* c = context(n, false);
+  expect(pw_diagnose_wakes(c, 1, 1, std::vector<double>(16).data(), 16) == PW_OK, "build");
+  const int64_t all = 30000 + 7 + 4001;
+  std::vector<double> x(3 * all), a(3 * all);
+  const auto is = [&](const std::vector<double>& v, int64_t from, int64_t m, double sign, double shift) {
+    for (int64_t i = 0; i < m; ++i)
+      if (v[i] != sign * (from + i) + shift) return false;
+    return true;
+  };
+  expect(pw_get_all_state(c, x.data(), a.data()) == PW_OK, "all state");
+  expect(is(x, 0, 3 * all, 1.0, 0.0) && is(a, 0, 3 * all, -1.0, -0.5), "the state of all wakes");
+  expect(pw_get_wake_state(c, 2, x.data(), a.data()) == PW_OK, "a wake's state");
+  expect(is(x, 3 * 30007, 3 * 4001, 1.0, 0.0) && is(a, 3 * 30007, 3 * 4001, -1.0, -0.5), "the state of a wake");
+  std::vector<double> x0(3 * 30000), a0(3 * 30000);
+  for (size_t i = 0; i < x0.size(); ++i) {
+    x0[i] = i + 0.25;
+    a0[i] = 2.0 - i;
+  }
+  expect(pw_set_wake_state(c, 0, x0.data(), a0.data()) == PW_OK, "set a wake's state");
+  expect(pw_get_all_state(c, x.data(), a.data()) == PW_OK, "all state");
+  expect(is(x, 0, 3 * 30000, 1.0, 0.25) && is(a, 0, 3 * 30000, -1.0, 2.0), "the state that was set");
+  expect(pw_get_all_rates(c, x.data(), a.data()) == PW_OK, "all rates");
+  const int64_t batch = 5000;  // 560 kB of samples
+  std::vector<float> w(pw::kMlpParams, 0.5f), X(16 * batch, 1.0f), Y(12 * batch, 2.0f), grad(pw::kMlpParams);
+  double loss = 0.0;
+  expect(pw_ff_set_weights(c, w.data(), pw::kMlpParams) == PW_OK, "weights");
+  expect(pw_ff_mlp_grad(c, X.data(), Y.data(), batch, grad.data(), &loss) == PW_OK, "gradient");
+  expect(grad[0] == 16.0f * batch && grad[pw::kMlpParams - 1] == 16.0f * batch && loss == 24.0f * batch,
+         "the gradient's result");
+  pw_destroy(c);
+  expect(g_pinned.empty() && g_device.empty(), "everything is given back");
+  g_pinned_limit = std::numeric_limits<size_t>::max();
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> checks = {{"partial_buffer", partial_buffer},
-                                                      {"diagnose_items", diagnose_items}};
+                                                      {"diagnose_items", diagnose_items},
+                                                      {"little_pinned_memory", little_pinned_memory}};
   if (argc != 2 || !checks.count(argv[1])) {
     std::fprintf(stderr, "usage: host_logic CHECK\n");
     return 2;

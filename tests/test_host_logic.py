@@ -41,3 +41,9 @@ def test_diagnostics_of_wake_blocks_stay_bounded(host_logic):
     """However large two wakes are, their block is a bounded number of items
     that cover it, and its sums come from all of them."""
     _run(host_logic, "diagnose_items")
+
+
+def test_transfers_with_little_pinned_memory(host_logic):
+    """States, rates and training samples pass where the staging of their
+    whole size cannot be pinned."""
+    _run(host_logic, "little_pinned_memory")
