@@ -297,7 +297,8 @@ int pw_diagnose(pw_ctx *ctx, double *out, int64_t out_len);
 int pw_synchronize(pw_ctx *ctx);
 
 /* Kernel timing with HIP events on the context's stream.  While enabled,
- * every launch of the pair-interaction kernel is bracketed by events; the
+ * every launch of the pair-interaction kernel is bracketed by events, with
+ * the kernel that sums its partial rates where the sources are split; the
  * totals accumulate until reset.  pw_get_pair_timing synchronises and
  * returns the summed kernel time in milliseconds and the number of
  * launches. */

@@ -622,11 +622,15 @@ int rhs(pw_ctx* c, int kind, const Rec64* state, Rate64* out, const pw::StageOp&
     PW_HIP(hipEventRecord(e0, c->stream));
   }
   PW_HIP(pw::launch_pair(launch_kind, k.run, args, grid, c->stream));
+  // the timing holds the sum of the partial rates (and the stage arithmetic that
+  // goes with it), but no pass of its own over finished rates
+  const bool summed = sum.groups || sum.parts > 1;
+  if (c->profiling && !summed) PW_HIP(hipEventRecord(e1, c->stream));
+  PW_HIP(pw::launch_finish(sum, out, n, c->h_flag, op, c->stream));
   if (c->profiling) {
-    PW_HIP(hipEventRecord(e1, c->stream));
+    if (summed) PW_HIP(hipEventRecord(e1, c->stream));
     c->ev_used.emplace_back(e0, e1);
   }
-  PW_HIP(pw::launch_finish(sum, out, n, c->h_flag, op, c->stream));
   return PW_OK;
 }
 

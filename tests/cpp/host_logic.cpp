@@ -323,12 +323,35 @@ void little_pinned_memory() {
   g_pinned_limit = std::numeric_limits<size_t>::max();
 }
 
+// The pair timing holds the sum of the partial rates, where there are any.
+void timed_launches() {
+  using Calls = std::vector<std::string>;
+  const Calls summed = {"event", "pair", "finish", "event"}, whole = {"event", "pair", "event", "finish"};
+  pw_ctx* c = context({5000});
+  expect(pw_set_profiling(c, 1) == PW_OK, "profiling");
+  const auto solve = [&](int precision, const Calls& order, const char* what) {
+    g_calls.clear();
+    expect(pw_solve(c, precision) == PW_OK && g_calls == order, what);
+  };
+  solve(PW_FP64, summed, "the default launch of a small system");
+  expect(pw_set_pair_config(c, PW_FP32C, 8, 1, 0) == PW_OK, "8 parts");
+  solve(PW_FP32C, summed, "8 parts");
+  solve(PW_FP64_REF, whole, "one part");
+  expect(pw_set_pair_config(c, PW_FP32C, 1, 1, 0) == PW_OK, "1 part");
+  solve(PW_FP32C, whole, "one part, persistent");
+  double ms = 0.0;
+  int64_t launches = 0;
+  expect(pw_get_pair_timing(c, &ms, &launches) == PW_OK && launches == 4 && ms == 4.0, "totals");
+  pw_destroy(c);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> checks = {{"partial_buffer", partial_buffer},
                                                       {"diagnose_items", diagnose_items},
-                                                      {"little_pinned_memory", little_pinned_memory}};
+                                                      {"little_pinned_memory", little_pinned_memory},
+                                                      {"timed_launches", timed_launches}};
   if (argc != 2 || !checks.count(argv[1])) {
     std::fprintf(stderr, "usage: host_logic CHECK\n");
     return 2;

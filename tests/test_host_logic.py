@@ -47,3 +47,7 @@ def test_transfers_with_little_pinned_memory(host_logic):
     """States, rates and training samples pass where the staging of their
     whole size cannot be pinned."""
     _run(host_logic, "little_pinned_memory")
+
+
+def test_pair_timing_holds_the_sum_of_partial_rates(host_logic):
+    _run(host_logic, "timed_launches")
