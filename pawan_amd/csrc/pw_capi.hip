@@ -161,24 +161,26 @@ void build_items(pw_ctx* c) {
   c->h_lin_items.clear();
   c->lin_wake.clear();
   const int nw = static_cast<int>(c->wn.size());
-  struct Sys {
-    int64_t a, b;
-    int id;
-  };
-  std::vector<Sys> sys;
-  if (c->coupled)
-    sys.push_back({0, c->n, 0});
-  else
-    for (int w = 0; w < nw; ++w) sys.push_back({c->woff[w], c->woff[w + 1], w});
-  std::stable_sort(sys.begin(), sys.end(),
-                   [](const Sys& p, const Sys& q) { return (p.b - p.a) > (q.b - q.a); });
+  // source chunks of the scalar-fed and split kernels: runs of up to 64
+  // particles of one system, in particle order
   c->systems.clear();
-  for (const Sys& s : sys) c->systems.push_back({s.a, s.b, s.id});
-  for (const Sys& s : sys)
+  c->chunk_first.clear();
+  const auto add_system = [&](int64_t a, int64_t b, int id) {
+    c->systems.push_back({a, b, id, static_cast<int32_t>(c->chunk_first.size())});
+    for (int64_t i = a; i < b; i += 64) c->chunk_first.push_back(static_cast<int32_t>(i));
+  };
+  if (c->coupled)
+    add_system(0, c->n, 0);
+  else
+    for (int w = 0; w < nw; ++w) add_system(c->woff[w], c->woff[w + 1], w);
+  c->nchunks = static_cast<int>(c->chunk_first.size());
+  std::stable_sort(c->systems.begin(), c->systems.end(),
+                   [](const pw_ctx::SysRange& p, const pw_ctx::SysRange& q) { return (p.b - p.a) > (q.b - q.a); });
+  for (const auto& s : c->systems)
     for (int64_t t0 = s.a; t0 < s.b; t0 += kTargetsPerItem) {
       c->h_pair_items.push_back({static_cast<int32_t>(t0),
                                  static_cast<int32_t>(std::min<int64_t>(t0 + kTargetsPerItem, s.b)),
-                                 static_cast<int32_t>(s.a), static_cast<int32_t>(s.b), -1, 0, 0, 0});
+                                 static_cast<int32_t>(s.a), static_cast<int32_t>(s.b), -1, 0, s.chunk, 0});
     }
   for (int w = 0; w < nw; ++w)
     for (int64_t t0 = c->woff[w]; t0 < c->woff[w + 1]; t0 += kTargetsPerItem) {
@@ -190,17 +192,6 @@ void build_items(pw_ctx* c) {
     }
   c->npair = static_cast<int>(c->h_pair_items.size());
   c->nlin = static_cast<int>(c->h_lin_items.size());
-  // source chunks of the scalar-fed FP32C kernel: runs of up to 64
-  // particles of one system, in particle order
-  c->chunk_first.clear();
-  if (c->coupled) {
-    for (int64_t i = 0; i < c->n; i += 64) c->chunk_first.push_back(static_cast<int32_t>(i));
-  } else {
-    for (int w = 0; w < nw; ++w)
-      for (int64_t i = c->woff[w]; i < c->woff[w + 1]; i += 64) c->chunk_first.push_back(static_cast<int32_t>(i));
-  }
-  c->nchunks = static_cast<int>(c->chunk_first.size());
-  for (auto& it : c->h_pair_items) it.chunk0 = chunk_of(c, it.s0);
 }
 
 int ensure_built(pw_ctx* c) {
@@ -283,6 +274,7 @@ int kind_of(int precision, int* kind) {
 // FP32 source records), instead of every range at once.
 std::vector<WorkItem> make_items(const pw_ctx* c, int parts) {
   std::vector<WorkItem> items;
+  items.reserve(c->h_pair_items.size() * static_cast<size_t>(parts));
   for (const auto& s : c->systems) {
     const int64_t ntile = (s.b - s.a + kTargetsPerItem - 1) / kTargetsPerItem;
     for (int p = 0; p < parts; ++p) {
@@ -291,7 +283,8 @@ std::vector<WorkItem> make_items(const pw_ctx* c, int parts) {
       for (int64_t t0 = s.a; t0 < s.b; t0 += kTargetsPerItem) {
         const int32_t t1 = static_cast<int32_t>(std::min<int64_t>(t0 + kTargetsPerItem, s.b));
         items.push_back({static_cast<int32_t>(t0), t1, static_cast<int32_t>(a),
-                         static_cast<int32_t>(std::max(a, b)), parts == 1 ? -1 : p, 0, chunk_of(c, a), 0});
+                         static_cast<int32_t>(std::max(a, b)), parts == 1 ? -1 : p, 0,
+                         s.chunk + static_cast<int32_t>((a - s.a) / 64), 0});
       }
     }
   }
@@ -322,9 +315,18 @@ bool is_default(const pw::PairConfig& p) {
   return p.parts == 1 && !p.persistent && !p.waves8 && !p.scalar_feed && !p.two_per_lane && p.split == 0;
 }
 
+int64_t split_items(const pw_ctx* c, int split) {
+  int64_t items = 0;
+  for (const auto& s : c->systems) items += ((s.b - s.a + 63) / 64) * ((s.b - s.a + split - 1) / split);
+  return items;
+}
+
 // Items and groups of a split launch: every system's targets in groups of 64,
-// each against source ranges of `split` particles, items group by group.
+// each against source ranges of `split` particles, items group by group.  Built
+// on the first launch, so counted first and without a search per item (48 rings
+// of 512-16,384, 105,000 items: 2.3 -> 0.12 ms).
 void make_split(const pw_ctx* c, int split, std::vector<WorkItem>& items, std::vector<pw::SplitGroup>& groups) {
+  items.reserve(static_cast<size_t>(split_items(c, split)));
   for (const auto& s : c->systems)
     for (int64_t t0 = s.a; t0 < s.b; t0 += 64) {
       const int32_t t1 = static_cast<int32_t>(std::min<int64_t>(t0 + 64, s.b));
@@ -332,15 +334,10 @@ void make_split(const pw_ctx* c, int split, std::vector<WorkItem>& items, std::v
       for (int64_t a = s.a; a < s.b; a += split, ++g.count)
         items.push_back({static_cast<int32_t>(t0), t1, static_cast<int32_t>(a),
                          static_cast<int32_t>(std::min<int64_t>(a + split, s.b)),
-                         static_cast<int32_t>(items.size()), 0, chunk_of(c, a), chunk_of(c, t0)});
+                         static_cast<int32_t>(items.size()), 0,
+                         s.chunk + static_cast<int32_t>((a - s.a) / 64), s.chunk + static_cast<int32_t>((t0 - s.a) / 64)});
       groups.push_back(g);
     }
-}
-
-int64_t split_items(const pw_ctx* c, int split) {
-  int64_t items = 0;
-  for (const auto& s : c->systems) items += ((s.b - s.a + 63) / 64) * ((s.b - s.a + split - 1) / split);
-  return items;
 }
 
 // The launch of a kind whose configuration is the default (one part, grid, LDS

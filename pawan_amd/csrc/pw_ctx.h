@@ -148,6 +148,7 @@ struct pw_ctx {
   struct SysRange {
     int64_t a, b;
     int id;
+    int32_t chunk;  // its first source chunk
   };
   std::vector<SysRange> systems;  // largest first
 

@@ -137,6 +137,15 @@ hipError_t launch_pair(int, const PairConfig& cfg, const PairArgs& a, int, hipSt
   expect(room(a.items) >= a.nitems * sizeof(WorkItem), "pair items hold the launch");
   const size_t rows = cfg.split > 0 ? 64 * static_cast<size_t>(a.nitems)
                                     : cfg.parts > 1 ? static_cast<size_t>(cfg.parts) * a.n : 0;
+  bool chunks = true;
+  for (int b = 0; b < a.nitems; ++b) {
+    const WorkItem& it = a.items[b];
+    const auto holds = [&](int32_t chunk, int32_t s) {
+      return chunk >= 0 && chunk < a.nchunks && a.chunks[chunk].first <= s && s < a.chunks[chunk].first + a.chunks[chunk].count;
+    };
+    chunks = chunks && holds(it.chunk0, it.s0) && (cfg.split == 0 || holds(it.tchunk, it.t0));
+  }
+  expect(chunks, "the items name their chunks");
   expect(room(a.partial) >= rows * sizeof(Rate64), "the partial rows hold the launch");
   return hipSuccess;
 }
@@ -345,13 +354,31 @@ void timed_launches() {
   pw_destroy(c);
 }
 
+// Every launch's items name the chunks that hold their sources (and targets).
+void item_chunks() {
+  const std::vector<std::vector<int64_t>> sizes = {{1}, {64}, {65}, {1000}, {5000, 0, 777}, {63, 64, 65, 300, 1, 9001}, {41000}, {70001, 3}};
+  for (const auto& n : sizes)
+    for (const bool coupled : {false, true}) {
+      pw_ctx* c = context(n, coupled);
+      for (const int precision : {PW_FP64, PW_FP32C, PW_FP64_REF}) {
+        expect(pw_solve(c, precision) == PW_OK, "the default launch");
+        for (const int parts : {1, 2, 7}) {
+          expect(pw_set_pair_config(c, precision, parts, 1, PW_VARIANT_SCALAR_FEED) == PW_OK, "parts");
+          expect(pw_solve(c, precision) == PW_OK, "a launch in parts");
+        }
+      }
+      pw_destroy(c);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> checks = {{"partial_buffer", partial_buffer},
                                                       {"diagnose_items", diagnose_items},
                                                       {"little_pinned_memory", little_pinned_memory},
-                                                      {"timed_launches", timed_launches}};
+                                                      {"timed_launches", timed_launches},
+                                                      {"item_chunks", item_chunks}};
   if (argc != 2 || !checks.count(argv[1])) {
     std::fprintf(stderr, "usage: host_logic CHECK\n");
     return 2;

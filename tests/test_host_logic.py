@@ -51,3 +51,8 @@ def test_transfers_with_little_pinned_memory(host_logic):
 
 def test_pair_timing_holds_the_sum_of_partial_rates(host_logic):
     _run(host_logic, "timed_launches")
+
+
+def test_items_name_their_chunks(host_logic):
+    """Coupled and independent wakes, the default launch and source parts."""
+    _run(host_logic, "item_chunks")
