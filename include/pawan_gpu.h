@@ -323,7 +323,9 @@ int pw_get_pair_timing(pw_ctx *ctx, double *total_ms, int64_t *launches);
  * No counterpart in the reference (its OpenMP loops have no launch shape);
  * defaults are parts 1, grid launch, variant 0, which leaves the launch to
  * the library: source ranges split over the chip for small systems, the
- * scalar-fed kernels over many parts for large ones.  A variant outside those
+ * scalar-fed kernels over many parts for large ones.  Setting them asks for
+ * that again, and pw_get_pair_config and the autotuner's file report it so;
+ * LDS tiles in one part are parts 1, persistent 1.  A variant outside those
  * bits is PW_ERR_ARG. */
 enum {
   PW_VARIANT_WAVES8 = 1,

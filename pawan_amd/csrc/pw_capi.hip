@@ -1657,7 +1657,8 @@ namespace {
 // problem's shape; optionally also appended to / read from the text file
 // named by $PAWAN_TUNE_CACHE ("kind n nsys largest parts persistent variant",
 // kind the pair-kernel family: 0-2 for the Gaussian precisions, 4 and 5
-// for the high-order FP64 and FP32C kernels; variant the PW_VARIANT_* bits).
+// for the high-order FP64 and FP32C kernels; variant the PW_VARIANT_* bits;
+// 1 0 0 leaves the launch to auto_config).
 using TuneKey = std::tuple<int, int64_t, int, int64_t>;
 std::map<TuneKey, pw::PairConfig>& tune_cache() {
   static std::map<TuneKey, pw::PairConfig> m;

@@ -159,7 +159,7 @@ struct SumForm {
 // rate, and the stage arithmetic, in one pass.  flag: a word of pinned host
 // memory.
 hipError_t launch_finish(const SumForm& sum, Rate64* rates, int n, int* flag, const StageOp& op, hipStream_t st);
-// count of non-finite entries of the rates -> *flag (device int)
+// *flag = 1 if any rate is not finite (flag: a word of pinned host memory)
 hipError_t launch_check_finite(const Rate64* k, int n, int* flag,
                                hipStream_t st);
 
