@@ -26,8 +26,8 @@ times RK4 steps at it.  The drift leg runs 200 RK4 steps of the
 leapfrogging rings (N = 65,536) at nu = 1e-4 and nu = 0 with FP64, FP32C and
 the tree path side by side: every 10 steps it records each path's
 conserved quantities against FP64's at the same time, and the velocity
-error of its right-hand side against FP64 on its own state.  The CPU
-baseline is the oracle's restatement of the reference's OpenMP loops
+error of its right-hand side against FP64 on its own state (the JSON line has
+their maxima, with --drift-series the values too).  The CPU baseline is the oracle's restatement of the reference's OpenMP loops
 (parallel.cpp), timed on a sample of source rows of the same system and
 extrapolated to one RK4 step.
 
@@ -62,6 +62,33 @@ PEAK_FP32_TFLOPS = 157.3      # MI355X published FP32 vector peak
 PEAK_FP64_TFLOPS = 78.6       # MI355X published FP64 vector peak
 PEAK_BF16_TFLOPS = 2500.0     # MI355X published dense BF16 matrix-core peak
 FLOP_PER_MLP_EVAL = 72704     # 16-128-128-128-12 network, FMA = 2
+
+
+def short(o, digits: int = 7):
+    """o with its floats rounded to `digits` significant digits."""
+    if isinstance(o, dict):
+        return {k: short(v, digits) for k, v in o.items()}
+    if isinstance(o, (list, tuple)):
+        return [short(v, digits) for v in o]
+    return float(f"{o:.{digits}g}") if isinstance(o, float) else o
+
+
+SERIES = ("dev", "drift", "e_u_maxnorm", "e_u_rms")  # per path of the drift leg, one value a checkpoint
+
+
+def result_line(result: dict, series: bool = False) -> str:
+    """The bench's one JSON line.  The drift leg's time series (45 of 52 KB, too
+    long for readers that keep the end of the output) stay out of it unless asked
+    for; their maxima stay in.  Seven digits of the figures, five of the details,
+    three of the drift."""
+    if "drift" in result and not series:
+        runs = [{**run, "paths": {p: {k: v for k, v in rec.items() if k not in SERIES}
+                                  for p, rec in run["paths"].items()}} for run in result["drift"]["runs"]]
+        for run in runs:
+            run.pop("t", None)
+        result = {**result, "drift": short({**result["drift"], "runs": runs}, 3)}
+    return json.dumps({k: short(v, 5 if isinstance(v, dict) else 7) for k, v in result.items()},
+                      separators=(",", ":"))
 
 
 def log(msg: str) -> None:
@@ -172,7 +199,7 @@ def learned_leg(system, dt: float, steps: int, target_err: float, theta: float, 
     from pawan_amd import capi
 
     weights, rep, ttrain = train_network(train_n, train_samples, train_steps, theta)
-    log(f"network trained in {ttrain:.1f} s: {rep}")
+    log(f"network trained in {ttrain:.1f} s: {short(rep, 4)}")
     out = {"training": dict(rep, seconds=ttrain, samples=train_samples, wake_particles=train_n),
            "theta": theta, "target_error": target_err,
            "error_metric": "max_i |du_i| / max_i |u_i| against the FP64 direct sum on the same state"}
@@ -222,7 +249,7 @@ def learned_leg(system, dt: float, steps: int, target_err: float, theta: float, 
                     "flop_per_launch": flop, "avg_launch_ms": st["far_mlp_ms"],
                     "work": f"{info['mlp_evals']} network evaluations (one per target leaf and far node) "
                             f"x {FLOP_PER_MLP_EVAL} FLOP"}
-            log(f"{key}: {out[key]}")
+            log(f"{key}: {short(out[key], 4)}")
             if use_mlp:
                 out["_drift_cfg"] = {"weights": weights, "coef_md": rep["coef_md"], "coef_mlp": rep["coef_mlp"],
                                      "theta": theta, "tol_rel": tol / urms}
@@ -326,7 +353,7 @@ def drift_leg(steps: int, every: int, learned_cfg: dict | None, target_err: floa
             rec["max_drift"] = {k: max(v) for k, v in rec["drift"].items()}
             if rec["e_u_maxnorm"]:
                 rec["max_e_u_maxnorm"] = max(rec["e_u_maxnorm"])
-            log(f"drift nu={nu} {p}: max dev {rec['max_dev']} max drift {rec['max_drift']}"
+            log(f"drift nu={nu} {p}: max dev {short(rec['max_dev'], 3)}"
                 + (f" max e_u {rec['max_e_u_maxnorm']:.2e}" if rec["e_u_maxnorm"] else ""))
         run["seconds"] = time.perf_counter() - t0
         out["runs"].append(run)
@@ -648,6 +675,7 @@ def main() -> int:
     ap.add_argument("--no-drift", action="store_true")
     ap.add_argument("--drift-steps", type=int, default=200)
     ap.add_argument("--drift-every", type=int, default=10)
+    ap.add_argument("--drift-series", action="store_true", help="the drift leg's time series in the JSON line too")
     ap.add_argument("--save-weights", default="", help="write the trained network (npz) here")
     # other measurements
     ap.add_argument("--trajectory", action="store_true", help="FP32C vs FP64 trajectory of the helical wake")
@@ -710,7 +738,7 @@ def main() -> int:
     log(f"fp32c: {sps32:.4f} steps/s, pair kernel avg {avg32:.1f} ms over {l32} launches")
 
     ceil = valu_ceilings()
-    log(f"valu ceilings: {ceil}")
+    log(f"valu ceilings: {short(ceil, 4)}")
     out64 = {}
     if not args.no_fp64 and args.fp64_steps > 0:
         wall64, ms64, l64, tune64 = time_path(system, "fp64", dt, args.fp64_steps, 0,
@@ -735,7 +763,7 @@ def main() -> int:
         }
         log(f"fp64: {out64['fp64_steps_per_s']:.4f} steps/s, pair kernel avg {avg64:.1f} ms")
         out64["fp32c_error_vs_fp64"] = fp32c_error(system)
-        log(f"fp32c error vs fp64: {out64['fp32c_error_vs_fp64']}")
+        log(f"fp32c error vs fp64: {short(out64['fp32c_error_vs_fp64'], 4)}")
 
     achieved = FLOP_PER_PAIR * pairs / (avg32 * 1e-3) / 1e12
     traffic = measured_traffic(args.workload, system.n, "fp32c", tune32)
@@ -809,7 +837,7 @@ def main() -> int:
         result["cpu_baseline"] = cpu_baseline(system, args.cpu_seconds)
         log(f"cpu baseline: {result['cpu_baseline']['value']:.3e} steps/s on "
             f"{result['cpu_baseline']['cores']} threads")
-    print(json.dumps(result), flush=True)
+    print(result_line(result, args.drift_series), flush=True)
     return 0
 
 
