@@ -750,37 +750,93 @@ int ensure_stage(pw_ctx* c, int64_t count) {
   return c->stage_particles > 0 ? PW_OK : fail(PW_ERR_NOMEM, "pinned staging");
 }
 
-// positions and strengths (or, rates, velocities and vorticity rates) of
-// particles [first, first + count) into a and b (either may be null)
-int read_particles(pw_ctx* c, bool rates, int64_t first, int64_t count, double* a, double* b) {
-  if (count <= 0) return PW_OK;
-  PW_TRY(ensure_stage(c, count));
-  for (int64_t p = 0; p < count; p += static_cast<int64_t>(c->stage_particles)) {
-    const int64_t m = std::min<int64_t>(count - p, static_cast<int64_t>(c->stage_particles));
-    if (rates) PW_HIP(pw::launch_pack_rates(c->rates, first + p, m, c->h_stage, c->stream));
-    else PW_HIP(pw::launch_pack_state(c->y, first + p, m, c->h_stage, false, c->stream));
+// Where the caller's rows of particles [first, first + count) are: positions and
+// strengths (or velocities and vorticity rates), 3 doubles each.  A transfer takes
+// a list of consecutive ones, one per wake, in one launch per piece of the staging
+// (one per wake cost 12 us each: the state vector of 20,000 wakes 245 ms).
+template <typename T>
+struct Rows {
+  int64_t first, count;
+  T *a, *b;
+};
+
+// f(row, from, to) for the parts of the rows in particles [p, end); rows before
+// `at` are done with
+template <typename T, typename F>
+void each_part(const std::vector<Rows<T>>& rows, size_t& at, int64_t p, int64_t end, F f) {
+  while (at < rows.size() && rows[at].first + rows[at].count <= p) ++at;
+  for (size_t r = at; r < rows.size() && rows[r].first < end; ++r) {
+    const int64_t from = std::max(p, rows[r].first), to = std::min(end, rows[r].first + rows[r].count);
+    if (from < to) f(rows[r], from, to);
+  }
+}
+
+// the device's rows into the caller's (a or b may be null)
+int read_particles(pw_ctx* c, bool rates, const std::vector<Rows<double>>& rows) {
+  if (rows.empty()) return PW_OK;
+  const int64_t first = rows.front().first, last = rows.back().first + rows.back().count;
+  if (last <= first) return PW_OK;
+  PW_TRY(ensure_stage(c, last - first));
+  size_t at = 0;
+  for (int64_t p = first; p < last; p += static_cast<int64_t>(c->stage_particles)) {
+    const int64_t m = std::min<int64_t>(last - p, static_cast<int64_t>(c->stage_particles));
+    if (rates) PW_HIP(pw::launch_pack_rates(c->rates, p, m, c->h_stage, c->stream));
+    else PW_HIP(pw::launch_pack_state(c->y, p, m, c->h_stage, false, c->stream));
     PW_HIP(hipStreamSynchronize(c->stream));
-    const size_t bytes = 24 * static_cast<size_t>(m);
     std::vector<Segment> segs;
-    if (a) segs.push_back({a + 3 * p, c->h_stage, bytes});
-    if (b) segs.push_back({b + 3 * p, c->h_stage + 3 * m, bytes});
+    each_part(rows, at, p, p + m, [&](const Rows<double>& r, int64_t from, int64_t to) {
+      const size_t bytes = 24 * static_cast<size_t>(to - from);
+      if (r.a) segs.push_back({r.a + 3 * (from - r.first), c->h_stage + 3 * (from - p), bytes});
+      if (r.b) segs.push_back({r.b + 3 * (from - r.first), c->h_stage + 3 * (m + from - p), bytes});
+    });
     copy_segments(segs);
   }
   return PW_OK;
 }
 
-// positions and strengths of particles [first, first + count) from x and a
-int write_particles(pw_ctx* c, int64_t first, int64_t count, const double* x, const double* a) {
-  if (count <= 0) return PW_OK;
-  PW_TRY(ensure_stage(c, count));
-  for (int64_t p = 0; p < count; p += static_cast<int64_t>(c->stage_particles)) {
-    const int64_t m = std::min<int64_t>(count - p, static_cast<int64_t>(c->stage_particles));
-    if (p > 0) PW_HIP(hipStreamSynchronize(c->stream));  // the previous piece has been read
-    const size_t bytes = 24 * static_cast<size_t>(m);
-    copy_segments({{c->h_stage, x + 3 * p, bytes}, {c->h_stage + 3 * m, a + 3 * p, bytes}});
-    PW_HIP(pw::launch_pack_state(c->y, first + p, m, c->h_stage, true, c->stream));
+// the caller's positions and strengths into the state
+int write_particles(pw_ctx* c, const std::vector<Rows<const double>>& rows) {
+  if (rows.empty()) return PW_OK;
+  const int64_t first = rows.front().first, last = rows.back().first + rows.back().count;
+  if (last <= first) return PW_OK;
+  PW_TRY(ensure_stage(c, last - first));
+  size_t at = 0;
+  for (int64_t p = first; p < last; p += static_cast<int64_t>(c->stage_particles)) {
+    const int64_t m = std::min<int64_t>(last - p, static_cast<int64_t>(c->stage_particles));
+    if (p > first) PW_HIP(hipStreamSynchronize(c->stream));  // the previous piece has been read
+    std::vector<Segment> segs;
+    each_part(rows, at, p, p + m, [&](const Rows<const double>& r, int64_t from, int64_t to) {
+      const size_t bytes = 24 * static_cast<size_t>(to - from);
+      segs.push_back({c->h_stage + 3 * (from - p), r.a + 3 * (from - r.first), bytes});
+      segs.push_back({c->h_stage + 3 * (m + from - p), r.b + 3 * (from - r.first), bytes});
+    });
+    copy_segments(segs);
+    PW_HIP(pw::launch_pack_state(c->y, p, m, c->h_stage, true, c->stream));
   }
   return PW_OK;
+}
+
+// the rows of a state or rate vector in the reference's layout: per wake the
+// first 3-vectors of maxn particles, then the second ones (wake.cpp:860-866, :876)
+template <typename T>
+std::vector<Rows<T>> vector_rows(const pw_ctx* c, T* v) {
+  std::vector<Rows<T>> rows;
+  rows.reserve(c->wn.size());
+  for (size_t w = 0; w < c->wn.size(); ++w) {
+    rows.push_back({c->woff[w], c->wn[w], v, v + 3 * c->wmax[w]});
+    v += 6 * c->wmax[w];
+  }
+  return rows;
+}
+
+// zeros in the rows of such a vector that hold no particle
+void clear_unused_rows(const pw_ctx* c, double* v) {
+  for (size_t w = 0; w < c->wn.size(); ++w) {
+    const size_t pad = 24 * static_cast<size_t>(c->wmax[w] - c->wn[w]);
+    std::memset(v + 3 * c->wn[w], 0, pad);
+    std::memset(v + 3 * (c->wmax[w] + c->wn[w]), 0, pad);
+    v += 6 * c->wmax[w];
+  }
 }
 
 // velocities at m points on the device; the partial sums go to the second
@@ -963,7 +1019,7 @@ int pw_set_wake_state(pw_ctx* c, int w, const double* pos, const double* alpha) 
   PW_CTX(c);
   if (w < 0 || w >= static_cast<int>(c->wn.size())) return fail(PW_ERR_ARG, "wake index out of range");
   if (c->wn[w] > 0 && (!pos || !alpha)) return fail(PW_ERR_ARG, "null array");
-  if (c->built) return write_particles(c, c->woff[w], c->wn[w], pos, alpha);
+  if (c->built) return write_particles(c, {{c->woff[w], c->wn[w], pos, alpha}});
   for (int64_t i = 0; i < c->wn[w]; ++i) {
     Rec64& r = c->pending[c->woff[w] + i];
     r.x = pos[3 * i]; r.y = pos[3 * i + 1]; r.z = pos[3 * i + 2];
@@ -988,7 +1044,7 @@ int pw_set_wake_volume(pw_ctx* c, int w, const double* volume) {
 int pw_get_wake_state(pw_ctx* c, int w, double* pos, double* alpha) {
   PW_CTX(c);
   if (w < 0 || w >= static_cast<int>(c->wn.size())) return fail(PW_ERR_ARG, "wake index out of range");
-  if (c->built) return read_particles(c, false, c->woff[w], c->wn[w], pos, alpha);
+  if (c->built) return read_particles(c, false, {{c->woff[w], c->wn[w], pos, alpha}});
   for (int64_t i = 0; i < c->wn[w]; ++i) {
     const Rec64& r = c->pending[c->woff[w] + i];
     if (pos) { pos[3 * i] = r.x; pos[3 * i + 1] = r.y; pos[3 * i + 2] = r.z; }
@@ -1000,7 +1056,7 @@ int pw_get_wake_state(pw_ctx* c, int w, double* pos, double* alpha) {
 int pw_get_wake_rates(pw_ctx* c, int w, double* vel, double* retvor) {
   PW_CTX(c);
   if (w < 0 || w >= static_cast<int>(c->wn.size())) return fail(PW_ERR_ARG, "wake index out of range");
-  if (c->built) return read_particles(c, true, c->woff[w], c->wn[w], vel, retvor);
+  if (c->built) return read_particles(c, true, {{c->woff[w], c->wn[w], vel, retvor}});
   const size_t bytes = 24 * static_cast<size_t>(c->wn[w]);
   if (vel) std::memset(vel, 0, bytes);
   if (retvor) std::memset(retvor, 0, bytes);
@@ -1011,7 +1067,7 @@ int pw_get_wake_rates(pw_ctx* c, int w, double* vel, double* retvor) {
 // wake (the rates of 48 rings, 167,000 particles: a solve 5.35 -> 4.34 ms).
 int pw_get_all_state(pw_ctx* c, double* pos, double* alpha) {
   PW_CTX(c);
-  if (c->built) return read_particles(c, false, 0, c->n, pos, alpha);
+  if (c->built) return read_particles(c, false, {{0, c->n, pos, alpha}});
   for (size_t w = 0; w < c->wn.size(); ++w)
     PW_TRY(pw_get_wake_state(c, static_cast<int>(w), pos ? pos + 3 * c->woff[w] : nullptr,
                              alpha ? alpha + 3 * c->woff[w] : nullptr));
@@ -1020,7 +1076,7 @@ int pw_get_all_state(pw_ctx* c, double* pos, double* alpha) {
 
 int pw_get_all_rates(pw_ctx* c, double* vel, double* retvor) {
   PW_CTX(c);
-  if (c->built) return read_particles(c, true, 0, c->n, vel, retvor);
+  if (c->built) return read_particles(c, true, {{0, c->n, vel, retvor}});
   const size_t bytes = 24 * static_cast<size_t>(c->n);
   if (vel) std::memset(vel, 0, bytes);
   if (retvor) std::memset(retvor, 0, bytes);
@@ -1031,11 +1087,9 @@ int pw_set_states(pw_ctx* c, const double* state, int64_t len) {
   PW_CTX(c);
   if (!state) return fail(PW_ERR_ARG, "null state");
   if (len != total_maxsize(c)) return fail(PW_ERR_ARG, "state length != sum of 6*maxn");
-  // per wake the pos block, maxn x 3, then the alpha block (wake.cpp:860-866)
-  for (size_t w = 0; w < c->wn.size(); ++w) {
-    PW_TRY(pw_set_wake_state(c, static_cast<int>(w), state, state + 3 * c->wmax[w]));
-    state += 6 * c->wmax[w];
-  }
+  const auto rows = vector_rows(c, state);
+  if (c->built) return write_particles(c, rows);
+  for (size_t w = 0; w < rows.size(); ++w) PW_TRY(pw_set_wake_state(c, static_cast<int>(w), rows[w].a, rows[w].b));
   return PW_OK;
 }
 
@@ -1043,14 +1097,10 @@ int pw_get_states(pw_ctx* c, double* state, int64_t len) {
   PW_CTX(c);
   if (!state) return fail(PW_ERR_ARG, "null state");
   if (len != total_maxsize(c)) return fail(PW_ERR_ARG, "state length != sum of 6*maxn");
-  for (size_t w = 0; w < c->wn.size(); ++w) {
-    double *p = state, *a = state + 3 * c->wmax[w];
-    PW_TRY(pw_get_wake_state(c, static_cast<int>(w), p, a));
-    const size_t pad = 24 * static_cast<size_t>(c->wmax[w] - c->wn[w]);
-    std::memset(p + 3 * c->wn[w], 0, pad);
-    std::memset(a + 3 * c->wn[w], 0, pad);
-    state += 6 * c->wmax[w];
-  }
+  const auto rows = vector_rows(c, state);
+  clear_unused_rows(c, state);
+  if (c->built) return read_particles(c, false, rows);
+  for (size_t w = 0; w < rows.size(); ++w) PW_TRY(pw_get_wake_state(c, static_cast<int>(w), rows[w].a, rows[w].b));
   return PW_OK;
 }
 
@@ -1058,15 +1108,12 @@ int pw_get_rates(pw_ctx* c, double* rate, int64_t len) {
   PW_CTX(c);
   if (!rate) return fail(PW_ERR_ARG, "null rate");
   if (len != total_maxsize(c)) return fail(PW_ERR_ARG, "rate length != sum of 6*maxn");
-  for (size_t w = 0; w < c->wn.size(); ++w) {
-    double *u = rate, *q = rate + 3 * c->wmax[w];  // wake.cpp:876
-    PW_TRY(pw_get_wake_rates(c, static_cast<int>(w), u, q));
-    const size_t pad = 24 * static_cast<size_t>(c->wmax[w] - c->wn[w]);
-    std::memset(u + 3 * c->wn[w], 0, pad);
-    std::memset(q + 3 * c->wn[w], 0, pad);
-    rate += 6 * c->wmax[w];
+  if (!c->built) {
+    std::memset(rate, 0, sizeof(double) * static_cast<size_t>(len));
+    return PW_OK;
   }
-  return PW_OK;
+  clear_unused_rows(c, rate);
+  return read_particles(c, true, vector_rows(c, rate));
 }
 
 int pw_velocity_at(pw_ctx* c, const double* points, int64_t m, double* u) {

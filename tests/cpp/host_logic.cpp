@@ -5,6 +5,7 @@
 // GPU.  Usage: host_logic CHECK
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -179,6 +180,7 @@ hipError_t launch_diag_sum(const double* items, const int* first, int nsys, doub
   return hipSuccess;
 }
 hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* host, bool store, hipStream_t) {
+  g_calls.push_back("pack");
   expect(g_pinned.count(host) && g_pinned[host] >= 48 * static_cast<size_t>(count), "staging holds the piece");
   for (int64_t i = 0; i < count; ++i) {
     Rec64& r = y[first + i];
@@ -195,6 +197,7 @@ hipError_t launch_pack_state(Rec64* y, int64_t first, int64_t count, double* hos
 }
 
 hipError_t launch_pack_rates(const Rate64* k, int64_t first, int64_t count, double* host, hipStream_t) {
+  g_calls.push_back("pack");
   expect(g_pinned.count(host) && g_pinned[host] >= 48 * static_cast<size_t>(count), "staging holds the piece");
   for (int64_t i = 0; i < count; ++i) {
     std::memcpy(host + 3 * i, &k[first + i].ux, 24);
@@ -371,6 +374,50 @@ void item_chunks() {
     }
 }
 
+// The reference's state and rate vectors (per wake maxn rows twice) pass in one
+// launch whatever the number of wakes, or one per piece of the staging.
+void state_vectors() {
+  for (const size_t pinned : {std::numeric_limits<size_t>::max(), size_t(30000)}) {
+    g_pinned_limit = pinned;  // 625 particles a piece
+    pw_ctx* c = nullptr;
+    expect(pw_create(&c, 0) == PW_OK && pw_set_coupled(c, 0) == PW_OK, "create");
+    const int wakes = 500;
+    std::vector<int64_t> n(wakes), maxn(wakes);
+    std::vector<double> state;
+    int64_t all = 0;
+    for (int w = 0; w < wakes; ++w) {
+      n[w] = w % 7 == 3 ? 0 : 1 + w % 13;
+      maxn[w] = n[w] + w % 3;
+      all += n[w];
+      std::vector<double> x(3 * n[w] + 1, 0.0), r(n[w] + 1, 0.1), v(n[w] + 1, 1.0);
+      expect(pw_add_wake(c, n[w], maxn[w], x.data(), x.data(), r.data(), v.data(), nullptr) == PW_OK, "add_wake");
+      for (int64_t i = 0; i < 6 * maxn[w]; ++i) state.push_back(i % (3 * maxn[w]) < 3 * n[w] ? 1.0 + state.size() : 0.0);
+    }
+    std::vector<double> out16(16), back(state.size(), -1.0);
+    expect(pw_diagnose_wakes(c, 0, 0, out16.data(), 16) == PW_OK, "build");
+    const size_t pieces = pinned < 40000 ? (all + 299) / 300 + 1 : 1;
+    const int64_t len = static_cast<int64_t>(state.size());
+    const auto calls = [&](const char* what) {
+      expect(g_calls.size() <= pieces, std::string(what) + ": " + std::to_string(g_calls.size()) + " launches");
+      g_calls.clear();
+    };
+    g_calls.clear();
+    expect(pw_set_states(c, state.data(), len) == PW_OK, "set_states");
+    calls("set_states");
+    expect(pw_get_states(c, back.data(), len) == PW_OK && back == state, "get_states returns what was set");
+    calls("get_states");
+    for (int64_t i = 0; i < all; ++i) {
+      std::memcpy(&c->rates[i].ux, &c->y[i].x, 24);
+      std::memcpy(&c->rates[i].wx, &c->y[i].ax, 24);
+    }
+    std::fill(back.begin(), back.end(), -1.0);
+    expect(pw_get_rates(c, back.data(), len) == PW_OK && back == state, "get_rates");
+    calls("get_rates");
+    pw_destroy(c);
+  }
+  g_pinned_limit = std::numeric_limits<size_t>::max();
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -378,7 +425,8 @@ int main(int argc, char** argv) {
                                                       {"diagnose_items", diagnose_items},
                                                       {"little_pinned_memory", little_pinned_memory},
                                                       {"timed_launches", timed_launches},
-                                                      {"item_chunks", item_chunks}};
+                                                      {"item_chunks", item_chunks},
+                                                      {"state_vectors", state_vectors}};
   if (argc != 2 || !checks.count(argv[1])) {
     std::fprintf(stderr, "usage: host_logic CHECK\n");
     return 2;

@@ -56,3 +56,9 @@ def test_pair_timing_holds_the_sum_of_partial_rates(host_logic):
 def test_items_name_their_chunks(host_logic):
     """Coupled and independent wakes, the default launch and source parts."""
     _run(host_logic, "item_chunks")
+
+
+def test_state_vectors_of_many_wakes_in_one_launch(host_logic):
+    """pw_set_states, pw_get_states and pw_get_rates of 500 wakes, empty ones
+    and unused rows among them."""
+    _run(host_logic, "state_vectors")
