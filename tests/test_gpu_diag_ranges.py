@@ -35,8 +35,8 @@ def _scales(s):
     return sh / (4 * np.pi), sk / (8 * np.pi), 47 * se / (8 * np.pi)
 
 
-def _check(d, ref, s, kernel):
-    sh, sk, se = _scales(s)
+def _check(d, ref, s, kernel, scales):
+    sh, sk, se = scales
     tol = 4 * (np.sqrt(s.n) + 8) * 2.0 ** -52
     assert abs(d[H] - ref[H]) <= tol * sh
     assert abs(d[KE] - ref[KE]) <= tol * sk and abs(d[KEF] - ref[KEF]) <= tol * sk
@@ -44,7 +44,7 @@ def _check(d, ref, s, kernel):
         assert abs(d[EN] - ref[EN]) <= tol * se and abs(d[ENF] - ref[ENF]) <= tol * se
 
 
-@pytest.mark.parametrize("n", [6501, 13001, 24001])
+@pytest.mark.parametrize("n", [6501, 13001, 18001])
 @pytest.mark.parametrize("kernel", [0, 1])
 def test_long_ranges(oracle, n, kernel):
     s = _wake(n, n)
@@ -54,17 +54,18 @@ def test_long_ranges(oracle, n, kernel):
         g.set_kernel(kernel)
         d = g.diagnose()[:15]
         own = g.diagnose_wakes(0, 0)
-    _check(d, ref, s, kernel)
-    _check(own, ref, s, kernel)
+    scales = _scales(s)
+    _check(d, ref, s, kernel, scales)
+    _check(own, ref, s, kernel, scales)
 
 
 @pytest.mark.parametrize("kernel", [0, 1])
 def test_blocks_of_two_wakes(oracle, kernel):
-    parts = [_wake(9001, 5), _wake(12343, 6)]
+    parts = [_wake(5001, 5), _wake(8343, 6)]
     c = W.concat(parts, coupled=True, nu=0.0, name="two")
     with oracle.smoothing(kernel):
         ref = oracle.diagnose(c)
     with capi.Solver(c) as g:
         g.set_kernel(kernel)
         blocks = [g.diagnose_wakes(*p) for p in ((0, 0), (1, 1), (0, 1))]
-    _check(np.sum(blocks, axis=0), ref, c, kernel)
+    _check(np.sum(blocks, axis=0), ref, c, kernel, _scales(c))
